@@ -146,6 +146,45 @@ def test_attention_bf16(gpu, lens):
         assert rel_err(out[s0:s0 + n], want) < 1e-2, n
 
 
+@pytest.mark.parametrize("nh,nkv,scale,lens", [
+    (16, 8, 128 ** -0.5, [2048]),                    # 128-row workgroups: whole tiles only
+    (16, 8, 128 ** -0.5, [2049, 65, 1, 64]),         # a last tile of one key, sequences far below the longest
+    (16, 8, -0.05, [1100, 1023, 130]),               # a negative scale
+    (8, 8, 128 ** -0.5, [1999, 2500]),               # one q head per kv head
+    (24, 8, 128 ** -0.5, [700, 701]),                # three
+    (6, 1, 128 ** -0.5, [150, 3, 32, 33]),           # one kv head; 32-row workgroups with the keys split
+    (16, 8, -0.05, [97, 128, 129]),
+    (3, 3, 0.0, [40, 200])])                         # scale 0: the mean of V
+def test_attention_bf16_forms(gpu, nh, nkv, scale, lens):
+    """Both workgroup forms at the edges of their key tiles and row blocks, and head groupings, scale signs:
+    each sequence against the float64 attention of the same bf16 values. P and the output are rounded to bf16
+    (2^-9 relative each, averaged over the keys): 1e-2 in relative norm."""
+    from torch_xdna import kernels
+
+    g = torch.Generator().manual_seed(sum(lens) + nh)
+    T = sum(lens)
+    q = (torch.randn(T, nh, 128, generator=g) * 2).to(torch.bfloat16)
+    k = (torch.randn(T, nkv, 128, generator=g) * 2).to(torch.bfloat16)
+    v = torch.randn(T, nkv, 128, generator=g).to(torch.bfloat16)
+    starts, vts, s, c = [], [], 0, 0
+    for n in lens:
+        starts.append(s)
+        vts.append(c)
+        s, c = s + n, c + -(-n // 32) * 32
+    vt = torch.zeros(nkv, 128, c, dtype=torch.bfloat16)
+    for n, s0, c0 in zip(lens, starts, vts):
+        vt[:, :, c0:c0 + n] = v[s0:s0 + n].permute(1, 2, 0)
+    i32 = dict(dtype=torch.int32, device=gpu)
+    out = kernels.attention_bf16(q.to(gpu), k.to(gpu), vt.to(gpu), torch.tensor(starts, **i32),
+                                 torch.tensor(lens, **i32), torch.tensor(vts, **i32), max(lens), scale)
+    out = out.cpu().double()
+    for n, s0 in zip(lens, starts):
+        for h in range(nh):
+            kv = h // (nh // nkv)
+            p = torch.softmax(q[s0:s0 + n, h].double() @ k[s0:s0 + n, kv].double().t() * scale, dim=-1)
+            assert rel_err(out[s0:s0 + n, h], p @ v[s0:s0 + n, kv].double()) < 1e-2, (n, h)
+
+
 def test_silu_mul_and_add(gpu):
     from torch_xdna import kernels
 

@@ -7,11 +7,12 @@
 //                  RoPE at the token's position; V written transposed (dims x tokens) for attention
 //   attention      softmax(q k^T * scale) v per sequence and head, bidirectional over the sequence's
 //                  tokens, grouped-query (q head h reads kv head h / (nh / nkv)), bf16 MFMA with an
-//                  online softmax in float32 (32 queries per wave, keys in blocks of 32)
+//                  online softmax in float32 (32 rows per wave, keys in LDS tiles of 64 or 32)
 //   silu_mul       bf16(silu(gate) * up)
 //   add_f32        x += y (the residual adds)
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "xdna_common.h"
@@ -119,105 +120,281 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const float* __restri
 }
 
 // ------------------------------------------------------------------------------ attention
-// Grid (nseq * qblocks_max, nh); one wave per block: 32 queries of one head of one sequence.
-// MFMA (srcA = X, srcB = Y) gives, in lane l, row l % 32 of Y and, in element 4 g + r, row
-// 8 g + 4 (l / 32) + r of X. S = K Q^T: lane l <-> query l % 32, elements <-> 16 of 32 keys. The
-// softmax statistics of a query are kept identical in lanes l and l ^ 32. O^T = V^T P^T accumulates
-// with lane l <-> query l % 32 and elements <-> dims. P's operand needs keys 8 (l / 32) .. +7 of each
-// 16-key step in lane l: lanes l and l ^ 32 swap one group of 4 keys per step.
-__global__ __launch_bounds__(64) void attention_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
-                                                       const uint16_t* __restrict__ vt, int64_t ld_vt,
-                                                       const int32_t* __restrict__ seq_start,
-                                                       const int32_t* __restrict__ seq_len,
-                                                       const int32_t* __restrict__ seq_vt, int qblocks, int nh,
-                                                       int nkv, float scale, uint16_t* __restrict__ out) {
-  const int lane = threadIdx.x;
-  const int seq = blockIdx.x / qblocks;
-  const int qb = blockIdx.x - seq * qblocks;
-  const int h = blockIdx.y;
+// A kv head's queries are its rows: row i of sequence s and kv head g is query i / grp of q head
+// g * grp + i % grp (grp = nh / nkv), so the heads that share K and V also share their loads. A workgroup has QW
+// waves of 32 rows each and KW groups of such waves; group g takes the key tiles g, g + KW, ... of KT keys, and at
+// the end the groups' maxima, sums and outputs meet in LDS. K [KT keys][128] and V^T [128 dims][KT keys] of a tile
+// are brought into LDS by the DMA form of the global load. Grid: kv heads fastest, so that with 8 of them each
+// XCD's L2 holds the K and V of its own head.
+//
+// MFMA (srcA = X, srcB = Y) gives, in lane l, row l % 32 of Y and, in element 4 g + r, row 8 g + 4 (l / 32) + r of
+// X; lane l supplies values 8 (l / 32) .. + 7 of the 16-deep step of its operand's row l % 32. S = K Q^T: lane l
+// <-> row l % 32, elements <-> 16 of 32 keys. O^T = V^T P^T wants keys 8 (l / 32) .. + 7 of each 16-key step in
+// lane l; reading K's fragment row i from key swap23(i) (bits 2 and 3 of i exchanged) makes a lane's elements
+// 8 u .. 8 u + 7 exactly those of step u, so P goes from one product to the next without leaving its lane.
+// LDS chunks of 16 bytes are XORed with the row so that the 16 lanes of a fragment read's phase cover the banks.
+//
+// Softmax: p = 2^(c (s - m)), c = scale * log2(e) > 0 (a negative scale goes into Q's sign), in float32; O and l
+// are rescaled only in the tiles where some row's running maximum m grows; P is rounded to bf16 for the second
+// product, l sums the unrounded p. (Letting m lag by up to 2^8 skips more of the rescales and runs 4% faster, but
+// the rounding of P then errs by 5% more against 64 bits: not done.)
+//
+// What bounds it: per 64 keys and 32 rows a wave issues 32 MFMAs (1024 cycles of its SIMD) and about 400 vector
+// instructions of softmax, so two waves per SIMD (two workgroups per CU, 64 KB of LDS each) fill each other's
+// gaps; with the registers for one wave per SIMD only (no spills either way) the long shapes run 1.5x slower.
+// Measured, 16 q and 8 kv heads: 1 x 4096 queries 189 us (727 TFLOP/s), 4 x 4096 706 us; lengths 4096 / 1500 / 700
+// in one call 206 us against 557 us for one wave per 32 queries of a q head reading its K and V fragments straight
+// from memory, 264 / 222 (the split form) 9.1 against 18.7 us. MFMA issue has priority over the other wave's
+// softmax (s_setprio): 4% on the long shapes.
+__device__ __forceinline__ int swap23(int i) { return (i & ~12) | ((i & 4) << 1) | ((i & 8) >> 1); }
+
+typedef __attribute__((address_space(3))) void* lds_ptr;
+typedef const __attribute__((address_space(1))) void* glb_ptr;
+__device__ __forceinline__ void gload_lds16(const void* g, int8_t* l) {   // lane i's 16 bytes land at l + 16 i
+  __builtin_amdgcn_global_load_lds((glb_ptr)g, (lds_ptr)l, 16, 0, 0);
+}
+
+// the larger of a lane's value and that of lane l ^ 32, and their sum
+__device__ __forceinline__ float half_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __builtin_elementwise_maximum(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float half_sum(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// ST: LDS stages of a group. 2: tile t + 1 loads while t is used, one workgroup barrier per tile. 1 (QW == 1, the
+// group's LDS is its wave's own, no barriers): the next K loads once S is done, the next V after the tile.
+template <int QW, int KW, int KT, int ST>
+__global__ __launch_bounds__(QW* KW * 64, 2) void attention_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ vt, int64_t ld_vt,
+    const int32_t* __restrict__ seq_start, const int32_t* __restrict__ seq_len, const int32_t* __restrict__ seq_vt,
+    int qblocks, int nh, int nkv, float c, uint32_t qsign, uint16_t* __restrict__ out) {
+  static_assert(ST == 2 || QW == 1, "a single stage is one wave's own");
+  constexpr int NB = KT / 32;              // 32-key blocks of a tile
+  constexpr int KB = KT * 256, VB = KT * 256, STAGE = KB + VB;
+  constexpr int NI = KT / 4 / QW;          // 1 KB loads of K, and of V, per wave and tile
+  constexpr int VCH = KT / 8, VD = 512 / KT;   // chunks of a V^T row; rows of one 1 KB load
+  constexpr int VSH = KT == 64 ? 1 : 2;    // V^T rows per 256 bytes, as a shift
+  static_assert(KT == 64 || KT == 32, "V^T rows of 128 or 64 bytes");
+  __shared__ __attribute__((aligned(1024))) int8_t lds_all[KW * ST * STAGE];
+  __shared__ float ml[KW > 1 ? 2 * KW * 64 : 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = wave / QW, qw = wave - kg * QW;
+  const int kvh = blockIdx.x % nkv;
+  const int sb = blockIdx.x / nkv;
+  const int seq = sb / qblocks, qb = sb - seq * qblocks;
   const int n = seq_len[seq];
-  if (qb * 32 >= n) return;
+  const int grp = nh / nkv;
+  const int nrows = n * grp;
+  if (qb * (QW * 32) >= nrows) return;     // uniform
   const int64_t start = seq_start[seq];
-  const int64_t vt0 = seq_vt[seq];
-  const int kvh = h / (nh / nkv);
   const int half = lane >> 5, row = lane & 31;
-  // this lane's query and its 8 fragments (16 bytes of dims 16 s + 8 half .. +7)
-  const int qi = min(qb * 32 + row, n - 1);
+  const int idx = (qb * QW + qw) * 32 + row;
+  const int idc = min(idx, nrows - 1);
+  const int qi = idc / grp;
+  const int64_t qoff = ((start + qi) * nh + (int64_t)kvh * grp + (idc - qi * grp)) * 128;
   i32x4 qf[8];
-  const uint16_t* qrow = q + ((start + qi) * nh + h) * 128 + 8 * half;
 #pragma unroll
-  for (int s = 0; s < 8; ++s) qf[s] = *reinterpret_cast<const i32x4*>(qrow + 16 * s);
+  for (int s = 0; s < 8; ++s) {
+    qf[s] = *reinterpret_cast<const i32x4*>(q + qoff + 8 * half + 16 * s);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) qf[s][e] ^= (int)qsign;
+  }
+  int8_t* const lds = lds_all + kg * (ST * STAGE);
+  const uint16_t* const kbase = k + (start * nkv + kvh) * 128;
+  const uint16_t* const vbase = vt + (int64_t)kvh * 128 * ld_vt + seq_vt[seq];
+  // this lane's K rows and V^T rows: load j fills 16-byte chunk lane of KB j
+  uint32_t krow[NI], kch[NI];
+  const uint16_t* vp[NI];
+  int vc[NI];
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const int ld = qw * NI + j;
+    krow[j] = (uint32_t)(ld * 4 + (lane >> 4));
+    kch[j] = (uint32_t)(((lane & 15) ^ (krow[j] & 15)) * 16);
+    const int dim = ld * VD + lane / VCH;
+    vc[j] = ((lane & (VCH - 1)) ^ ((dim >> VSH) & (VCH - 1))) * 8;
+    vp[j] = vbase + dim * ld_vt + vc[j];
+  }
+  const uint32_t kpitch = (uint32_t)nkv * 256u;
+  // keys past the sequence read its last key (their p are set to 0); V chunks wholly past it read its last chunk
+  // (their fragments are set to 0)
+  auto load_k = [&](int kb, int8_t* st) {
+    const char* base = reinterpret_cast<const char*>(kbase) + (int64_t)kb * kpitch;
+    const uint32_t last = (uint32_t)(n - 1 - kb);
+#pragma unroll
+    for (int j = 0; j < NI; ++j) gload_lds16(base + min(krow[j], last) * kpitch + kch[j], st + ((qw * NI + j) << 10));
+  };
+  auto load_v = [&](int kb, int8_t* st) {
+    if (kb + KT <= n) {
+#pragma unroll
+      for (int j = 0; j < NI; ++j) gload_lds16(vp[j] + kb, st + KB + ((qw * NI + j) << 10));
+    } else {
+      const int lastc = (n - 1) & ~7;
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+        gload_lds16(vp[j] + (min(kb + vc[j], lastc) - vc[j]), st + KB + ((qw * NI + j) << 10));
+    }
+  };
   f32x16s o[4];
 #pragma unroll
   for (int db = 0; db < 4; ++db) o[db] = f32x16s{};
   float m = -INFINITY, l = 0.0f;
-  for (int kb = 0; kb < n; kb += 32) {
-    // S block: keys kb .. kb + 31
-    const int ki = min(kb + row, n - 1);
-    const uint16_t* krow = k + ((start + ki) * nkv + kvh) * 128 + 8 * half;
-    f32x16s sc = f32x16s{};
-#pragma unroll
-    for (int s = 0; s < 8; ++s) sc = mfma_bf16(*reinterpret_cast<const i32x4*>(krow + 16 * s), qf[s], sc);
-    float p[16];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int key = kb + 8 * (e >> 2) + 4 * half + (e & 3);
-      p[e] = key < n ? sc[e] * scale : -INFINITY;
-      mx = fmaxf(mx, p[e]);
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mn = fmaxf(m, mx);        // finite: every block has at least one key < n
-    const float alpha = m == -INFINITY ? 0.0f : __expf(m - mn);
-    float ps = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      p[e] = __expf(p[e] - mn);           // exp(-inf) = 0 for keys past n
-      ps += p[e];
-    }
-    ps += __shfl_xor(ps, 32, 64);
-    l = l * alpha + ps;
-    m = mn;
-#pragma unroll
-    for (int db = 0; db < 4; ++db) o[db] *= alpha;
-    // P V for the two 16-key steps of this block
-#pragma unroll
-    for (int st = 0; st < 2; ++st) {
-      // own keys 16 st + 4 half + (0..3) (group g = 2 st) and 16 st + 8 + 4 half + (0..3) (g = 2 st + 1);
-      // half 0 needs 16 st + 0..7, half 1 needs 16 st + 8..15
-      float send[4], recv[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) send[r] = half == 0 ? p[4 * (2 * st + 1) + r] : p[4 * (2 * st) + r];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) recv[r] = __shfl_xor(send[r], 32, 64);
-      float lo[4], hi[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        lo[r] = half == 0 ? p[4 * (2 * st) + r] : recv[r];
-        hi[r] = half == 0 ? recv[r] : p[4 * (2 * st + 1) + r];
+  const int krd = swap23(row) * 256;       // the lane's fragment row of each 32-key block
+  const int kx = swap23(row) & 15;
+  const int vx = (row >> VSH) & (VCH - 1);
+  const int nt = (n + KT * KW - 1) / (KT * KW);
+  if (kg * KT < n) {
+    load_k(kg * KT, lds);
+    load_v(kg * KT, lds);
+  }
+  for (int t = 0; t < nt; ++t) {
+    const int kb = (t * KW + kg) * KT;
+    const int kn = kb + KW * KT;           // the group's next tile
+    int8_t* const cur = lds + (ST == 2 ? (t & 1) * STAGE : 0);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    if constexpr (ST == 2) {
+      __builtin_amdgcn_s_barrier();        // tile t is whole; every wave is done with tile t - 1
+      __builtin_amdgcn_sched_barrier(0);
+      if (kn < n) {
+        load_k(kn, lds + ((t + 1) & 1) * STAGE);
+        load_v(kn, lds + ((t + 1) & 1) * STAGE);
       }
-      const i32x4 pf = {(int)f32x2_to_bf16x2_bits(lo[0], lo[1]), (int)f32x2_to_bf16x2_bits(lo[2], lo[3]),
-                        (int)f32x2_to_bf16x2_bits(hi[0], hi[1]), (int)f32x2_to_bf16x2_bits(hi[2], hi[3])};
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (KW > 1 && kb >= n) continue;       // uniform over the group; the last tile at the earliest
+    f32x16s sc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) sc[b] = f32x16s{};
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        sc[b] = mfma_bf16(*reinterpret_cast<const i32x4*>(cur + b * 8192 + krd + (((2 * s + half) ^ kx) << 4)), qf[s], sc[b]);
+    if constexpr (ST == 1) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      if (kn < n) load_k(kn, cur);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    const bool part = kb + KT > n;         // uniform
+    float mx = -INFINITY;
+    if (part) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (kb + 32 * b + 16 * (e >> 3) + 8 * half + (e & 7) >= n) sc[b][e] = -INFINITY;
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; e += 2)
+        mx = __builtin_elementwise_maximum(mx, __builtin_elementwise_maximum(sc[b][e], sc[b][e + 1]));
+    mx = half_max(mx);
+    const bool grow = mx > m;
+    if (__builtin_amdgcn_ballot_w64(grow)) {
+      const float mn = grow ? mx : m;
+      const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - mn) * c);
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) o[db] *= alpha;
+      m = mn;
+    }
+    const float mc = m * c;
+    i32x4 pf[2 * NB];
+    float ps[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      float p[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[b][e], c, -mc));
+        if (part && kb + 32 * b + 16 * (e >> 3) + 8 * half + (e & 7) >= n) p[e] = 0.0f;
+      }
+#pragma unroll
+      for (int e = 0; e < 16; e += 2) {
+        ps[0] += p[e];
+        ps[1] += p[e + 1];
+        pf[2 * b + (e >> 3)][(e & 7) >> 1] = (int)f32x2_to_bf16x2_bits(p[e], p[e + 1]);
+      }
+    }
+    l += ps[0] + ps[1];
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int u = 0; u < 2 * NB; ++u)
 #pragma unroll
       for (int db = 0; db < 4; ++db) {
-        const uint16_t* vrow = vt + ((int64_t)kvh * 128 + db * 32 + row) * ld_vt + vt0 + kb + 16 * st + 8 * half;
-        o[db] = mfma_bf16(*reinterpret_cast<const i32x4*>(vrow), pf, o[db]);
+        i32x4 vf = *reinterpret_cast<const i32x4*>(cur + KB + (db * 32 + row) * (2 * KT) + (((2 * u + half) ^ vx) << 4));
+        if (part && kb + 16 * u + 8 * half >= n) vf = i32x4{0, 0, 0, 0};
+        o[db] = mfma_bf16(vf, pf[u], o[db]);
       }
+    __builtin_amdgcn_s_setprio(0);
+    if constexpr (ST == 1) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      if (kn < n) load_v(kn, cur);
     }
   }
-  const int qo = qb * 32 + row;
-  if (qo >= n) return;
-  const float inv = 1.0f / l;
-  uint16_t* orow = out + ((start + qo) * nh + h) * 128;
-#pragma unroll
-  for (int db = 0; db < 4; ++db)
+  l = half_sum(l);
+  uint16_t* const orow = out + qoff;
+  auto store = [&](const f32x16s& v, int db, float inv) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const int d = db * 32 + 8 * g + 4 * half;
-      const uint32_t w0 = f32x2_to_bf16x2_bits(o[db][4 * g] * inv, o[db][4 * g + 1] * inv);
-      const uint32_t w1 = f32x2_to_bf16x2_bits(o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv);
-      *reinterpret_cast<uint2*>(orow + d) = make_uint2(w0, w1);
+      const uint32_t w0 = f32x2_to_bf16x2_bits(v[4 * g] * inv, v[4 * g + 1] * inv);
+      const uint32_t w1 = f32x2_to_bf16x2_bits(v[4 * g + 2] * inv, v[4 * g + 3] * inv);
+      *reinterpret_cast<uint2*>(orow + db * 32 + 8 * g + 4 * half) = make_uint2(w0, w1);
     }
+  };
+  if constexpr (KW == 1) {
+    if (idx >= nrows) return;
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) store(o[db], db, inv);
+  } else {
+    // each wave leaves its m, l and O; wave kg then combines dims 32 (4 / KW) kg .. of the 32 rows
+    static_assert(QW == 1 && 4 % KW == 0 && KW * 16384 <= KW * ST * STAGE, "one row block, its outputs in LDS");
+    __syncthreads();
+    ml[kg * 64 + lane] = m;
+    ml[(KW + kg) * 64 + lane] = l;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(lds_all + kg * 16384 + (db * 4 + g) * 1024 + lane * 16) =
+            f32x4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
+    __syncthreads();
+    float mt = ml[lane];
+#pragma unroll
+    for (int g = 1; g < KW; ++g) mt = __builtin_elementwise_maximum(mt, ml[g * 64 + lane]);
+    float w[KW], lt = 0.0f;
+#pragma unroll
+    for (int g = 0; g < KW; ++g) {
+      const float mg = ml[g * 64 + lane];
+      w[g] = mg == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((mg - mt) * c);   // a group without keys: nothing
+      lt += ml[(KW + g) * 64 + lane] * w[g];
+    }
+    if (idx >= nrows) return;              // no barrier follows
+    const float inv = 1.0f / lt;
+#pragma unroll
+    for (int d = 0; d < 4 / KW; ++d) {
+      const int db = kg * (4 / KW) + d;
+      f32x16s v = f32x16s{};
+#pragma unroll
+      for (int g = 0; g < KW; ++g)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(lds_all + g * 16384 + (db * 4 + h) * 1024 + lane * 16);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[4 * h + r] += x[r] * w[g];
+        }
+      store(v, db, inv);
+    }
+  }
 }
 
 // ------------------------------------------------------------------------------ SiLU * up, residual add
@@ -299,12 +476,29 @@ int xdna_attention_bf16(const void* q, const void* k, const void* vt, int64_t ld
   XDNA_REQUIRE(q && k && vt && seq_start && seq_len && seq_vt && out, "null pointer");
   XDNA_REQUIRE(ld_vt % 8 == 0 && aligned(q, 16) && aligned(k, 16) && aligned(vt, 16) && aligned(out, 8),
                "misaligned operands (ld_vt % 8, 16-byte q / k / vt)");
-  const int64_t qblocks = cdiv(max_len, 32);
-  XDNA_REQUIRE(nseq * qblocks < (1ll << 31), "too many sequences");
-  dim3 g((unsigned)(nseq * qblocks), (unsigned)nh);
-  attention_kernel<<<g, 64, 0, as_stream(stream)>>>(static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
-                                                     static_cast<const uint16_t*>(vt), ld_vt, seq_start, seq_len,
-                                                     seq_vt, (int)qblocks, nh, nkv, scale, static_cast<uint16_t*>(out));
+  const int64_t grp = nh / nkv;
+  const float c = fabsf(scale) * 1.44269504088896340736f;
+  const uint32_t qsign = scale < 0.0f ? 0x80008000u : 0u;
+  // 128 rows per workgroup, sharing each key tile, once such workgroups cover three quarters of the CUs; below that
+  // 32 rows with the keys split over four waves, which quarters the chain of tiles a wave walks. Measured, 16 / 8
+  // heads, wide against split: one sequence of 512 20.4 / 10.8 us, 1024 36.6 / 23.5, 1300 (168 wide workgroups)
+  // 47.6 / 44.8, 1500 (192) 53.9 / 53.3, 1800 64.9 / 66.5, 3000 133 / 159; four of 500 (256) 23.4 / 28.2
+  const bool wide = 4 * nseq * cdiv(max_len * grp, 128) * nkv >= 3 * (int64_t)device_cus();
+  const int64_t qblocks = cdiv(max_len * grp, wide ? 128 : 32);
+  XDNA_REQUIRE(qblocks * nkv < (1ll << 31), "sequence too long");
+  const int64_t step = ((1ll << 31) - 1) / (qblocks * nkv);   // sequences per launch
+  for (int64_t s0 = 0; s0 < nseq; s0 += step) {
+    const dim3 g((unsigned)(std::min(step, nseq - s0) * qblocks * nkv));
+    const uint16_t *qp = static_cast<const uint16_t*>(q), *kp = static_cast<const uint16_t*>(k),
+                   *vp = static_cast<const uint16_t*>(vt);
+    uint16_t* op = static_cast<uint16_t*>(out);
+    if (wide)
+      attention_kernel<4, 1, 64, 2><<<g, 256, 0, as_stream(stream)>>>(qp, kp, vp, ld_vt, seq_start + s0, seq_len + s0,
+                                                                       seq_vt + s0, (int)qblocks, nh, nkv, c, qsign, op);
+    else
+      attention_kernel<1, 4, 32, 1><<<g, 256, 0, as_stream(stream)>>>(qp, kp, vp, ld_vt, seq_start + s0, seq_len + s0,
+                                                                       seq_vt + s0, (int)qblocks, nh, nkv, c, qsign, op);
+  }
   return launch_status("attention_bf16");
 }
 
