@@ -117,6 +117,60 @@ def test_qk_norm_rope(gpu):
     assert torch.equal(got_v, v)
 
 
+@pytest.mark.parametrize("d,rows", [(256, 3), (768, 70), (1280, 5), (4096, 2)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_rmsnorm_bf16_widths(gpu, d, rows, shift):
+    """Row widths at the edges of the one-wave and four-wave forms, and operands one element past a 16-byte
+    boundary: the norm and the add + norm within two bf16 ulps of float64, x after the add exactly x + a."""
+    from torch_xdna import kernels
+
+    g = torch.Generator().manual_seed(d + rows)
+
+    def moved(t):
+        buf = torch.empty(t.numel() + shift, dtype=t.dtype, device=gpu)
+        buf[shift:].copy_(t.reshape(-1))
+        return buf[shift:].view(t.shape)
+
+    x, a = torch.randn(rows, d, generator=g), torch.randn(rows, d, generator=g)
+    for wt in (torch.float32, torch.bfloat16, torch.float16):
+        w = (1 + 0.1 * torch.randn(d, generator=g)).to(wt)
+        _close_bf16(kernels.rmsnorm_bf16(moved(x), moved(w), 1e-6), Q.rms_norm(x.double(), w.double(), 1e-6))
+        xg = moved(x)
+        _close_bf16(kernels.add_rmsnorm_bf16(xg, moved(a), moved(w), 1e-6), Q.rms_norm((x + a).double(), w.double(), 1e-6))
+        assert torch.equal(xg.cpu(), x + a)
+
+
+@pytest.mark.parametrize("T,nh,nkv,perm", [(1, 16, 8, False), (31, 16, 8, False), (32, 4, 4, True), (33, 6, 1, False),
+                                           (97, 3, 1, True)])
+def test_qk_norm_rope_forms(gpu, T, nh, nkv, perm):
+    """Token counts at the edges of the V copy's 32-token blocks, head counts off the eight half waves, V columns
+    in order and permuted: q and k within two bf16 ulps of float64, V exactly the rounded values in their columns
+    and nothing else written."""
+    from torch_xdna import kernels
+
+    g = torch.Generator().manual_seed(T + nh)
+    qkv = torch.randn(T, (nh + 2 * nkv) * 128, generator=g)
+    qw, kw = 1 + 0.1 * torch.randn(128, generator=g), 1 + 0.1 * torch.randn(128, generator=g)
+    inv_freq = 1.0 / (1e6 ** (torch.arange(0, 128, 2, dtype=torch.float32) / 128))
+    pos = torch.randint(0, 4096, (T,), generator=g, dtype=torch.int32)
+    col = (torch.randperm(T + 24, generator=g)[:T] if perm else torch.arange(T) + 8).to(torch.int32)
+    vt = torch.full((nkv, 128, T + 32), 7.0, dtype=torch.bfloat16, device=gpu)
+    q, k = kernels.qk_norm_rope(qkv.to(gpu), nh, nkv, qw.to(gpu), kw.to(gpu), inv_freq.to(gpu), pos.to(gpu),
+                                col.to(gpu), 1e-6, vt)
+    x = qkv.double()
+    for heads, off, w, got in ((nh, 0, qw, q), (nkv, nh * 128, kw, k)):
+        h = Q.rms_norm(x[:, off:off + heads * 128].view(T, heads, 128), w.double(), 1e-6)
+        ang = pos.float()[:, None] * inv_freq[None, :]
+        ang = torch.cat([ang, ang], -1)[:, None, :]
+        rot = torch.cat([-h[..., 64:], h[..., :64]], -1)
+        # near-cancelling pairs: float32 errors of the two products (2^-22 of their size) under the two ulps
+        err = (got.double().cpu() - (h * ang.cos().double() + rot * ang.sin().double())).abs()
+        assert bool((err <= 2 * BF16_ULP * got.double().cpu().abs() + 1e-5).all())
+    want = torch.full((nkv, 128, T + 32), 7.0, dtype=torch.bfloat16)
+    want[:, :, col.long()] = qkv[:, (nh + nkv) * 128:].view(T, nkv, 128).to(torch.bfloat16).permute(1, 2, 0)
+    assert torch.equal(vt.cpu(), want)
+
+
 @pytest.mark.parametrize("lens", [[1], [31, 32, 33], [100, 65, 7], [257]])
 def test_attention_bf16(gpu, lens):
     """Ragged sequences (partial and single query / key blocks): each sequence's heads against the

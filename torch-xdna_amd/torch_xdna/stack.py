@@ -56,7 +56,7 @@ VERIFY_TOL = 0.1               # relative norm error of the first fused call aga
 # Longest sequence the fused op takes. The reference's NPU program stops at 384 positions; the GPU
 # attention streams the keys, so the cap only bounds the work of one call.
 MAX_TOKENS = 4096
-QBLOCK = 32                    # queries per attention wave
+QBLOCK = 32                    # a sequence's V columns are padded to, and its first-call check counted in, blocks of these
 
 _ROOT_CLASS = "Qwen3Model"
 _LINEAR = frozenset({torch._C._nn.linear, F.linear})
