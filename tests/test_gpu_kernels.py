@@ -710,6 +710,35 @@ def test_tiles_forced(gpu, tile, tile_table):
             assert kernels.conv3x3_calibrate(x_nhwc, packed.to(gpu), False) == int(np.abs(acc).max())
 
 
+@pytest.mark.parametrize("tile", ["t256x256w8", "t256x256w4", "t256x128", "t128x256", "t128x128", "t64x64", "t192x256",
+                                  "t256x192", "t64x32", "t32x64", "t32x32", "t128x128k2", "t128x256w8", "t256x128w8",
+                                  "t256x64"])
+def test_tiles_slices(gpu, tile, tile_table):
+    """K at the edges of the engine's 128-byte slices (less than one, one, one and 16 bytes, a half more, more slices
+    than stages) with ragged M and N, and convs whose channels are one, two and three such slices, whole or with
+    images the conv's other loaders take: int32 sums and requantized integers exact. 2300 x 2100 x 2064 gives
+    128 x 128 tiles more than one per CU (their long-slice form)."""
+    from torch_xdna import kernels
+
+    shapes = [(130, 70, k) for k in (16, 64, 112, 128, 144, 192, 240, 256, 400, 1040)]
+    if tile == "t128x128":
+        shapes.append((2300, 2100, 2064))
+    for m, n, k in shapes:
+        kernels.tile_set("i8", m, n, k, tile)
+        a, w = _i8((m, k), seed=m + k), _i8((n, k), seed=n + k)
+        want = torch._int_mm(a, w.t().contiguous())
+        assert torch.equal(kernels.mm_i8(a.to(gpu), w.to(gpu)).cpu(), want), (m, n, k)
+    for n, ci, co, h, w_ in [(2, 128, 72, 5, 9), (1, 256, 40, 7, 6), (1, 384, 40, 4, 5), (2, 144, 40, 5, 7), (1, 20, 72, 9, 7)]:
+        c_pad = -(-ci // 16) * 16
+        kernels.tile_set("conv", n * h * w_, co, 9 * c_pad, tile)
+        xq, wq = _i8((n, ci, h, w_), seed=ci + h), _i8((co, ci, 3, 3), seed=co + w_)
+        packed = torch.zeros(co, 9, c_pad, dtype=torch.int8)
+        packed[:, :, :ci] = wq.permute(0, 2, 3, 1).reshape(co, 9, ci)
+        q = kernels.conv3x3(kernels.nchw_to_nhwc(xq.to(gpu), c_pad), packed.to(gpu), 9, False)
+        assert np.array_equal(_np(q).transpose(0, 3, 1, 2),
+                              O.requant(c_oracle.conv3x3_acc(xq.numpy(), wq.numpy()), 9, False)), (n, ci, co, h, w_)
+
+
 def _ksplit(cus, bm, bn, kg, tiles, k):
     """Workgroups per tile along K that the library gives a launch: 1 above 64 x 64 or when the tiles fill
     more than half of the CUs, else up to CUs / tiles, at most 16, with at least 16 slices of 64 per K

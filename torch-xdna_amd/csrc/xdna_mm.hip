@@ -7,9 +7,9 @@
 // columns n of one row m. Tiles: 256x256 with 8 waves (two per SIMD), 256x128 / 128x256 /
 // 128x128 with 4 waves, 64x64 with 4 waves; the host picks one per shape.
 //
-// K is staged through S LDS stages of 64-byte slices by the LDS-DMA form of the raw buffer load:
+// K is staged through S LDS stages of 64- or 128-byte slices by the LDS-DMA form of the raw buffer load:
 // each lane's 16 bytes land at M0 + 16 * lane, so no VGPRs carry the tile, and S - 1 slices are in
-// flight while one is consumed. LDS rows are 64 bytes; the 16-byte chunk c of row r sits at chunk
+// flight while one is consumed. With 64-byte slices LDS rows are 64 bytes; the 16-byte chunk c of row r sits at chunk
 // c ^ f(r) with f(r) = (r >> 2) & 3. gfx950's LDS has 64 banks (a 256-byte period) and serves a
 // 64-lane ds_read_b128 in 4 cycles when it is conflict-free; a fragment read (32 rows x 2 chunks)
 // under this f measured 4.0 cycles per instruction and no SQ_LDS_BANK_CONFLICT cycles, where
@@ -398,7 +398,12 @@ __device__ __forceinline__ void tile_coords(uint32_t pid, uint32_t tiles_m, uint
 // measured on gfx950 (rocprofv3 SQ_LDS_IDX_ACTIVE / SQ_INSTS_LDS) at 4.0 cycles per ds_read_b128,
 // the conflict-free minimum. f depends only on r & 15, so fragments 32 rows apart differ by a
 // constant offset.
-__device__ __forceinline__ int swz_f(int row) { return (row >> 2) & 3; }
+// BK = 128: rows of 128 bytes, chunk c (0..7) at c ^ ((r >> 1) & 7): again 16 consecutive rows at one chunk cover the
+// 16 groups of a 256-byte line, and f depends only on r & 15.
+template <int BK = 64>
+__device__ __forceinline__ int swz_f(int row) {
+  return BK == 64 ? (row >> 2) & 3 : (row >> 1) & 7;
+}
 
 // CONVM 3: haloed pixels (a multiple of 16) one halo buffer of a tile with BN columns, S weight stages and
 // NW waves holds: what the LDS leaves after the weight stages and the sink, and what the loads can carry
@@ -409,7 +414,10 @@ __host__ __device__ constexpr int conv_halo_max(int bn, int s, int nw) {
   const int by_loads = (10 - s) * nw * 16;
   return by_lds < by_loads ? by_lds : by_loads;
 }
-__device__ __forceinline__ int swz(int row, int chunk) { return (row << 6) + ((chunk ^ swz_f(row)) << 4); }
+template <int BK = 64>
+__device__ __forceinline__ int swz(int row, int chunk) {
+  return row * BK + ((chunk ^ swz_f<BK>(row)) << 4);
+}
 
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
@@ -464,14 +472,14 @@ struct PinTwo {
   }
 };
 
-// Tile engine. Each 64-deep K slice of the A and W tiles is brought into LDS by the DMA form of the
-// buffer load: one wave instruction fills 16 whole 64-byte LDS rows, and each lane fetches the global
+// Tile engine. Each BK-deep K slice (64 or 128 bytes) of the A and W tiles is brought into LDS by the DMA form of
+// the buffer load: one wave instruction fills 1024 / BK whole LDS rows, and each lane fetches the global
 // chunk that belongs at its LDS position under the swizzle. S LDS stages hold slices kt .. kt+S-1, so
-// the loads of a slice have S - 1 slices of MFMAs to land. Per slice kt (two 32-deep MFMA steps):
-//   step 0: MFMAs of the step-0 fragments, with the reads of the step-1 fragments in between;
+// the loads of a slice have S - 1 slices of MFMAs to land. Per slice kt (NS = BK / 32 MFMA steps):
+//   steps 0 .. NS-2: MFMAs of the step's fragments, with the reads of the next step's fragments in between;
 //   wait for this wave's DMA of slice kt+1; barrier (every wave has read all of slice kt, and slice
 //   kt+1 is complete);
-//   step 1: MFMAs of the step-1 fragments, with the DMA of slice kt+S into slice kt's stage and the
+//   step NS-1: its MFMAs, with the DMA of slice kt+S into slice kt's stage and the
 //   reads of slice kt+1's step-0 fragments in between.
 // Slices past the end of K are loaded as out-of-range (zero) reads, which keeps the wait counts and
 // the loop uniform.
@@ -489,21 +497,24 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-template <int BM, int BN, int WM, int WN, int S, int CONVM, int EPI, bool KFULL, int KG = 1, bool PP = false>
+template <int BM, int BN, int WM, int WN, int S, int CONVM, int EPI, bool KFULL, int KG = 1, bool PP = false,
+          int BK = 64>
 __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t* __restrict__ a, int64_t lda,
                                                                const int8_t* __restrict__ w, int64_t ldw, int64_t M,
                                                                int64_t N, int64_t K, ConvGeom cg, EpiArgs e) {
   // CONVM: 0 GEMM, 1 conv with C_pad % 64 == 0, 2 any C_pad, 3 conv from a haloed input tile (below)
   constexpr bool CONV = CONVM != 0;
   constexpr bool HALO = CONVM == 3;
-  constexpr int BK = 64;
+  static_assert(BK == 64 || (BK == 128 && !HALO && !PP), "slices of 64 or 128 bytes");
+  constexpr int RPI = 1024 / BK;         // rows of one DMA instruction
+  constexpr int NS = BK / 32;            // MFMA steps of a slice
   constexpr int NW = WM * WN;
   constexpr int TM = BM / WM, TN = BN / WN;
   constexpr int FM = TM / 32, FN = TN / 32;  // 32 x 32 MFMA tiles per wave
-  constexpr int IA = BM / 16 / NW;       // DMA instructions per wave per slice (16 rows each)
-  constexpr int IW = BN / 16 / NW;
+  constexpr int IA = BM / RPI / NW;      // DMA instructions per wave per slice (RPI rows each)
+  constexpr int IW = BN / RPI / NW;
   static_assert(FM >= 1 && FN >= 1, "wave tile below 32 x 32");
-  static_assert(IA >= 1 && IW >= 1 && BM % (16 * NW) == 0 && BN % (16 * NW) == 0, "tile / wave mismatch");
+  static_assert(IA >= 1 && IW >= 1 && BM % (RPI * NW) == 0 && BN % (RPI * NW) == 0, "tile / wave mismatch");
   // CONVM 3: the K slices are (64-channel slice, tap) pairs, taps inner. The stages hold only the weight
   // slices; the tile's input pixels plus a one-pixel border ("halo"), one channel slice at a time, sit in
   // two halo buffers after them (the slice being read, the next one being loaded), then a 1 KB sink for
@@ -557,10 +568,10 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
   const __amdgpu_buffer_rsrc_t ra_rsrc = make_rsrc(a, (uint32_t)(CONV ? (conv_px * cg.c_pad) : (M * lda)));
   const __amdgpu_buffer_rsrc_t rw_rsrc = make_rsrc(w, (uint32_t)(N * ldw));
 
-  // This lane's rows: DMA instruction j of this wave covers tile rows r0 = (wave * I + j) * 16 .. +16,
-  // and lane l fills LDS chunk l % 4 of row r0 + l / 4, i.e. logical chunk (l % 4) ^ f(row).
-  const int lrow = lane >> 2;
-  const int pch = lane & 3;
+  // This lane's rows: DMA instruction j of this wave covers tile rows r0 = (wave * I + j) * RPI .. + RPI,
+  // and lane l fills LDS chunk l % (BK / 16) of row r0 + l / (BK / 16), i.e. logical chunk (l % (BK / 16)) ^ f(row).
+  const int lrow = lane / (BK / 16);
+  const int pch = lane & (BK / 16 - 1);
   uint32_t oa[IA], ow[IW];
   int ca[IA], cw[IW];                    // logical chunk per slot
   int py[IA], px[IA];
@@ -570,8 +581,8 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
   (void)ca;
 #pragma unroll
   for (int j = 0; j < (HALO ? 0 : IA); ++j) {
-    const int row = (wave * IA + j) * 16 + lrow;
-    ca[j] = pch ^ swz_f(row);
+    const int row = (wave * IA + j) * RPI + lrow;
+    ca[j] = pch ^ swz_f<BK>(row);
     const int64_t m = m0 + row;
     if constexpr (CONV) {
       // 32-bit: M * c_pad stays below 2^30 (the launcher splits larger batches)
@@ -588,8 +599,8 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
   }
 #pragma unroll
   for (int j = 0; j < IW; ++j) {
-    const int row = (wave * IW + j) * 16 + lrow;
-    cw[j] = pch ^ swz_f(row);
+    const int row = (wave * IW + j) * RPI + lrow;
+    cw[j] = pch ^ swz_f<BK>(row);
     const int64_t n = n0 + row;
     ow[j] = n < N ? (uint32_t)(n * ldw + cw[j] * 16) : OOB;
   }
@@ -667,7 +678,7 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
   }
   // CONVM 1: a group's slices are issued in order, KG slices apart, so the tap and channel offset of
   // its next slice are kept as running counters instead of being divided out of k (the launcher takes
-  // CONVM 1 with KG > 1 only when c_pad is a multiple of KG * 64, so each step wraps at most once).
+  // CONVM 1 only when c_pad is a multiple of KG * BK, so each step wraps at most once).
   int dtap = 0, dc0 = 0;
   if constexpr (CONVM == 1) {
     dtap = (kg * BK) / (int)cg.c_pad;
@@ -675,13 +686,18 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
   }
   (void)dtap;
   (void)dc0;
+  // CONVM 2: 16-byte chunks per tap and their reciprocal (0: divide)
+  const uint32_t c2_cp = CONVM == 2 ? (uint32_t)(cg.c_pad >> 4) : 1u;
+  const uint32_t c2_inv = CONVM == 2 && c2_cp > 1 && c2_cp < 16384 ? 0xffffffffu / c2_cp + 1u : 0u;
+  (void)c2_cp;
+  (void)c2_inv;
   auto dma_slice = [&](int64_t kt, int8_t* stage) {
     const int64_t k0 = (kbase + kt) * BK;
     const bool live = kt < nk;           // uniform; dead slices read zeros without memory traffic
     int8_t* sa = stage;
     int8_t* sw = stage + BM * BK;
     if constexpr (CONVM == 1) {
-      // C_pad % 64 == 0: the whole slice is one tap
+      // C_pad % BK == 0: the whole slice is one tap
       const int dy = (dtap >= 3) + (dtap >= 6) - 1;
       const int dx = dtap - 3 * (dy + 1) - 1;
       const int64_t delta = ((int64_t)dy * cg.w + dx) * cg.c_pad + dc0;
@@ -699,17 +715,19 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
     } else if constexpr (CONVM == 2) {
 #pragma unroll
       for (int j = 0; j < IA; ++j) {
-        const uint32_t kb = (uint32_t)k0 + ca[j] * 16;
-        const uint32_t tap = kb / (uint32_t)cg.c_pad;
-        const uint32_t c = kb - tap * (uint32_t)cg.c_pad;
-        const int dy = (int)(tap / 3) - 1, dx = (int)(tap % 3) - 1;
-        const int sy = py[j] + dy, sx = px[j] + dx;
-        const bool ok = kb < K && sy >= 0 && sy < cg.h && sx >= 0 && sx < cg.w;
-        const int64_t delta = ((int64_t)dy * cg.w + dx) * cg.c_pad + c;
-        dma16(ra_rsrc, ok ? (uint32_t)(oa[j] + delta) : OOB, sa + ((wave * IA + j) << 10));
+        // tap = chunk / (c_pad / 16) as a product with the rounded-up reciprocal (exact below 9 taps for c_pad under
+        // 2^18: the error, chunk * cp16 / 2^32 at most, stays below 1 / cp16); wider inputs divide
+        const uint32_t kc = ((uint32_t)k0 >> 4) + (uint32_t)ca[j];
+        const uint32_t tap = c2_inv ? __umulhi(kc, c2_inv) : kc / c2_cp;
+        const uint32_t c = (kc - tap * c2_cp) << 4;
+        const int dy = (int)((tap * 11u) >> 5), dx = (int)tap - 3 * dy;   // tap / 3 and tap % 3 for tap < 9
+        const int sy = py[j] + dy - 1, sx = px[j] + dx - 1;
+        const bool ok = kc < (uint32_t)(K >> 4) && (uint32_t)sy < (uint32_t)cg.h && (uint32_t)sx < (uint32_t)cg.w;
+        const uint32_t off = oa[j] + (uint32_t)((dy - 1) * (int)cg.w + dx - 1) * (uint32_t)cg.c_pad + c;
+        dma16(ra_rsrc, ok ? off : OOB, sa + ((wave * IA + j) << 10));
       }
     } else {
-      if (KFULL) {                         // K % 64 == 0: the per-slot offsets are constant
+      if (KFULL) {                         // K % BK == 0: the per-slot offsets are constant
 #pragma unroll
         for (int j = 0; j < IA; ++j)
           dma16(ra_rsrc, live ? oa[j] : OOB, sa + ((wave * IA + j) << 10), live ? (uint32_t)k0 : 0u);
@@ -735,7 +753,7 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
     }
   };
 
-  // Fragments of one 32-deep k step ks (2 per slice): lane l holds 16 bytes of row
+  // Fragments of one 32-deep k step ks (NS per slice): lane l holds 16 bytes of row
   // (frag base + l % 32) at logical chunk 2 * ks + l / 32. Two register sets alternate: while the
   // MFMAs of one step run, the fragments of the next are read into the other set.
   const int frow = lane & 31;
@@ -744,10 +762,10 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
   auto read_frags = [&](const int8_t* stage, int ks, int set) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
-      fa[set][i] = *reinterpret_cast<const i32x4*>(stage + swz(wm * TM + i * 32 + frow, ks * 2 + fk));
+      fa[set][i] = *reinterpret_cast<const i32x4*>(stage + swz<BK>(wm * TM + i * 32 + frow, ks * 2 + fk));
 #pragma unroll
     for (int j = 0; j < FN; ++j)
-      fw[set][j] = *reinterpret_cast<const i32x4*>(stage + BM * BK + swz(wn * TN + j * 32 + frow, ks * 2 + fk));
+      fw[set][j] = *reinterpret_cast<const i32x4*>(stage + BM * BK + swz<BK>(wn * TN + j * 32 + frow, ks * 2 + fk));
   };
   // CONVM 3: the input fragment of a slice comes from its channel slice's halo buffer hb, each row at its
   // haloed pixel moved by the tap (dy, dx): toff = dy * hw_halo + dx
@@ -914,19 +932,22 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
     int8_t* cur = lds + cur_s * STAGE;
     const int nxt_s = cur_s + 1 == S ? 0 : cur_s + 1;
     const int8_t* nxt = lds + nxt_s * STAGE;
-    // step 0
-    read_frags(cur, 1, 1);
-    mfmas(0);
-    PinGroups<SG_DS_READ, NRD, NMF, 0>::emit();
-    __builtin_amdgcn_sched_barrier(0);
+    // steps 0 .. NS-2
+    static_for<0, NS - 1>([&](auto sc) {
+      constexpr int ks = decltype(sc)::value;
+      read_frags(cur, ks + 1, (ks + 1) & 1);
+      mfmas(ks & 1);
+      PinGroups<SG_DS_READ, NRD, NMF, 0>::emit();
+      __builtin_amdgcn_sched_barrier(0);
+    });
     // slice kt+1 landed (this wave's part), this wave's reads of slice kt done; then all waves
     wait_vmcnt_lgkm0<(S - 2) * NDMA>();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    // step 1
+    // step NS-1
     dma_slice(kt + (int64_t)KG * S, cur);
     read_frags(nxt, 0, 0);
-    mfmas(1);
+    mfmas((NS - 1) & 1);
     PinTwo<SG_VMEM_READ, NDMA, SG_DS_READ, NRD, NMF>::emit();
     __builtin_amdgcn_sched_barrier(0);
     cur_s = nxt_s;
@@ -1753,70 +1774,93 @@ int launch_tiles_once(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw
       grid.y = (unsigned)ks;
     }
   }
-  const bool kfull = K % 64 == 0;
-  // LDS stages per tile shape, from a measured sweep of 3 / 4 / 5 (and 4 / 8 / 12 for 64 x 64): 3 for
-  // the large tiles (96 KB at 256 x 256; 48 KB at 128 x 128, three workgroups per CU), 4 for 64 x 64
-#define XDNA_TILE_WK(BM_, BN_, WM_, WN_, S_, KG_)                                                             \
-  if (kfull) mm_tile_kernel<BM_, BN_, WM_, WN_, S_, CONVM, EPI, true, KG_><<<grid, WM_ * WN_ * KG_ * 64, 0, st>>>(a, lda, w, ldw, M, N, K, cg, e); \
-  else mm_tile_kernel<BM_, BN_, WM_, WN_, S_, CONVM, EPI, false, KG_><<<grid, WM_ * WN_ * KG_ * 64, 0, st>>>(a, lda, w, ldw, M, N, K, cg, e);
-#define XDNA_TILE_W(BM_, BN_, WM_, WN_, S_) XDNA_TILE_WK(BM_, BN_, WM_, WN_, S_, 1)
-#define XDNA_TILE(BM_, BN_, S_) XDNA_TILE_W(BM_, BN_, 2, 2, S_)
+  // K slices of 128 bytes (whole cache lines) or 64, and LDS stages, per tile. With 64-byte slices a line's second
+  // half is fetched a slice later, by which time a large tile's other rows have pushed it out of the 32 KB L1: 5.2M
+  // line requests to the L2 for 6.0M half-line loads at 699 x 14336 x 4096 in 256 x 256 tiles. 128-byte slices ask
+  // for each line once and pass half as many barriers. Same LDS bytes in flight, measured 64 -> 128 (int8 unless
+  // stated): 256 x 256 with 8 waves (3 -> 2 stages) 8192 x 14336 x 4096 449 -> 429 us; 256 x 128 / 128 x 256 with 8
+  // waves (4 -> 3) 1999 x 4096 x 4096 41.4 -> 37.1 us; 64 x 64 (4 -> 3) 512 x 4096 x 4096 18.6 -> 15.8 us, bf16 486 x
+  // 4096 x 1024 10.6 -> 9.3 us; 32 x 64 (4) 32 x 4096 x 14336 18.5 -> 15.4 us. The tiles with K groups keep 64
+  // bytes (64 x 64 in 2 groups, 200 x 4096 x 4096: 10.2 against 12.6 us), except 128 x 128 in 2 (bf16 2000 x 2048 x
+  // 4096 38.6 -> 36.8 us).
+#define XDNA_TILE_K(BM_, BN_, WM_, WN_, S_, KG_, BK_)                                                         \
+  if (K % BK_ == 0) mm_tile_kernel<BM_, BN_, WM_, WN_, S_, CONVM, EPI, true, KG_, false, BK_><<<grid, WM_ * WN_ * KG_ * 64, 0, st>>>(a, lda, w, ldw, M, N, K, cg, e); \
+  else mm_tile_kernel<BM_, BN_, WM_, WN_, S_, CONVM, EPI, false, KG_, false, BK_><<<grid, WM_ * WN_ * KG_ * 64, 0, st>>>(a, lda, w, ldw, M, N, K, cg, e);
+  // S64 / S128: stages with 64- and 128-byte slices; a conv takes the long ones where a slice stays within one tap
+#define XDNA_TILE(BM_, BN_, WM_, WN_, KG_, S64_, S128_)                                                       \
+  if constexpr (CONVM == 0) {                                                                                 \
+    XDNA_TILE_K(BM_, BN_, WM_, WN_, S128_, KG_, 128)                                                          \
+  } else if constexpr (CONVM == 1) {                                                                          \
+    if (cg.c_pad % (128 * KG_) == 0) {                                                                        \
+      XDNA_TILE_K(BM_, BN_, WM_, WN_, S128_, KG_, 128)                                                        \
+    } else {                                                                                                  \
+      XDNA_TILE_K(BM_, BN_, WM_, WN_, S64_, KG_, 64)                                                          \
+    }                                                                                                         \
+  } else {                                                                                                    \
+    XDNA_TILE_K(BM_, BN_, WM_, WN_, S64_, KG_, 64)                                                            \
+  }
   if constexpr (CONVM == 3) {
     // the haloed conv: the 8-wave 256 x 256 tile (3 stages) and, for tails, the 8-wave 128 x 256 (4 stages)
     if (tile == T_256x256W8) {
-      XDNA_TILE_W(256, 256, 2, 4, 3)
+      XDNA_TILE_K(256, 256, 2, 4, 3, 1, 64)
     } else {
-      XDNA_TILE_W(128, 256, 2, 4, 4)
+      XDNA_TILE_K(128, 256, 2, 4, 4, 1, 64)
     }
   } else if (tile == T_256x256PP) {
     // the ping-pong schedule: 4 stages (S - 2 = 2 slices between a DMA and its use)
-    if (kfull) mm_tile_kernel<256, 256, 2, 4, 4, CONVM, EPI, true, 1, true><<<grid, 512, 0, st>>>(a, lda, w, ldw, M, N, K, cg, e);
+    if (K % 64 == 0) mm_tile_kernel<256, 256, 2, 4, 4, CONVM, EPI, true, 1, true><<<grid, 512, 0, st>>>(a, lda, w, ldw, M, N, K, cg, e);
     else mm_tile_kernel<256, 256, 2, 4, 4, CONVM, EPI, false, 1, true><<<grid, 512, 0, st>>>(a, lda, w, ldw, M, N, K, cg, e);
   } else if (t.kg > 1) {
     // K groups (in-workgroup split-K) for tiles with few tiles and deep K
     if (t.bm == 128) {
-      XDNA_TILE_WK(128, 128, 2, 2, 4, 2)
+      XDNA_TILE(128, 128, 2, 2, 2, 4, 2)
     } else if (t.bm == 64 && t.kg == 2) {
-      XDNA_TILE_WK(64, 64, 2, 2, 4, 2)
+      XDNA_TILE_K(64, 64, 2, 2, 4, 2, 64)
     } else if (t.bm == 64) {
-      XDNA_TILE_WK(64, 64, 2, 2, 4, 4)
+      XDNA_TILE_K(64, 64, 2, 2, 4, 4, 64)
     } else if (t.bn == 64) {
-      XDNA_TILE_WK(32, 64, 1, 2, 4, 4)
+      XDNA_TILE_K(32, 64, 1, 2, 4, 4, 64)
     } else {
-      XDNA_TILE_WK(32, 32, 1, 1, 4, 4)
+      XDNA_TILE_K(32, 32, 1, 1, 4, 4, 64)
     }
   } else if (t.waves == 8 && t.bm == 128) {
-    XDNA_TILE_W(128, 256, 2, 4, 4)
+    XDNA_TILE(128, 256, 2, 4, 1, 4, 3)
   } else if (t.waves == 8 && t.bn == 128) {
-    XDNA_TILE_W(256, 128, 4, 2, 4)
+    XDNA_TILE(256, 128, 4, 2, 1, 4, 3)
   } else if (t.bm == 256 && t.bn == 64) {
-    XDNA_TILE_W(256, 64, 4, 1, 4)
+    XDNA_TILE(256, 64, 4, 1, 1, 4, 2)
   } else if (t.bm == 256 && t.bn == 256 && t.waves == 8) {
-    XDNA_TILE_W(256, 256, 2, 4, 3)
+    XDNA_TILE(256, 256, 2, 4, 1, 3, 2)
   } else if (t.bm == 256 && t.bn == 256) {
-    XDNA_TILE(256, 256, 4)
+    XDNA_TILE(256, 256, 2, 2, 1, 4, 2)
   } else if (t.bm == 192) {
-    XDNA_TILE(192, 256, 4)
+    XDNA_TILE(192, 256, 2, 2, 1, 4, 2)
   } else if (t.bn == 192) {
-    XDNA_TILE(256, 192, 4)
+    XDNA_TILE(256, 192, 2, 2, 1, 4, 2)
   } else if (t.bm == 256) {
-    XDNA_TILE(256, 128, 4)
+    XDNA_TILE(256, 128, 2, 2, 1, 4, 3)
   } else if (t.bn == 256) {
-    XDNA_TILE(128, 256, 4)
+    XDNA_TILE(128, 256, 2, 2, 1, 4, 3)
   } else if (t.bm == 128) {
-    XDNA_TILE(128, 128, 3)
+    // more than one tile per CU and some depth: long slices (1999 x 4096 x 4096 43.8 -> 38.1 us, bf16 2000 x 6144 x
+    // 1024 32.4 -> 30.1); else three workgroups per CU of short ones start and finish sooner (699 x 4096 x 1024 9.3
+    // against 9.9 us, bf16 486 x 6144 x 1024 12.7 against 13.8, 2000 x 2048 x 4096 39.1 against 42.3)
+    if (tiles > device_cus() && K >= 2048) {
+      XDNA_TILE(128, 128, 2, 2, 1, 3, 2)
+    } else {
+      XDNA_TILE_K(128, 128, 2, 2, 3, 1, 64)
+    }
   } else if (t.bn == 32 && t.bm == 64) {
-    XDNA_TILE_W(64, 32, 2, 1, 4)
+    XDNA_TILE(64, 32, 2, 1, 1, 4, 4)
   } else if (t.bm == 32 && t.bn == 64) {
-    XDNA_TILE_W(32, 64, 1, 2, 4)
+    XDNA_TILE(32, 64, 1, 2, 1, 4, 4)
   } else if (t.bm == 32) {
-    XDNA_TILE_W(32, 32, 1, 1, 4)
+    XDNA_TILE(32, 32, 1, 1, 1, 4, 4)
   } else {
-    XDNA_TILE(64, 64, 4)
+    XDNA_TILE(64, 64, 2, 2, 1, 4, 3)
   }
 #undef XDNA_TILE
-#undef XDNA_TILE_W
-#undef XDNA_TILE_WK
+#undef XDNA_TILE_K
   return launch_status("mm_tile");
 }
 
