@@ -739,6 +739,23 @@ def test_tiles_slices(gpu, tile, tile_table):
                               O.requant(c_oracle.conv3x3_acc(xq.numpy(), wq.numpy()), 9, False)), (n, ci, co, h, w_)
 
 
+@pytest.mark.parametrize("m,n,k", [(16, 8192, 4096), (17, 5120, 1024), (17, 5104, 1024), (33, 2560, 2064), (64, 12900, 512),
+                                   (65, 1001, 1552), (257, 1000, 1024), (513, 1024, 1040), (768, 16384, 1024),
+                                   (340, 14336, 1024)])
+def test_rule_tiles(gpu, m, n, k, tile_table):
+    """Shapes on both sides of the tile rule's lines (small-M kernel or engine, K groups, one round of the large
+    tiles), as the rule plans them: int32 sums exact and, for bf16 operands of the same bytes, within 1e-5
+    of the float64 product's norm (float32 sums: about 2^-24 times the square root of K roundings)."""
+    a, w = _i8((m, k), seed=m + k), _i8((n, k), seed=n + k)
+    want = torch._int_mm(torch.cat([a, a.new_zeros(max(0, 17 - m), k)]), w.t().contiguous())[:m]
+    assert torch.equal(tile_table.mm_i8(a.to(gpu), w.to(gpu)).cpu(), want)
+    x = _rand((m, k // 2), torch.float32, seed=m).to(torch.bfloat16).to(gpu)
+    v = _rand((n, k // 2), torch.float32, seed=n, scale=0.05).to(torch.bfloat16).to(gpu)
+    y = tile_table.mm_bf16(x, v, None, torch.float32)
+    ref = x.double() @ v.double().t()
+    assert float((y.double() - ref).norm() / ref.norm()) < 1e-5
+
+
 def _ksplit(cus, bm, bn, kg, tiles, k):
     """Workgroups per tile along K that the library gives a launch: 1 above 64 x 64 or when the tiles fill
     more than half of the CUs, else up to CUs / tiles, at most 16, with at least 16 slices of 64 per K

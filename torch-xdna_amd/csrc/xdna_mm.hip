@@ -1658,38 +1658,56 @@ int tile_lookup(int kind, int64_t m, int64_t n, int64_t k) {
   return it == g_tiles.end() ? T_AUTO : it->second;
 }
 
-// The built-in rule, from back-to-back timed sweeps of every tile shape over the BASELINE GEMM and
-// conv shapes on MI355X (t128 / t256: tiles of that size the problem needs; kbytes: K in bytes):
+// The built-in rule, from back-to-back timed sweeps of every tile shape (rotating weights; kbytes: K in bytes):
 //   * M == 1: the one-row kernel, 4 waves (one output column each) per workgroup;
 //   * 2 <= M <= 8 with K of at least 2 KB: the few-row kernel, 8 output columns per workgroup;
-//   * M <= 64 (decode): the small-M kernel, 2 waves per workgroup, 4 once K exceeds 8 KB;
+//   * M <= 64 with a weight small enough that reading it again for every 16 rows stays cheap (5 MB, or 32 MB up to 16
+//     rows): the small-M kernel, 2 waves per workgroup, 4 once K exceeds 8 KB. Either side of the line, int8, small-M
+//     kernel / tile: 64 x 1024 x 3072 5.0 / 5.7 us, bf16 40 x 1024 x 2048 5.6 / 5.9, 20 x 12900 x 512 6.2 / 4.7, bf16
+//     40 x 4096 x 1024 7.5 / 4.8, 40 x 14336 x 4096 42 / 16.5, 16 x 4096 x 4096 6.1 / 6.3, 16 x 14336 x 4096 18 / 14.7;
+//   * GEMMs with few tiles and K of at least 1 KB: the smallest of 32 x 32, 32 x 64 (4 K groups each) and, from 2 KB,
+//     64 x 64 (2 groups) that makes at most one round of workgroups (128 x 1024 x 3072 5.7 against 7.1 us in 32 x 64,
+//     200 x 1001 x 1552 5.4 against 7.8 in 64 x 64 without groups, 512 x 1001 x 1552 7.2 against 8.1);
+//   * convs with few tiles and K of at least 2 KB: 32 x 32 x 4 groups below an eighth of a round of 64 x 64 tiles,
+//     32 x 64 x 4 groups up to half a round, 64 x 64 x 2 groups up to a round;
 //   * 64 x 64 for N <= 64; for N <= 128 no 256-wide tile (half of it would be idle);
-//   * 256 x 256 with 8 waves (one workgroup per CU) from 1.5 rounds of such tiles, or from three
-//     quarters of a round for deep K (>= 4096 bytes), where its lower LDS traffic per MAC outweighs
-//     the idle CUs;
+//   * 256 x 256 with 8 waves (one workgroup per CU) from 1.5 rounds of such tiles, from three quarters of a round for
+//     deep K (>= 4096 bytes), where its lower LDS traffic per MAC outweighs the idle CUs, and, GEMMs, between three
+//     quarters and one round (3000 x 4096 x 1024 21.5 against 23.3 us in 128 x 128); then, GEMMs of K of at least 1 KB,
+//     192 x 256 (699 x 14336 x 4096 50 against 61 us) and the 8-wave 256 x 128 (333 x 14336 x 4096 32 against 36 us,
+//     bf16 1056 x 6144 x 1024 19.1 against 20.1) where they make 0.8 to 1 round;
 //   * otherwise, once 128 x 128 tiles fill three quarters of the CUs: 128 x 256 (four waves) for deep K
-//     when there are at least half a round of 256-wide tiles, else 128 x 128 (three workgroups per CU);
-//   * smaller problems with deep K (at least 2 KB): tiles whose workgroups split K between wave groups,
-//     32 x 32 x 4 groups below an eighth of a round of 64 x 64 tiles, 32 x 64 x 4 groups up to half a
-//     round, 64 x 64 x 2 groups up to a round;
+//     when there are at least half a round of 256-wide tiles, else 128 x 128;
 //   * 64 x 64 otherwise.
 // A shape the tuned table lists uses the table's tile instead.
-int rule_tile(int64_t M, int64_t N, int64_t kbytes, bool small_ok) {
+int rule_tile(int64_t M, int64_t N, int64_t kbytes, bool small_ok, bool conv) {
   if (small_ok && M == 1) return T_GEMV4;
   if (small_ok && M <= 8 && kbytes >= 2048) return T_SEG4R2;
-  if (small_ok && M <= 64) return (kbytes + 63) / 64 > 128 ? T_SMALL4 : T_SMALL2;
+  if (small_ok && M <= 64 && N * kbytes < (M <= 16 ? int64_t(32) << 20 : int64_t(5) << 20))
+    return (kbytes + 63) / 64 > 128 ? T_SMALL4 : T_SMALL2;
   const int64_t cus = device_cus();
+  auto tiles = [&](int64_t bm, int64_t bn) { return cdiv(M, bm) * cdiv(N, bn); };
+  const int64_t t64 = tiles(64, 64), t128 = tiles(128, 128), t256 = tiles(256, 256);
+  if (!conv && kbytes >= 1024) {
+    if (tiles(32, 32) <= cus) return T_32x32K4;
+    if (tiles(32, 64) <= cus) return T_32x64K4;
+    if (kbytes >= 2048 && t64 <= cus) return T_64x64K2;
+  }
+  if (!conv && M <= 32) return T_32x64;
   // narrow outputs with rows for at least two rounds of 256 x 64 tiles (the VGG-16 224 x 224 convs): a
   // quarter of the 64 x 64 tiles, each paying its fixed prologue / epilogue cost once for four times the work
-  if (N <= 64 && ((M + 255) / 256) * ((N + 63) / 64) >= 2 * cus) return T_256x64;
+  if (N <= 64 && tiles(256, 64) >= 2 * cus) return T_256x64;
   if (M <= 64 || N <= 64) return T_64x64;
-  const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
-  const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
   const bool deep = kbytes >= 4096;
   if (N > 128 && (2 * t256 >= 3 * cus || (deep && 4 * t256 >= 3 * cus))) return T_256x256W8;
+  if (!conv && N > 128) {
+    auto round = [&](int64_t t) { return 5 * t >= 4 * cus && t <= cus; };
+    if (4 * t256 >= 3 * cus && t256 <= cus) return T_256x256W8;
+    if (kbytes >= 1024 && round(tiles(192, 256))) return T_192x256;
+    if (kbytes >= 1024 && round(tiles(256, 128))) return T_256x128W8;
+  }
   if (4 * t128 >= 3 * cus) return (N > 128 && deep && 2 * t256 >= cus) ? T_128x256 : T_128x128;
   if (kbytes >= 2048) {
-    const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
     if (8 * t64 < cus) return T_32x32K4;
     if (2 * t64 <= cus) return T_32x64K4;
     if (t64 <= cus) return T_64x64K2;
@@ -1703,7 +1721,7 @@ int choose_tile(int kind, int64_t m, int64_t n, int64_t k, int64_t kbytes) {
   if (t == T_DIRECT && !(kind == XDNA_KIND_CONV && direct_ok(n, k))) t = T_AUTO;   // not a shape it takes
   if (t != T_AUTO) return t;
   if (kind == XDNA_KIND_CONV && direct_ok(n, k)) return T_DIRECT;
-  return rule_tile(m, n, kbytes, kind != XDNA_KIND_CONV);
+  return rule_tile(m, n, kbytes, kind != XDNA_KIND_CONV, kind == XDNA_KIND_CONV);
 }
 
 // Buffer resources address at most 2 GB; larger operands are processed in row chunks.
@@ -1896,7 +1914,7 @@ TilePlan plan_tiles(int kind, int64_t M, int64_t N, int64_t kbytes, int64_t ktab
   int tail = tile_lookup(kind, M - m1, N, ktab);
   if (is_small(tail) || is_gemv(tail) || is_seg4(tail) || tail == T_DIRECT) tail = T_AUTO;
   if (tail == T_AUTO)
-    tail = (tile == T_256x256W8 || tile == T_256x256PP) ? T_128x256W8 : rule_tile(M - m1, N, kbytes, false);
+    tail = (tile == T_256x256W8 || tile == T_256x256PP) ? T_128x256W8 : rule_tile(M - m1, N, kbytes, false, kind == XDNA_KIND_CONV);
   // only when the leftover rows fit one round of the tail's tiles (8192 x 3072 in 256 x 256 tiles leaves
   // 2816 rows, 264 tiles of 128 x 256: measured slower split than not)
   const TileCfg tt = tile_cfg(tail);
@@ -1948,11 +1966,11 @@ int launch_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, int6
                 const EpiArgs& e, int tile, hipStream_t st) {
   // the one-row kernel takes one row; the small-M kernel addresses the whole activation with one buffer
   // resource, 16 rows per grid row
-  if (is_gemv(tile) && M != 1) tile = rule_tile(M, N, K, M > 1);
-  if (is_seg4(tile) && M > 16) tile = rule_tile(M, N, K, true);
+  if (is_gemv(tile) && M != 1) tile = rule_tile(M, N, K, M > 1, false);
+  if (is_seg4(tile) && M > 16) tile = rule_tile(M, N, K, true, false);
   // the one-row and few-row kernels write one column per lane: the fused SiLU needs a column's partner
   if (EPI == EPI_BF_SILU && (is_gemv(tile) || is_seg4(tile))) tile = T_SMALL2;
-  if (is_small(tile) && (M * lda > MAX_BUF || (M + 15) / 16 >= 65536)) tile = rule_tile(M, N, K, false);
+  if (is_small(tile) && (M * lda > MAX_BUF || (M + 15) / 16 >= 65536)) tile = rule_tile(M, N, K, false, false);
   if constexpr (EPI != EPI_BF_SILU) {
   if (is_seg4(tile)) {
     // four rows per segment group; the workgroup's 4 waves split K into multiples of 256 bytes
@@ -2388,7 +2406,7 @@ int launch_conv(const int8_t* x, int64_t nb, int64_t h, int64_t w, int64_t c_pad
         continue;
       }
     }
-    const int etile = tile == T_DIRECT ? rule_tile(nb * h * w, co, K, false) : tile;
+    const int etile = tile == T_DIRECT ? rule_tile(nb * h * w, co, K, false, true) : tile;
     // the haloed input tile where the tile allows it; the running tap counters of CONVM 1 step by KG
     // slices of 64 channels
     const int mode = conv_mode(etile, h, w, c_pad);
@@ -2607,9 +2625,9 @@ int xdna_tile_plan(int kind, int64_t m, int64_t n, int64_t k, int* head, int64_t
   // the launchers' own substitutions: the one-row and few-row kernels take only their row counts, and
   // the small-M kernel addresses the whole activation with one buffer resource
   if (kind != XDNA_KIND_CONV) {
-    if (is_gemv(t) && m != 1) t = rule_tile(m, n, kbytes, m > 1);
-    if (is_seg4(t) && m > 16) t = rule_tile(m, n, kbytes, true);
-    if (is_small(t) && (m * kbytes > MAX_BUF || (m + 15) / 16 >= 65536)) t = rule_tile(m, n, kbytes, false);
+    if (is_gemv(t) && m != 1) t = rule_tile(m, n, kbytes, m > 1, false);
+    if (is_seg4(t) && m > 16) t = rule_tile(m, n, kbytes, true, false);
+    if (is_small(t) && (m * kbytes > MAX_BUF || (m + 15) / 16 >= 65536)) t = rule_tile(m, n, kbytes, false, false);
   }
   // GEMM operands above one buffer resource run in row chunks (with dense rows, lda = k): the plan of
   // the first chunk
