@@ -79,6 +79,47 @@ def test_quant_rows_ties_zero_rows_strided(gpu):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("rows,k,ld,k_pad", [(5, 15, 15, 16), (7, 17, 19, 48), (3, 1023, 1023, 1024), (4, 1024, 1031, 1024),
+                                             (6, 1025, 1025, 1040), (2, 2049, 2051, 2064), (5, 4097, 4097, 4112),
+                                             (2, 16383, 16383, 16400), (1, 16385, 16385, 16400), (3, 1000, 1001, 1000)])
+def test_quant_rows_ragged(gpu, dtype, rows, k, ld, k_pad):
+    """Rows that start off 16 bytes (odd strides, a base one element in) at the edges of the wave's and the block's
+    16-element groups, one whose last group has no room in its output row, one longer than the registers hold:
+    integers and scales against the oracle, padding zero, also for a row with a NaN (its scale NaN)."""
+    from torch_xdna import kernels
+
+    x = _rand((rows, ld), DT[dtype], seed=k, outliers=1e-3)
+    if rows > 2:
+        x[2, k // 2] = float("nan")
+    buf = torch.empty(rows * ld + 1, dtype=DT[dtype], device=gpu)
+    buf[1:].copy_(x.reshape(-1))
+    q = torch.full((rows, k_pad), 77, dtype=torch.int8, device=gpu)
+    s = torch.empty(rows, dtype=torch.float32, device=gpu)
+    kernels.quant_rows(buf[1:].view(rows, ld)[:, :k], k_pad, out=(q, s))
+    wq, ws = O.quant_rows(x[:, :k].float().numpy())
+    fine = [r for r in range(rows) if not (rows > 2 and r == 2)]
+    assert np.array_equal(_np(q)[fine, :k], wq[fine]) and np.array_equal(_np(s)[fine], ws[fine])
+    assert rows <= 2 or np.isnan(_np(s)[2])
+    assert not _np(q)[:, k:].any()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("n,ch,h,w,c_pad", [(3, 5, 1, 3, 16), (3, 5, 1, 5, 16), (2, 20, 1, 9, 32), (2, 20, 3, 43, 32),
+                                            (3, 70, 7, 9, 80), (2, 300, 1, 129, 304), (2, 3, 181, 183, 16),
+                                            (2, 40, 95, 97, 48)])
+def test_conv_quant_ragged(gpu, dtype, n, ch, h, w, c_pad):
+    """Images whose pixels are no whole 16-byte loads, down to fewer than one load, at the edges of the pixel tiles,
+    with channels past one tile, and a batch that starts off 16 bytes: against the oracle, padding zero."""
+    from torch_xdna import kernels
+
+    x = _rand((n + 1, ch, h, w), DT[dtype], seed=ch * h + w, outliers=1e-3).to(gpu)[1:]
+    q, s = kernels.conv_quant(x, c_pad)
+    wq, ws = O.conv_quant_images(x.float().cpu().numpy())
+    assert np.array_equal(_np(s), ws.reshape(-1))
+    assert np.array_equal(_np(q)[..., :ch].transpose(0, 3, 1, 2), wq) and not _np(q)[..., ch:].any()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("k", [1024, 200, 16384, 40000])
 def test_quant_rows_near_half(gpu, dtype, k):
     """Quotients x / s placed within 6e-5 of half-integers, on both sides, exactly on them and at fractions

@@ -356,6 +356,94 @@ __global__ __launch_bounds__(256) void quant_rows_stream_kernel(const void* __re
   }
 }
 
+// 16 bytes at any alignment of the elements (global loads take them whole).
+typedef uint32_t u32x4_e4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_e2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_e2 __attribute__((ext_vector_type(2), aligned(2)));
+template <int DT>
+__device__ __forceinline__ uint4 load_u4_any(const void* p) {
+  if constexpr (DT == XDNA_F32) {
+    const u32x4_e4 v = *reinterpret_cast<const u32x4_e4*>(p);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+  } else {
+    const u32x4_e2 v = *reinterpret_cast<const u32x4_e2*>(p);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+  }
+}
+// The first n elements (0 .. Vec16::N) at p, zeros after them, loaded one by one.
+template <int DT>
+__device__ __forceinline__ uint4 load_u4_first(const void* p, int n) {
+  uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int e = 0; e < Vec16<DT>::N; ++e) {
+    if (e < n) {
+      if constexpr (DT == XDNA_F32) w[e] = reinterpret_cast<const uint32_t*>(p)[e];
+      else w[e >> 1] |= (uint32_t) reinterpret_cast<const uint16_t*>(p)[e] << (16 * (e & 1));
+    }
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// Rows of any length and stride (their starts aligned to the element only), kept in registers like those of the
+// kernels above: TPR threads per row (a wave, four rows per block, or the block), thread t owning groups t, t + TPR,
+// ... of 16 elements, read with unaligned 16-byte loads and written as one 16-byte store; the row's last group is
+// read element by element, its padding bytes cleared. Needs 16-byte aligned output rows with room for whole groups.
+// float32 1999 x 1537: 5.7 us, 8.8 us one element per lane with the row read twice.
+template <int DT, int TPR, int G>
+__global__ __launch_bounds__(256) void quant_rows_ragged_kernel(const void* __restrict__ x, int64_t rows, int64_t k,
+                                                                int64_t ld_x, int8_t* __restrict__ q, int64_t ld_q,
+                                                                int64_t k_pad, float* __restrict__ s) {
+  using V = Vec16<DT>;
+  constexpr int VEC = V::N;
+  constexpr int ESZ = (DT == XDNA_F32) ? 4 : 2;
+  constexpr int LPG = 16 / VEC;
+  __shared__ int red[4];
+  const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  const int t = threadIdx.x % TPR;
+  if (TPR == 64 && row >= rows) return;    // wave-uniform, and a wave's row meets no barrier
+  const char* xr = reinterpret_cast<const char*>(x) + row * ld_x * ESZ;
+  const int ki = (int)k;                   // at most 16 TPR G (checked by the launcher)
+  V v[G][LPG];
+#pragma unroll
+  for (int j = 0; j < G; ++j) {
+    const int e0 = (t + j * TPR) * 16;
+    if (e0 + 16 <= ki) {
+#pragma unroll
+      for (int l = 0; l < LPG; ++l) v[j][l].raw = load_u4_any<DT>(xr + (e0 + l * VEC) * ESZ);
+    } else {
+#pragma unroll
+      for (int l = 0; l < LPG; ++l)
+        v[j][l].raw = load_u4_first<DT>(xr + (int64_t)min(e0 + l * VEC, ki) * ESZ, ki - (e0 + l * VEC));
+    }
+  }
+  AbsMaxBits<DT> am;
+#pragma unroll
+  for (int j = 0; j < G; ++j)
+#pragma unroll
+    for (int l = 0; l < LPG; ++l) am.add(v[j][l]);
+  const float amax = group_absmax<DT, TPR>(am, red);
+  const float sc = scale_from_amax(amax);
+  const float rc = 1.0f / sc;
+  if (t == 0) s[row] = sc;
+  int8_t* qr = q + row * ld_q;
+#pragma unroll
+  for (int j = 0; j < G; ++j) {
+    const int e0 = (t + j * TPR) * 16;
+    if (e0 < ki) {
+      float f[16];
+#pragma unroll
+      for (int l = 0; l < LPG; ++l)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) f[l * VEC + e] = v[j][l].get(e);
+      uint32_t w[4], keep[4];
+      quant_pack<16>(f, sc, rc, w);
+      valid_masks(min(16, ki - e0), keep);
+      *reinterpret_cast<uint4*>(qr + e0) = make_uint4(w[0] & keep[0], w[1] & keep[1], w[2] & keep[2], w[3] & keep[3]);
+    }
+  }
+  for (int64_t c = (int64_t)cdiv(k, 16) * 16 + t; c < k_pad; c += TPR) qr[c] = 0;
+}
+
 // Scalar path for any k / stride / alignment: one block per row, the row read twice.
 template <int DT>
 __global__ __launch_bounds__(256) void quant_rows_scalar_kernel(const void* __restrict__ x, int64_t rows, int64_t k,
@@ -394,6 +482,20 @@ int launch_quant_rows(const void* x, int64_t rows, int64_t k, int64_t ld_x, int8
                       float* s, hipStream_t st) {
   constexpr int VEC = (DT == XDNA_F32) ? 4 : 8;
   const bool vec_ok = (k % VEC == 0) && (ld_x % VEC == 0) && aligned(x, 16) && aligned(q, 16) && (ld_q % 16 == 0);
+  // rows without whole 16-element groups or 16-byte starts, into output rows with room for whole groups
+  const int64_t rg = cdiv(k, 16);
+  if (!vec_ok && aligned(q, 16) && ld_q % 16 == 0 && k_pad >= rg * 16 && rg <= 256 * (DT == XDNA_F32 ? 4 : 8)) {
+#define XDNA_QG(TPR_, G_) \
+  quant_rows_ragged_kernel<DT, TPR_, G_><<<dim3((unsigned)cdiv(rows, 256 / TPR_)), 256, 0, st>>>(x, rows, k, ld_x, q, ld_q, k_pad, s)
+    if (rg <= 64) XDNA_QG(64, 1);
+    else if (rg <= 128) XDNA_QG(64, 2);
+    else if (rg <= 256) XDNA_QG(256, 1);
+    else if (rg <= 512) XDNA_QG(256, 2);
+    else if (rg <= 1024) XDNA_QG(256, 4);
+    else if constexpr (DT != XDNA_F32) XDNA_QG(256, 8);
+#undef XDNA_QG
+    return launch_status("quant_rows_ragged");
+  }
   if (!vec_ok) {
     quant_rows_scalar_kernel<DT><<<dim3((unsigned)rows), 256, 0, st>>>(x, rows, k, ld_x, q, ld_q, k_pad, s);
     return launch_status("quant_rows_scalar");
@@ -503,14 +605,22 @@ __global__ __launch_bounds__(1024) void image_absmax_kernel(const void* __restri
   const char* xb = reinterpret_cast<const char*>(x) + b * per * ESZ;
   const int t = threadIdx.x;
   float m = 0.0f;
-  const bool vec_ok = ((per * ESZ) % 16 == 0) && aligned(x, 16) && per * ESZ < (int64_t(1) << 31);
-  if (vec_ok) {
+  if (per * ESZ < (int64_t(1) << 31)) {
+    // the image's whole 16-byte pieces, and the elements before and after them (images of any size follow each other,
+    // so they start anywhere)
     constexpr int U = 8;
     using V = Vec16<DT>;
-    const __amdgpu_buffer_rsrc_t r = make_rsrc(xb, (uint32_t)(per * ESZ));
+    const uint32_t head = min((uint32_t)(-reinterpret_cast<uintptr_t>(xb) & 15) / ESZ, (uint32_t)per);
+    const uint32_t nvec = (uint32_t)((per - head) * ESZ / 16);
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(xb + head * ESZ, nvec * 16);
     // 32-bit: nvec < 2^27, so every offset below stays under 2^32
-    const uint32_t nvec = (uint32_t)(per * ESZ / 16);
     const uint32_t step = gridDim.x * 1024u * U;
+    const uint32_t done = head + nvec * V::N;
+    float edge = 0.0f;
+    if (blockIdx.x == 0 && t < 16) {       // at most 7 elements on either side: lanes 0-7 those before, 8-15 those after
+      const uint32_t i = t < 8 ? (uint32_t)t : done + (uint32_t)t - 8u;
+      if (t < 8 ? i < head : i < (uint32_t)per) edge = fabsf(load_as_f32<DT>(xb, i));
+    }
     AbsMaxBits<DT> am;
     for (uint32_t base = blockIdx.x * 1024u * U + t; base < nvec; base += step) {
       V u[U];
@@ -519,7 +629,7 @@ __global__ __launch_bounds__(1024) void image_absmax_kernel(const void* __restri
 #pragma unroll
       for (int j = 0; j < U; ++j) am.add(u[j]);
     }
-    m = bits_to_abs<DT>(am.lane_bits());
+    m = mag_max(edge, bits_to_abs<DT>(am.lane_bits()));
   } else {
     for (int64_t i = (int64_t)blockIdx.x * 1024 + t; i < per; i += (int64_t)gridDim.x * 1024)
       m = mag_max(m, fabsf(load_as_f32<DT>(xb, i)));
@@ -594,9 +704,9 @@ __global__ __launch_bounds__(256) void conv_quant_nhwc_vec_kernel(const void* __
 // channel tile: lane i of the block owns PPL consecutive pixels, and per group of 16 channels it reads
 // each real channel's PPL pixels with one 16-byte load (channels past ch are not read: they quantize to
 // 0), quantizes each pixel's 16 channels and writes them as one 16-byte store. Lanes read consecutive 16
-// bytes of a channel and write consecutive pixels. Grid (cdiv(hw, 256 PPL), nb); needs hw % PPL == 0 and
-// an image below 2 GB.
-template <int DT, bool NT>
+// bytes of a channel and write consecutive pixels. Grid (cdiv(hw, 256 PPL), nb). ANY: images of any size and
+// alignment, as in conv_quant_nhwc_any_kernel; else hw % PPL == 0, aligned, an image below 2 GB.
+template <int DT, bool NT, bool ANY>
 __global__ __launch_bounds__(256) void conv_quant_nhwc_narrow_kernel(const void* __restrict__ x, int64_t ch,
                                                                      int64_t hw, const float* __restrict__ parts,
                                                                      int nparts, int8_t* __restrict__ q,
@@ -606,16 +716,23 @@ __global__ __launch_bounds__(256) void conv_quant_nhwc_narrow_kernel(const void*
   __shared__ float red[4];
   using V = Vec16<DT>;
   const int64_t b = blockIdx.y;
-  const int64_t p = ((int64_t)blockIdx.x * 256 + threadIdx.x) * PPL;     // the lane's first pixel
+  int64_t p = ((int64_t)blockIdx.x * 256 + threadIdx.x) * PPL;           // the lane's first pixel
+  if constexpr (ANY) p = min(p, max<int64_t>(0, hw - PPL));              // past the last whole PPL: those (the same bytes)
   const __amdgpu_buffer_rsrc_t r = make_rsrc(reinterpret_cast<const char*>(x) + b * ch * hw * ESZ,
                                              (uint32_t)(ch * hw * ESZ));
   const int groups = (int)(c_pad / 16);
   // the first group's loads go out before the image's scale is reduced
   V v[16];
   int nc = (int)min<int64_t>(16, ch);
+  const char* xb = reinterpret_cast<const char*>(x) + (b * ch * hw + p) * ESZ;
+  const int np = (int)max<int64_t>(0, min<int64_t>(PPL, hw - p));          // the lane's pixels
+  auto load = [&](int c, bool in) {
+    if (!in) return make_uint4(0, 0, 0, 0);                                // uniform
+    if constexpr (!ANY) return buf_load_u4<NT>(r, (uint32_t)((c * hw + p) * ESZ));
+    else return hw >= PPL ? load_u4_any<DT>(xb + c * hw * ESZ) : load_u4_first<DT>(xb + c * hw * ESZ, (int)hw);
+  };
 #pragma unroll
-  for (int i = 0; i < 16; ++i)
-    v[i].raw = i < nc ? buf_load_u4<NT>(r, (uint32_t)((i * hw + p) * ESZ)) : make_uint4(0, 0, 0, 0);
+  for (int i = 0; i < 16; ++i) v[i].raw = load(i, i < nc);
   const float sc = scale_from_amax(image_amax(parts, b, nparts, red));
   const float rc = 1.0f / sc;
   if (blockIdx.x == 0 && threadIdx.x == 0) sx[b] = sc;
@@ -624,8 +741,7 @@ __global__ __launch_bounds__(256) void conv_quant_nhwc_narrow_kernel(const void*
     if (g > 0) {
       nc = (int)max<int64_t>(0, min<int64_t>(16, ch - 16 * g));
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        v[i].raw = i < nc ? buf_load_u4<NT>(r, (uint32_t)(((16 * g + i) * hw + p) * ESZ)) : make_uint4(0, 0, 0, 0);
+      for (int i = 0; i < 16; ++i) v[i].raw = load(16 * g + i, i < nc);
     }
     uint32_t keep[4];
     valid_masks(nc, keep);
@@ -636,54 +752,75 @@ __global__ __launch_bounds__(256) void conv_quant_nhwc_narrow_kernel(const void*
       for (int i = 0; i < 16; ++i) f[i] = v[i].get(j);
       uint32_t w[4];
       quant_pack<16>(f, sc, rc, w);
-      if (p < hw)
+      if (j < np)
         *reinterpret_cast<uint4*>(qp + j * c_pad + 16 * g) =
             make_uint4(w[0] & keep[0], w[1] & keep[1], w[2] & keep[2], w[3] & keep[3]);
     }
   }
 }
 
-// Quantize + NCHW -> NHWC: tile of 64 channels x 64 pixels per block (256 threads). Wave w
-// reads channels [w*16, w*16+16) of the tile, lane = pixel, so every global read is 64
-// consecutive pixels of one channel; four channels pack into one LDS word per pixel. The
-// write-out gives each thread 16 channels of one pixel (a 16-byte store).
-template <int DT>
-__global__ __launch_bounds__(256) void conv_quant_nhwc_kernel(const void* __restrict__ x, int64_t ch, int64_t hw,
-                                                              const float* __restrict__ parts, int nparts,
-                                                              int8_t* __restrict__ q, int64_t c_pad,
-                                                              float* __restrict__ sx) {
-  __shared__ uint32_t tile[64][17];
+// The same for images of any size and alignment: a block covers 64 channels x 64 P pixels, wave w pixels 16 P w ..,
+// lane l channels 16 (l / 16) .. of P pixels (4, or 1 where that leaves blocks for less than a round), read as one
+// load at the elements' alignment; a lane past the channel's last whole P takes the P that end it (some pixels twice:
+// the same bytes). Tile rows of 80 bytes: the 16 pixels x 4 chunks of a write fall evenly on the banks. With the
+// image max: 4 x 100 x 75 x 93 bf16 10.4 us (28.6 us one pixel per lane and quotient), 3 x 256 x 37 x 37 float32
+// 7.5 (11.5), 2 x 40 x 31 x 33 bf16 8.5 (8.1).
+template <int DT, int P>
+__global__ __launch_bounds__(256) void conv_quant_nhwc_any_kernel(const void* __restrict__ x, int64_t ch, int64_t hw,
+                                                                  const float* __restrict__ parts, int nparts,
+                                                                  int8_t* __restrict__ q, int64_t c_pad,
+                                                                  float* __restrict__ sx) {
+  static_assert(P == 4 || P == 1, "pixels per lane");
+  constexpr int ESZ = (DT == XDNA_F32) ? 4 : 2;
+  constexpr int PITCH = 80;
+  __shared__ __attribute__((aligned(16))) uint8_t tile[64 * P * PITCH];
   __shared__ float red[4];
   const int64_t b = blockIdx.z;
-  const int64_t p0 = (int64_t)blockIdx.x * 64;
-  const int64_t c0 = (int64_t)blockIdx.y * 64;
+  const int64_t p0 = (int64_t)blockIdx.x * (64 * P), c0 = (int64_t)blockIdx.y * 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t cl = c0 + 16 * (lane >> 4);                // the lane's first channel
+  const int64_t pe = max<int64_t>(0, min<int64_t>(p0 + 16 * P * wave + P * (lane & 15), hw - P));   // and pixel
+  const char* xb = reinterpret_cast<const char*>(x) + (b * ch * hw + pe) * ESZ;
+  const int nl = (int)min<int64_t>(16, ch - c0);           // uniform: below 16 only where the block has no more channels
+  Vec16<DT> v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    v[i].raw = make_uint4(0, 0, 0, 0);
+    if (i < nl) {
+      const char* px = xb + min(cl + i, ch - 1) * hw * ESZ;   // channels past ch: cleared below
+      if (P == 1 || hw < P) v[i].raw = load_u4_first<DT>(px, (int)min<int64_t>(P, hw));
+      else if constexpr (DT == XDNA_F32) v[i].raw = load_u4_any<DT>(px);
+      else {
+        const u32x2_e2 h = *reinterpret_cast<const u32x2_e2*>(px);
+        v[i].raw = make_uint4(h[0], h[1], 0, 0);
+      }
+    }
+  }
   const float sc = scale_from_amax(image_amax(parts, b, nparts, red));
   const float rc = 1.0f / sc;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) sx[b] = sc;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int64_t p = p0 + lane;
+  uint32_t keep[4];
+  valid_masks((int)max<int64_t>(0, min<int64_t>(16, ch - cl)), keep);
+  const int row0 = (int)max<int64_t>(-P, pe - p0);         // below 0: pixels of the tile before
 #pragma unroll
-  for (int c4 = 0; c4 < 4; ++c4) {
-    uint32_t packed = 0;
+  for (int j = 0; j < P; ++j) {
+    float f[16];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int64_t c = c0 + wave * 16 + c4 * 4 + e;
-      int qv = 0;
-      if (c < ch && p < hw) qv = quant1(load_as_f32<DT>(x, (b * ch + c) * hw + p), sc, rc);
-      packed |= ((uint32_t)(uint8_t)(int8_t)qv) << (8 * e);
-    }
-    tile[lane][wave * 4 + c4] = packed;
+    for (int i = 0; i < 16; ++i) f[i] = v[i].get(j);
+    uint32_t w[4];
+    quant_pack<16>(f, sc, rc, w);
+    if (row0 + j >= 0)
+      *reinterpret_cast<uint4*>(&tile[(row0 + j) * PITCH + 16 * (lane >> 4)]) =
+          make_uint4(w[0] & keep[0], w[1] & keep[1], w[2] & keep[2], w[3] & keep[3]);
   }
   __syncthreads();
-  const int pix = threadIdx.x >> 2;
-  const int part = threadIdx.x & 3;
-  const int64_t po = p0 + pix;
-  const int64_t co = c0 + part * 16;
-  if (po < hw && co < c_pad) {
-    uint4 v = make_uint4(tile[pix][part * 4 + 0], tile[pix][part * 4 + 1], tile[pix][part * 4 + 2],
-                         tile[pix][part * 4 + 3]);
-    *reinterpret_cast<uint4*>(q + (b * hw + po) * c_pad + co) = v;
+#pragma unroll
+  for (int j = 0; j < P; ++j) {
+    const int k = threadIdx.x + 256 * j;                   // 16-byte chunk of the tile
+    const int64_t p = p0 + (k >> 2), c = c0 + (k & 3) * 16;
+    if (p < hw && c < c_pad)
+      *reinterpret_cast<uint4*>(q + (b * hw + p) * c_pad + c) =
+          *reinterpret_cast<const uint4*>(&tile[(k >> 2) * PITCH + (k & 3) * 16]);
   }
 }
 
@@ -1291,23 +1428,29 @@ int xdna_conv_quant_nhwc(const void* x, int x_dtype, int64_t nb, int64_t ch, int
   const int parts = (int)std::max<int64_t>(
       1, std::min<int64_t>({cdiv(per * esz, 1024 * 8 * 16), (int64_t)AMAX_PARTS, std::max<int64_t>(1, resident / nb)}));
   dim3 g1((unsigned)parts, (unsigned)nb, 1);
-  dim3 g2((unsigned)cdiv(hw, 64), (unsigned)cdiv(c_pad, 64), (unsigned)nb);
   XDNA_REQUIRE(cdiv(hw, 64) < (1ll << 31) && cdiv(c_pad, 64) < 65536, "image too large");
   // the 16-byte path: pixel rows in whole 16-byte loads, an image's bytes addressable by one buffer resource
   const bool vec = hw % (16 / esz) == 0 && aligned(x, 16) && per * esz < (int64_t(1) << 31);
   const dim3 gv((unsigned)cdiv(hw, 16 * (16 / esz)), (unsigned)cdiv(c_pad, 256), (unsigned)nb);
   // narrow images: the pixel-major kernel reads only the real channels (a 256-channel tile spends most of its
   // loads past ch: 8x3x448x448 float32 took 114 us, 20 us this way); at c_pad 64 the tile is faster again
-  const bool narrow = vec && c_pad <= 48;
+  // (off the 16-byte path: while its 256 PPL pixels a block still make a quarter of a round; 2 x 40 x 31 x 33 bf16, two
+  // blocks, took 19 us, 8.5 us in tiles)
+  const bool narrow = c_pad <= 48 && (vec || 4 * cdiv(hw, 256 * (16 / esz)) * nb >= device_cus());
   const dim3 gn((unsigned)cdiv(hw, 256 * (16 / esz)), (unsigned)nb, 1);
+  const dim3 ga((unsigned)cdiv(hw, 256), (unsigned)cdiv(c_pad, 64), (unsigned)nb);
+  const dim3 g1p((unsigned)cdiv(hw, 64), (unsigned)cdiv(c_pad, 64), (unsigned)nb);
+  const bool four = 2 * cdiv(hw, 256) * cdiv(c_pad, 64) * nb >= device_cus();
 #define XDNA_CQ(DT)                                                                                        \
   if (nt) image_absmax_kernel<DT, true><<<g1, 1024, 0, st>>>(x, per, amax_ws);                              \
   else image_absmax_kernel<DT, false><<<g1, 1024, 0, st>>>(x, per, amax_ws);                                \
-  if (narrow && nt) conv_quant_nhwc_narrow_kernel<DT, true><<<gn, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx); \
-  else if (narrow) conv_quant_nhwc_narrow_kernel<DT, false><<<gn, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx); \
-  else if (vec && nt) conv_quant_nhwc_vec_kernel<DT, true><<<gv, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx); \
-  else if (vec) conv_quant_nhwc_vec_kernel<DT, false><<<gv, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx); \
-  else conv_quant_nhwc_kernel<DT><<<g2, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx);
+  if (narrow && !vec) conv_quant_nhwc_narrow_kernel<DT, false, true><<<gn, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx); \
+  else if (narrow && nt) conv_quant_nhwc_narrow_kernel<DT, true, false><<<gn, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx); \
+  else if (narrow) conv_quant_nhwc_narrow_kernel<DT, false, false><<<gn, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx); \
+  else if (!vec && four) conv_quant_nhwc_any_kernel<DT, 4><<<ga, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx); \
+  else if (!vec) conv_quant_nhwc_any_kernel<DT, 1><<<g1p, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx); \
+  else if (nt) conv_quant_nhwc_vec_kernel<DT, true><<<gv, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx); \
+  else conv_quant_nhwc_vec_kernel<DT, false><<<gv, 256, 0, st>>>(x, ch, hw, amax_ws, parts, q, c_pad, sx);
   switch (x_dtype) {
     case XDNA_F32: XDNA_CQ(XDNA_F32) break;
     case XDNA_BF16: XDNA_CQ(XDNA_BF16) break;
