@@ -170,6 +170,26 @@ int xdna_gemm_i8_dequant_ws(const int8_t* a, int64_t lda, const float* sx, const
                             const float* sw, const float* bias, void* y, int y_dtype, int64_t ldy,
                             int64_t m, int64_t n, int64_t k, void* ws, int64_t ws_bytes, void* stream);
 
+/* The entry points whose bias is float32, with the bias in bias_dtype (XDNA_F32 / BF16 / F16; widened exactly, so the
+ * results are those of the float32 copy) as the model holds it: no cast launch before each call. bias may be NULL.
+ * They replace the `bias.float()` of torch_xdna/runtime.py:352 and torch_xdna/conv.py:50 together with the calls they
+ * are named after. */
+int xdna_gemm_i8_dequant_bias(const int8_t* a, int64_t lda, const float* sx, const int8_t* w, int64_t ldw,
+                              const float* sw, const void* bias, int bias_dtype, void* y, int y_dtype, int64_t ldy,
+                              int64_t m, int64_t n, int64_t k, void* ws, int64_t ws_bytes, void* stream);
+int xdna_linear_row_bias(const void* x, int x_dtype, int64_t kx, const int8_t* w, int64_t ldw, const float* sw,
+                         const void* bias, int bias_dtype, void* y, int y_dtype, int64_t n, int64_t k, float* sx,
+                         void* stream);
+int xdna_gemm_bf16_bias(const void* a, int64_t lda, const void* w, int64_t ldw, const void* bias, int bias_dtype,
+                        void* y, int y_dtype, int64_t ldy, int64_t m, int64_t n, int64_t k, void* stream);
+int xdna_conv3x3_dequant_bias(const int8_t* x, int64_t nb, int64_t h, int64_t w, int64_t c_pad, const int8_t* wq,
+                              int64_t co, int shift, int relu, const float* scale, const float* sx, const void* bias,
+                              int bias_dtype, void* y, int y_dtype, void* stream);
+int xdna_conv_requant_next_bias(const void* q, int relu, int relu_y, int pool, int64_t nb, int64_t h, int64_t w,
+                                int64_t co, const float* scale, const float* sx, const void* bias, int bias_dtype,
+                                int x_dtype, int8_t* xq_next, int64_t c_pad_next, float* sx_next, float* amax_ws,
+                                void* stream);
+
 /* The W8A8 linear of ONE activation row (decode, M = 1) in one launch: the row's per-row quantize
  * (xdna_quant_rows' arithmetic, replacing torch_xdna/runtime.py:287 `_quant_rows` in `_gemm` and
  * :145-148) and the GEMM with the dequantize of xdna_gemm_i8_dequant (runtime.py:288-296 and :350-353,

@@ -797,6 +797,43 @@ def test_rule_tiles(gpu, m, n, k, tile_table):
     assert float((y.double() - ref).norm() / ref.norm()) < 1e-5
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_bias_dtypes(gpu, dtype, tile_table):
+    """16-bit biases, used as they are, against their float32 copies, bit for bit: every kernel family that adds one
+    (the tile engine with full and ragged tiles and with K groups, the small-M, one-row, few-row and row-quantizing
+    kernels, the fused conv, the chaining passes in their wide and general form), NaN and infinity among the values."""
+    k = tile_table
+    for m, n, kk in [(1, 300, 1024), (5, 300, 2048), (12, 300, 512), (70, 1000, 1040), (300, 520, 1024), (700, 1001, 208)]:
+        x = _rand((m, kk), DT[dtype], seed=m).to(gpu)
+        w = _rand((n, kk), torch.float32, seed=n, scale=0.02).to(gpu)
+        b = _rand((n,), DT[dtype], seed=m + n)
+        b[0], b[-1] = float("inf"), float("nan")
+        b = b.to(gpu)
+        xq, sx = k.quant_rows(x)
+        wq, sw = k.quant_rows(w)
+        for out in (torch.float32, DT[dtype]):
+            got, want = (k.mm_i8_dequant(xq, sx, wq, sw, t, out) for t in (b, b.float()))
+            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num()), (m, n, kk)
+            got, want = (k.mm_bf16(k.bf16_rows(x, kk), k.bf16_rows(w, kk), t, out) for t in (b, b.float()))
+            assert torch.equal(got.nan_to_num(), want.nan_to_num()), (m, n, kk)
+            if m == 1:
+                got, want = (k.linear_row(x, wq, sw, t, out) for t in (b, b.float()))
+                assert torch.equal(got.nan_to_num(), want.nan_to_num())
+    for n, ci, co, h, w_ in [(2, 3, 48, 13, 37), (1, 64, 128, 16, 64), (2, 16, 20, 5, 7)]:
+        x, wt = _conv_case(n, ci, co, h, w_, seed=co)
+        c_pad = -(-ci // 16) * 16
+        xq, sx = k.conv_quant(x.to(gpu), c_pad)
+        wq, sw = k.conv_weight_pack(wt.to(gpu), c_pad)
+        b = _rand((co,), DT[dtype], seed=co).to(gpu)
+        got, want = (k.conv3x3_dequant(xq, wq, 9, False, sw, sx, t, DT[dtype]) for t in (b, b.float()))
+        assert torch.equal(got, want), (n, ci, co)
+        q = k.conv3x3(xq, wq, 9, False)
+        for pool in (False, True):
+            got, want = (k.conv_requant_next(q, False, pool, sw, sx, t, DT[dtype], -(-co // 16) * 16, relu_y=pool)
+                         for t in (b, b.float()))
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), (n, ci, co, pool)
+
+
 def _ksplit(cus, bm, bn, kg, tiles, k):
     """Workgroups per tile along K that the library gives a launch: 1 above 64 x 64 or when the tiles fill
     more than half of the CUs, else up to CUs / tiles, at most 16, with at least 16 slices of 64 per K

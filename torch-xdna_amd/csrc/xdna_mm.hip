@@ -64,7 +64,8 @@ struct EpiArgs {
   int64_t ldo;          // elements between output rows
   const float* sx;      // [M]; with dq_out per image [nb]
   const float* sw;      // [N]
-  const float* bias;    // [N] or null
+  const void* bias;     // [N] or null, in bias_dt
+  int bias_dt;          // XDNA_F32 / BF16 / F16: the bias as the model holds it (a cast of its own would be a launch)
   int shift;            // EPI_REQUANT
   int relu;             // EPI_REQUANT / EPI_CALIB
   int32_t* acc_max;     // EPI_CALIB
@@ -112,6 +113,18 @@ __device__ __forceinline__ f32x4 mfma16x16x32bf(const i32x4& a, const i32x4& b, 
 }
 
 // ------------------------------------------------------------------------------ epilogue
+// Bias element n as loaded (a 16-bit value's bits in the low half), and as float32 (exact widening). Kernels that
+// load it ahead of their K loop convert it after the loop, so that nothing waits for it before.
+__device__ __forceinline__ float bias_raw(const EpiArgs& e, int64_t n) {
+  if (e.bias_dt == XDNA_F32) return reinterpret_cast<const float*>(e.bias)[n];
+  return __uint_as_float((uint32_t) reinterpret_cast<const uint16_t*>(e.bias)[n]);
+}
+__device__ __forceinline__ float bias_f32(const EpiArgs& e, float raw) {
+  if (e.bias_dt == XDNA_F32) return raw;
+  const uint16_t h = (uint16_t)__float_as_uint(raw);
+  return e.bias_dt == XDNA_BF16 ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
+}
+
 // Per-column values of CW consecutive output columns n .. n+CW-1 (weight scales and bias of the
 // dequantize), loaded once per column block and reused for every row.
 template <int EPI, int CW = 4>
@@ -123,7 +136,24 @@ struct EpiCols {
     if constexpr (epi_dq(EPI) || epi_bf(EPI)) {
 #pragma unroll
       for (int r = 0; r < CW; ++r) b[r] = 0.0f;
-      if (e.bias) load(e.bias, n, N, b);
+      if (e.bias) {
+        if (e.bias_dt == XDNA_F32) {
+          load(reinterpret_cast<const float*>(e.bias), n, N, b);
+        } else {
+          const uint16_t* p = reinterpret_cast<const uint16_t*>(e.bias);
+#pragma unroll
+          for (int r = 0; r < CW; ++r) b[r] = __uint_as_float((uint32_t)p[min(n + r, N - 1)]);
+        }
+      }
+    }
+  }
+  // after the K loop, once: the bias as float32
+  __device__ __forceinline__ void finish(const EpiArgs& e) {
+    if constexpr (epi_dq(EPI) || epi_bf(EPI)) {
+      if (e.bias && e.bias_dt != XDNA_F32) {
+#pragma unroll
+        for (int r = 0; r < CW; ++r) b[r] = bias_f32(e, b[r]);
+      }
     }
   }
   // One straight-line path: no per-lane branch merges the loaded values, so nothing waits for them
@@ -1049,6 +1079,8 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
       if (lane == 0) __hip_atomic_store(e.cnt + slot, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
     }
   }
+#pragma unroll
+  for (int jp = 0; jp < FN / CB; ++jp) cols_pre[jp].finish(e);
   int8_t* stg = lds + wave * 32 * PITCH;     // group 0: lds == lds_all
   int calib = 0;
   // uniform: the whole tile is inside M x N and the output rows take CW-wide vector stores
@@ -1088,7 +1120,7 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
       if (rqdq) {
         const int64_t nl = min<int64_t>(n0 + wn * TN + jp * COLS + (lane % COLS), N - 1);
         rq_fo = e.sw[nl];
-        rq_bo = e.bias ? e.bias[nl] : 0.0f;
+        rq_bo = e.bias ? bias_f32(e, bias_raw(e, nl)) : 0.0f;
       }
     }
     (void)rq_fo;
@@ -1228,6 +1260,7 @@ __global__ __launch_bounds__(WAVES * 64) void mm_small_kernel(const int8_t* __re
   for (int v = 1; v < WAVES; ++v) acc += red[v][lane];
   int calib = 0;
   if constexpr (!PRE) load_epi();
+  cols.finish(e);
   epilogue4<EPI>(e, mrow, n0 + 4 * (lane >> 4), M, N, __builtin_bit_cast(i32x4, acc), calib, cols, sxm);
   calib_flush<EPI>(e, calib);
 }
@@ -1254,7 +1287,7 @@ struct Epi1Ops {
       sw = e.sw[n];
     }
     if constexpr (epi_dq(EPI) || epi_bf(EPI)) {
-      if (e.bias) b = e.bias[n];
+      if (e.bias) b = bias_raw(e, n);
     }
   }
 };
@@ -1277,7 +1310,7 @@ __device__ __forceinline__ void epilogue1(const EpiArgs& e, int64_t m, int64_t n
       t = t * o.sx;
       t = t * o.sw;
     }
-    if (e.bias) t = t + o.b;
+    if (e.bias) t = t + bias_f32(e, o.b);
     if constexpr (EPI == EPI_DQ_F32 || EPI == EPI_BF_F32) reinterpret_cast<float*>(e.out)[off] = t;
     else if constexpr (EPI == EPI_DQ_BF16 || EPI == EPI_BF_BF16) reinterpret_cast<uint16_t*>(e.out)[off] = f32_to_bf16_bits(t);
     else reinterpret_cast<uint16_t*>(e.out)[off] = f32_to_f16_bits(t);
@@ -1540,7 +1573,7 @@ __global__ __launch_bounds__(512) void mm_rowq_kernel(const void* __restrict__ x
   auto column_ops = [&](int64_t n) {
     const int64_t nc = min(n, N - 1);
     ops.sw = e.sw[nc];
-    ops.b = e.bias ? e.bias[nc] : 0.0f;
+    ops.b = e.bias ? bias_raw(e, nc) : 0.0f;
   };
   column_ops(ncol0);
   int cc = 0, rr = 0;                     // the item being consumed
@@ -1733,7 +1766,7 @@ inline EpiArgs shift_epi(const EpiArgs& e, int out_bytes, int64_t m0, int64_t n0
   if (r.out) r.out = reinterpret_cast<char*>(r.out) + (m0 * e.ldo + n0) * out_bytes;
   if (r.sx) r.sx += m0;
   if (r.sw) r.sw += n0;
-  if (r.bias) r.bias += n0;
+  if (r.bias) r.bias = static_cast<const char*>(r.bias) + n0 * (r.bias_dt == XDNA_F32 ? 4 : 2);
   return r;
 }
 
@@ -2420,6 +2453,8 @@ int launch_conv(const int8_t* x, int64_t nb, int64_t h, int64_t w, int64_t c_pad
 
 __global__ void zero_i32_kernel(int32_t* p) { *p = 0; }
 
+inline bool float_dtype(int dt) { return dt == XDNA_F32 || dt == XDNA_BF16 || dt == XDNA_F16; }
+
 }  // namespace xdna
 
 using namespace xdna;
@@ -2449,9 +2484,10 @@ int xdna_gemm_i8_i32(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw,
   return xdna_gemm_i8_i32_ws(a, lda, w, ldw, c, ldc, m, n, k, nullptr, 0, stream);
 }
 
-int xdna_gemm_i8_dequant_ws(const int8_t* a, int64_t lda, const float* sx, const int8_t* w, int64_t ldw,
-                            const float* sw, const float* bias, void* y, int y_dtype, int64_t ldy, int64_t m,
-                            int64_t n, int64_t k, void* ws, int64_t ws_bytes, void* stream) {
+int xdna_gemm_i8_dequant_bias(const int8_t* a, int64_t lda, const float* sx, const int8_t* w, int64_t ldw,
+                              const float* sw, const void* bias, int bias_dtype, void* y, int y_dtype, int64_t ldy,
+                              int64_t m, int64_t n, int64_t k, void* ws, int64_t ws_bytes, void* stream) {
+  XDNA_REQUIRE(float_dtype(bias_dtype), "bias_dtype must be F32/BF16/F16");
   XDNA_REQUIRE(y_dtype == XDNA_F32 || y_dtype == XDNA_BF16 || y_dtype == XDNA_F16, "y_dtype must be F32/BF16/F16");
   XDNA_REQUIRE(m >= 0 && n >= 0 && k >= 0, "negative size");
   if (m == 0 || n == 0) return XDNA_OK;
@@ -2465,6 +2501,7 @@ int xdna_gemm_i8_dequant_ws(const int8_t* a, int64_t lda, const float* sx, const
   e.sx = sx;
   e.sw = sw;
   e.bias = bias;
+  e.bias_dt = bias_dtype;
   e.vec_ok = (ldy % 8 == 0) && aligned(y, 16);
   e.ws = ws;
   e.ws_bytes = ws ? ws_bytes : 0;
@@ -2475,14 +2512,23 @@ int xdna_gemm_i8_dequant_ws(const int8_t* a, int64_t lda, const float* sx, const
   return launch_gemm<EPI_DQ_F16>(a, lda, w, ldw, m, n, k, e, tile, st);
 }
 
+int xdna_gemm_i8_dequant_ws(const int8_t* a, int64_t lda, const float* sx, const int8_t* w, int64_t ldw,
+                            const float* sw, const float* bias, void* y, int y_dtype, int64_t ldy, int64_t m,
+                            int64_t n, int64_t k, void* ws, int64_t ws_bytes, void* stream) {
+  return xdna_gemm_i8_dequant_bias(a, lda, sx, w, ldw, sw, bias, XDNA_F32, y, y_dtype, ldy, m, n, k, ws, ws_bytes,
+                                   stream);
+}
+
 int xdna_gemm_i8_dequant(const int8_t* a, int64_t lda, const float* sx, const int8_t* w, int64_t ldw, const float* sw,
                          const float* bias, void* y, int y_dtype, int64_t ldy, int64_t m, int64_t n, int64_t k,
                          void* stream) {
   return xdna_gemm_i8_dequant_ws(a, lda, sx, w, ldw, sw, bias, y, y_dtype, ldy, m, n, k, nullptr, 0, stream);
 }
 
-int xdna_linear_row(const void* x, int x_dtype, int64_t kx, const int8_t* w, int64_t ldw, const float* sw,
-                    const float* bias, void* y, int y_dtype, int64_t n, int64_t k, float* sx, void* stream) {
+int xdna_linear_row_bias(const void* x, int x_dtype, int64_t kx, const int8_t* w, int64_t ldw, const float* sw,
+                         const void* bias, int bias_dtype, void* y, int y_dtype, int64_t n, int64_t k, float* sx,
+                         void* stream) {
+  XDNA_REQUIRE(float_dtype(bias_dtype), "bias_dtype must be F32/BF16/F16");
   XDNA_REQUIRE(x_dtype == XDNA_F32 || x_dtype == XDNA_BF16 || x_dtype == XDNA_F16, "x_dtype must be F32/BF16/F16");
   XDNA_REQUIRE(y_dtype == XDNA_F32 || y_dtype == XDNA_BF16 || y_dtype == XDNA_F16, "y_dtype must be F32/BF16/F16");
   XDNA_REQUIRE(n >= 0 && k >= 0 && kx >= 0, "negative size");
@@ -2498,14 +2544,21 @@ int xdna_linear_row(const void* x, int x_dtype, int64_t kx, const int8_t* w, int
   e.ldo = n;
   e.sw = sw;
   e.bias = bias;
+  e.bias_dt = bias_dtype;
   hipStream_t st = as_stream(stream);
   if (y_dtype == XDNA_F32) return launch_rowq_dt<EPI_DQ_F32>(x, x_dtype, kx, w, ldw, n, k, sx, e, st);
   if (y_dtype == XDNA_BF16) return launch_rowq_dt<EPI_DQ_BF16>(x, x_dtype, kx, w, ldw, n, k, sx, e, st);
   return launch_rowq_dt<EPI_DQ_F16>(x, x_dtype, kx, w, ldw, n, k, sx, e, st);
 }
 
-int xdna_gemm_bf16(const void* a, int64_t lda, const void* w, int64_t ldw, const float* bias, void* y, int y_dtype,
-                   int64_t ldy, int64_t m, int64_t n, int64_t k, void* stream) {
+int xdna_linear_row(const void* x, int x_dtype, int64_t kx, const int8_t* w, int64_t ldw, const float* sw,
+                    const float* bias, void* y, int y_dtype, int64_t n, int64_t k, float* sx, void* stream) {
+  return xdna_linear_row_bias(x, x_dtype, kx, w, ldw, sw, bias, XDNA_F32, y, y_dtype, n, k, sx, stream);
+}
+
+int xdna_gemm_bf16_bias(const void* a, int64_t lda, const void* w, int64_t ldw, const void* bias, int bias_dtype,
+                        void* y, int y_dtype, int64_t ldy, int64_t m, int64_t n, int64_t k, void* stream) {
+  XDNA_REQUIRE(float_dtype(bias_dtype), "bias_dtype must be F32/BF16/F16");
   XDNA_REQUIRE(y_dtype == XDNA_F32 || y_dtype == XDNA_BF16 || y_dtype == XDNA_F16, "y_dtype must be F32/BF16/F16");
   XDNA_REQUIRE(m >= 0 && n >= 0 && k >= 0, "negative size");
   if (m == 0 || n == 0) return XDNA_OK;
@@ -2516,6 +2569,7 @@ int xdna_gemm_bf16(const void* a, int64_t lda, const void* w, int64_t ldw, const
   e.out = y;
   e.ldo = ldy;
   e.bias = bias;
+  e.bias_dt = bias_dtype;
   e.vec_ok = (ldy % 8 == 0) && aligned(y, 16);
   // the engine stages bytes: a bf16 row of k values is 2 * k bytes
   const int8_t* ab = static_cast<const int8_t*>(a);
@@ -2525,6 +2579,11 @@ int xdna_gemm_bf16(const void* a, int64_t lda, const void* w, int64_t ldw, const
   if (y_dtype == XDNA_F32) return launch_gemm<EPI_BF_F32>(ab, 2 * lda, wb, 2 * ldw, m, n, 2 * k, e, tile, st);
   if (y_dtype == XDNA_BF16) return launch_gemm<EPI_BF_BF16>(ab, 2 * lda, wb, 2 * ldw, m, n, 2 * k, e, tile, st);
   return launch_gemm<EPI_BF_F16>(ab, 2 * lda, wb, 2 * ldw, m, n, 2 * k, e, tile, st);
+}
+
+int xdna_gemm_bf16(const void* a, int64_t lda, const void* w, int64_t ldw, const float* bias, void* y, int y_dtype,
+                   int64_t ldy, int64_t m, int64_t n, int64_t k, void* stream) {
+  return xdna_gemm_bf16_bias(a, lda, w, ldw, bias, XDNA_F32, y, y_dtype, ldy, m, n, k, stream);
 }
 
 int xdna_gemm_bf16_silu(const void* a, int64_t lda, const void* w, int64_t ldw, void* y, int64_t ldy, int64_t m,
@@ -2570,9 +2629,10 @@ int xdna_conv3x3_i8(const int8_t* x, int64_t nb, int64_t h, int64_t w, int64_t c
   return launch_conv<EPI_REQUANT>(x, nb, h, w, c_pad, wq, co, e, st);
 }
 
-int xdna_conv3x3_dequant(const int8_t* x, int64_t nb, int64_t h, int64_t w, int64_t c_pad, const int8_t* wq,
-                         int64_t co, int shift, int relu, const float* scale, const float* sx, const float* bias,
-                         void* y, int y_dtype, void* stream) {
+int xdna_conv3x3_dequant_bias(const int8_t* x, int64_t nb, int64_t h, int64_t w, int64_t c_pad, const int8_t* wq,
+                              int64_t co, int shift, int relu, const float* scale, const float* sx, const void* bias,
+                              int bias_dtype, void* y, int y_dtype, void* stream) {
+  XDNA_REQUIRE(float_dtype(bias_dtype), "bias_dtype must be F32/BF16/F16");
   XDNA_REQUIRE(nb >= 0 && h >= 1 && w >= 1 && co >= 1, "bad sizes");
   XDNA_REQUIRE(c_pad >= 16 && c_pad % 16 == 0, "c_pad must be a positive multiple of 16");
   XDNA_REQUIRE(y_dtype == XDNA_F32 || y_dtype == XDNA_BF16 || y_dtype == XDNA_F16,
@@ -2590,9 +2650,17 @@ int xdna_conv3x3_dequant(const int8_t* x, int64_t nb, int64_t h, int64_t w, int6
   e.sw = scale;
   e.sx = sx;
   e.bias = bias;
+  e.bias_dt = bias_dtype;
   e.dq_out = y_dtype + 1;
   e.px0 = 0;
   return launch_conv<EPI_REQUANT>(x, nb, h, w, c_pad, wq, co, e, as_stream(stream));
+}
+
+int xdna_conv3x3_dequant(const int8_t* x, int64_t nb, int64_t h, int64_t w, int64_t c_pad, const int8_t* wq,
+                         int64_t co, int shift, int relu, const float* scale, const float* sx, const float* bias,
+                         void* y, int y_dtype, void* stream) {
+  return xdna_conv3x3_dequant_bias(x, nb, h, w, c_pad, wq, co, shift, relu, scale, sx, bias, XDNA_F32, y, y_dtype,
+                                   stream);
 }
 
 int xdna_tile_set(int kind, int64_t m, int64_t n, int64_t k, int tile) {

@@ -983,9 +983,38 @@ struct ChainArgs {
   const uint8_t* q;
   uint32_t h, w, co, ho, wo, ng;
   const float* scale;
-  const float* bias;
+  const void* bias;    // in bias_dt (XDNA_F32 / BF16 / F16), or null
+  int bias_dt;
   int relu_y, vec_f;
 };
+
+// The bias of channels c0 .. c0+15 as float32 (0 past co or without one).
+__device__ __forceinline__ void chain_bias(const ChainArgs& a, uint32_t c0, float (&bv)[16]) {
+#pragma unroll
+  for (int e = 0; e < 16; ++e) bv[e] = 0.0f;
+  if (!a.bias) return;                     // uniform, as is the dtype
+  if (a.bias_dt == XDNA_F32) {
+    const float* p = reinterpret_cast<const float*>(a.bias);
+    if (a.vec_f && c0 + 16 <= a.co) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float4 b4 = reinterpret_cast<const float4*>(p + c0)[k];
+        bv[4 * k] = b4.x; bv[4 * k + 1] = b4.y; bv[4 * k + 2] = b4.z; bv[4 * k + 3] = b4.w;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) bv[e] = c0 + e < a.co ? p[c0 + e] : 0.0f;
+    }
+  } else {
+    const uint16_t* p = reinterpret_cast<const uint16_t*>(a.bias);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const uint16_t h = p[min(c0 + e, a.co - 1)];
+      const float v = a.bias_dt == XDNA_BF16 ? bf16_bits_to_f32(h) : f16_bits_to_f32(h);
+      bv[e] = c0 + e < a.co ? v : 0.0f;
+    }
+  }
+}
 
 // The (pooled) integers of channels c0 .. c0+15 of output pixel pix of image b (int domain: uint8
 // with ReLU, else int8); channels >= co read as the domain's minimum.
@@ -1022,14 +1051,12 @@ __device__ __forceinline__ void chain_q(const ChainArgs& a, int64_t b, uint32_t 
 // scale * sx and bias of channels c0 .. c0+15 (0 past co).
 __device__ __forceinline__ void chain_factors(const ChainArgs& a, uint32_t c0, float sxb, float (&f)[16],
                                               float (&bv)[16]) {
+  chain_bias(a, c0, bv);
   if (a.vec_f && c0 + 16 <= a.co) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const float4 s4 = reinterpret_cast<const float4*>(a.scale + c0)[k];
       f[4 * k] = s4.x * sxb; f[4 * k + 1] = s4.y * sxb; f[4 * k + 2] = s4.z * sxb; f[4 * k + 3] = s4.w * sxb;
-      float4 b4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (a.bias) b4 = reinterpret_cast<const float4*>(a.bias + c0)[k];
-      bv[4 * k] = b4.x; bv[4 * k + 1] = b4.y; bv[4 * k + 2] = b4.z; bv[4 * k + 3] = b4.w;
     }
   } else {
 #pragma unroll
@@ -1037,7 +1064,6 @@ __device__ __forceinline__ void chain_factors(const ChainArgs& a, uint32_t c0, f
       const uint32_t o = min(c0 + e, a.co - 1);
       const bool in = c0 + e < a.co;
       f[e] = in ? a.scale[o] * sxb : 0.0f;
-      bv[e] = (in && a.bias) ? a.bias[o] : 0.0f;
     }
   }
 }
@@ -1045,14 +1071,12 @@ __device__ __forceinline__ void chain_factors(const ChainArgs& a, uint32_t c0, f
 // The raw scale and bias of channels c0 .. c0+15 (0 past co), loaded without the image's factor so the
 // loads can go out before anything they would wait for; chain_scale then forms chain_factors' values.
 __device__ __forceinline__ void chain_factors_raw(const ChainArgs& a, uint32_t c0, float (&sr)[16], float (&bv)[16]) {
+  chain_bias(a, c0, bv);
   if (a.vec_f && c0 + 16 <= a.co) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const float4 s4 = reinterpret_cast<const float4*>(a.scale + c0)[k];
       sr[4 * k] = s4.x; sr[4 * k + 1] = s4.y; sr[4 * k + 2] = s4.z; sr[4 * k + 3] = s4.w;
-      float4 b4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (a.bias) b4 = reinterpret_cast<const float4*>(a.bias + c0)[k];
-      bv[4 * k] = b4.x; bv[4 * k + 1] = b4.y; bv[4 * k + 2] = b4.z; bv[4 * k + 3] = b4.w;
     }
   } else {
 #pragma unroll
@@ -1060,7 +1084,6 @@ __device__ __forceinline__ void chain_factors_raw(const ChainArgs& a, uint32_t c
       const uint32_t o = min(c0 + e, a.co - 1);
       const bool in = c0 + e < a.co;
       sr[e] = in ? a.scale[o] : 0.0f;
-      bv[e] = (in && a.bias) ? a.bias[o] : 0.0f;
     }
   }
 }
@@ -1515,9 +1538,11 @@ int xdna_conv_dequant(const void* q, int relu, int64_t nb, int64_t h, int64_t w,
   return launch_status("conv_dequant");
 }
 
-int xdna_conv_requant_next(const void* q, int relu, int relu_y, int pool, int64_t nb, int64_t h, int64_t w, int64_t co,
-                           const float* scale, const float* sx, const float* bias, int x_dtype, int8_t* xq_next,
-                           int64_t c_pad_next, float* sx_next, float* amax_ws, void* stream) {
+int xdna_conv_requant_next_bias(const void* q, int relu, int relu_y, int pool, int64_t nb, int64_t h, int64_t w,
+                                int64_t co, const float* scale, const float* sx, const void* bias, int bias_dtype,
+                                int x_dtype, int8_t* xq_next, int64_t c_pad_next, float* sx_next, float* amax_ws,
+                                void* stream) {
+  XDNA_REQUIRE(float_dtype(bias_dtype), "bias_dtype must be XDNA_F32, XDNA_BF16 or XDNA_F16");
   XDNA_REQUIRE(float_dtype(x_dtype), "x_dtype must be XDNA_F32, XDNA_BF16 or XDNA_F16");
   XDNA_REQUIRE(nb >= 0 && h >= 1 && w >= 1 && co >= 1 && nb < 65536, "bad sizes");
   XDNA_REQUIRE(c_pad_next >= co && c_pad_next % 16 == 0, "c_pad_next must be a multiple of 16 and >= co");
@@ -1538,7 +1563,7 @@ int xdna_conv_requant_next(const void* q, int relu, int relu_y, int pool, int64_
   const int parts = (int)std::max<int64_t>(1, std::min<int64_t>(cdiv(items, per_block), AMAX_PARTS));
   dim3 g0((unsigned)parts, (unsigned)nb), g1((unsigned)cdiv(items, per_block), (unsigned)nb);
   ChainArgs ca{static_cast<const uint8_t*>(q), (uint32_t)h, (uint32_t)w, (uint32_t)co, (uint32_t)ho, (uint32_t)wo,
-               (uint32_t)ng, scale, bias, relu_y ? 1 : 0,
+               (uint32_t)ng, scale, bias, bias_dtype, relu_y ? 1 : 0,
                (aligned(scale, 16) && (!bias || aligned(bias, 16))) ? 1 : 0};
 #define XDNA_CH(DT, R, P)                                                                                 \
   if (wide && u == 4) {                                                                                   \
@@ -1564,6 +1589,13 @@ int xdna_conv_requant_next(const void* q, int relu, int relu_y, int pool, int64_
 #undef XDNA_CH_RP
 #undef XDNA_CH
   return launch_status("conv_requant_next");
+}
+
+int xdna_conv_requant_next(const void* q, int relu, int relu_y, int pool, int64_t nb, int64_t h, int64_t w, int64_t co,
+                           const float* scale, const float* sx, const float* bias, int x_dtype, int8_t* xq_next,
+                           int64_t c_pad_next, float* sx_next, float* amax_ws, void* stream) {
+  return xdna_conv_requant_next_bias(q, relu, relu_y, pool, nb, h, w, co, scale, sx, bias, XDNA_F32, x_dtype, xq_next,
+                                     c_pad_next, sx_next, amax_ws, stream);
 }
 
 int xdna_nchw_to_nhwc_i8(const int8_t* src, int64_t nb, int64_t ch, int64_t h, int64_t w, int8_t* dst, int64_t c_pad,

@@ -290,7 +290,7 @@ def conv3x3_fused(cfg, x, weight, bias, relu):
                 xq, sx = kernels.conv_quant(x, layer.ci_pad)
                 if layer.shift is None:
                     layer.calibrate_gpu(xq[:1])
-                b = None if bias is None else bias.to(x.device, torch.float32).contiguous()
+                b = kernels.gpu_bias(bias, x.device)
                 y = layer.gpu_fused(xq, sx, b, x.dtype, verify=layer.must_check(cfg, "fused"),
                                     want=lambda: _cpu_composite(layer, x, bias))
                 layer.device = "gpu"
@@ -374,7 +374,7 @@ def _gpu_chain(cfg, x, layers, biases, relu_after, pools):
                 L.calibrate_gpu(xq[:1])
             if L.device == "cpu":
                 return None
-            b = None if biases[i] is None else biases[i].to(dev, torch.float32).contiguous()
+            b = kernels.gpu_bias(biases[i], dev)
             if i == last:    # the last conv with its dequantize in one launch, checked as that launch
                 y = L.gpu_fused(xq, sx, b, x.dtype, verify=L.must_check(cfg, "fused"))
                 L.device = "gpu"

@@ -99,8 +99,11 @@ def _declare(L):
         "xdna_gemm_ksplit": ([i64, i64, i64, p, p], i),
         "xdna_gemm_i8_i32_ws": ([p, i64, p, i64, p, i64, i64, i64, i64, p, i64, p], i),
         "xdna_gemm_i8_dequant_ws": ([p, i64, p, p, i64, p, p, p, i, i64, i64, i64, i64, p, i64, p], i),
+        "xdna_gemm_i8_dequant_bias": ([p, i64, p, p, i64, p, p, i, p, i, i64, i64, i64, i64, p, i64, p], i),
         "xdna_linear_row": ([p, i, i64, p, i64, p, p, p, i, i64, i64, p, p], i),
+        "xdna_linear_row_bias": ([p, i, i64, p, i64, p, p, i, p, i, i64, i64, p, p], i),
         "xdna_gemm_bf16": ([p, i64, p, i64, p, p, i, i64, i64, i64, i64, p], i),
+        "xdna_gemm_bf16_bias": ([p, i64, p, i64, p, i, p, i, i64, i64, i64, i64, p], i),
         "xdna_gemm_bf16_silu": ([p, i64, p, i64, p, i64, i64, i64, i64, p], i),
         "xdna_pad_rows_i8": ([p, i64, i64, i64, p, i64, i64, p], i),
         "xdna_conv_quant_nhwc": ([p, i, i64, i64, i64, i64, p, i64, p, p, p], i),
@@ -109,6 +112,8 @@ def _declare(L):
         "xdna_conv3x3_i8": ([p, i64, i64, i64, i64, p, i64, i, i, p, p, p], i),
         "xdna_conv_dequant": ([p, i, i64, i64, i64, i64, p, p, p, p, i, p], i),
         "xdna_conv3x3_dequant": ([p, i64, i64, i64, i64, p, i64, i, i, p, p, p, p, i, p], i),
+        "xdna_conv3x3_dequant_bias": ([p, i64, i64, i64, i64, p, i64, i, i, p, p, p, i, p, i, p], i),
+        "xdna_conv_requant_next_bias": ([p, i, i, i, i64, i64, i64, i64, p, p, p, i, i, p, i64, p, p, p], i),
         "xdna_conv_requant_next": ([p, i, i, i, i64, i64, i64, i64, p, p, p, i, p, i64, p, p, p], i),
         "xdna_nchw_to_nhwc_i8": ([p, i64, i64, i64, i64, p, i64, p], i),
         "xdna_nhwc_to_nchw_i8": ([p, i64, i64, i64, i64, p, p], i),
@@ -130,10 +135,11 @@ def _declare(L):
 
 EXPORTS = ("xdna_abi_version", "xdna_last_error", "xdna_device_info", "xdna_quant_rows", "xdna_gemm_i8_i32",
            "xdna_gemm_i8_dequant", "xdna_gemm_ws_bytes", "xdna_gemm_ksplit", "xdna_gemm_i8_i32_ws", "xdna_gemm_i8_dequant_ws",
-           "xdna_linear_row",
-           "xdna_gemm_bf16", "xdna_gemm_bf16_silu", "xdna_pad_rows_i8", "xdna_conv_quant_nhwc",
+           "xdna_gemm_i8_dequant_bias", "xdna_linear_row", "xdna_linear_row_bias",
+           "xdna_gemm_bf16", "xdna_gemm_bf16_bias", "xdna_gemm_bf16_silu", "xdna_pad_rows_i8", "xdna_conv_quant_nhwc",
            "xdna_conv_quant_nhwc_noalloc", "xdna_conv_weight_pack",
-           "xdna_conv3x3_i8", "xdna_conv_dequant", "xdna_conv3x3_dequant", "xdna_conv_requant_next", "xdna_nchw_to_nhwc_i8",
+           "xdna_conv3x3_i8", "xdna_conv_dequant", "xdna_conv3x3_dequant", "xdna_conv3x3_dequant_bias",
+           "xdna_conv_requant_next", "xdna_conv_requant_next_bias", "xdna_nchw_to_nhwc_i8",
            "xdna_nhwc_to_nchw_i8",
            "xdna_tile_set", "xdna_tile_get", "xdna_tile_plan", "xdna_tile_clear", "xdna_rmsnorm_bf16",
            "xdna_add_rmsnorm_bf16", "xdna_qk_norm_rope",
@@ -148,6 +154,20 @@ def _check(status, what):
 
 def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+
+
+def gpu_bias(bias, dev):
+    """A bias (or None) as the launchers read it: on dev, contiguous, float32 / bfloat16 / float16 (any other
+    dtype as float32). The kernels widen the 16-bit ones, so a model's bias is used where it lies."""
+    if bias is None:
+        return None
+    if bias.dtype not in _DTYPE_CODE:
+        return bias.to(dev, torch.float32).contiguous()
+    return bias.to(dev).contiguous()
+
+
+def _bias_code(bias):
+    return F32 if bias is None else _DTYPE_CODE[bias.dtype]
 
 
 def _stream(dev):
@@ -409,9 +429,9 @@ def mm_i8_dequant(a, sx, w, sw, bias, out_dtype):
     if M and N:
         with _on(dev):
             ws, wsb = _gemm_ws(dev, M, N, K)
-            _check(lib().xdna_gemm_i8_dequant_ws(_ptr(a), a.stride(0), _ptr(sx), _ptr(w), w.stride(0), _ptr(sw),
-                                                 _ptr(bias), _ptr(y), _DTYPE_CODE[out_dtype], y.stride(0), M, N, K,
-                                                 ws, wsb, _stream(dev)), "gemm_i8_dequant")
+            _check(lib().xdna_gemm_i8_dequant_bias(_ptr(a), a.stride(0), _ptr(sx), _ptr(w), w.stride(0), _ptr(sw),
+                                                   _ptr(bias), _bias_code(bias), _ptr(y), _DTYPE_CODE[out_dtype],
+                                                   y.stride(0), M, N, K, ws, wsb, _stream(dev)), "gemm_i8_dequant")
     return y
 
 
@@ -443,9 +463,9 @@ def linear_row(x2d, w, sw, bias, out_dtype, sx=None):
     y = torch.empty((1, N), dtype=out_dtype, device=dev)
     if N:
         with _on(dev):
-            _check(lib().xdna_linear_row(_ptr(x2d), _DTYPE_CODE[x2d.dtype], K, _ptr(w), w.stride(0), _ptr(sw),
-                                         _ptr(bias), _ptr(y), _DTYPE_CODE[out_dtype], N, Kp, _ptr(sx),
-                                         _stream(dev)), "linear_row")
+            _check(lib().xdna_linear_row_bias(_ptr(x2d), _DTYPE_CODE[x2d.dtype], K, _ptr(w), w.stride(0), _ptr(sw),
+                                              _ptr(bias), _bias_code(bias), _ptr(y), _DTYPE_CODE[out_dtype], N, Kp,
+                                              _ptr(sx), _stream(dev)), "linear_row")
     return y
 
 
@@ -475,8 +495,9 @@ def mm_bf16(a, w, bias, out_dtype):
     y = torch.empty((M, N), dtype=out_dtype, device=dev)
     if M and N:
         with _on(dev):
-            _check(lib().xdna_gemm_bf16(_ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(bias), _ptr(y),
-                                        _DTYPE_CODE[out_dtype], y.stride(0), M, N, K, _stream(dev)), "gemm_bf16")
+            _check(lib().xdna_gemm_bf16_bias(_ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(bias), _bias_code(bias),
+                                             _ptr(y), _DTYPE_CODE[out_dtype], y.stride(0), M, N, K, _stream(dev)),
+                   "gemm_bf16")
     return y
 
 
@@ -587,9 +608,9 @@ def conv3x3_dequant(xq, wq, shift, relu, scale, sx, bias, out_dtype):
     y = torch.empty((n, co, h, w), dtype=out_dtype, device=dev)
     if n:
         with _on(dev):
-            _check(lib().xdna_conv3x3_dequant(_ptr(xq), n, h, w, c_pad, _ptr(wq), co, int(shift), int(bool(relu)),
-                                              _ptr(scale), _ptr(sx), _ptr(bias), _ptr(y), _DTYPE_CODE[out_dtype],
-                                              _stream(dev)), "conv3x3_dequant")
+            _check(lib().xdna_conv3x3_dequant_bias(_ptr(xq), n, h, w, c_pad, _ptr(wq), co, int(shift), int(bool(relu)),
+                                                   _ptr(scale), _ptr(sx), _ptr(bias), _bias_code(bias), _ptr(y),
+                                                   _DTYPE_CODE[out_dtype], _stream(dev)), "conv3x3_dequant")
     return y
 
 
@@ -605,9 +626,10 @@ def conv_requant_next(q, relu, pool, scale, sx, bias, x_dtype, c_pad_next, relu_
     ws = torch.empty((n, AMAX_WS_PER_IMAGE), dtype=torch.float32, device=dev)
     if n:
         with _on(dev):
-            _check(lib().xdna_conv_requant_next(_ptr(q), int(bool(relu)), int(bool(relu_y)), int(bool(pool)), n, h, w,
-                                                co, _ptr(scale), _ptr(sx), _ptr(bias), _DTYPE_CODE[x_dtype], _ptr(xq),
-                                                c_pad_next, _ptr(sxn), _ptr(ws), _stream(dev)), "conv_requant_next")
+            _check(lib().xdna_conv_requant_next_bias(_ptr(q), int(bool(relu)), int(bool(relu_y)), int(bool(pool)), n, h,
+                                                     w, co, _ptr(scale), _ptr(sx), _ptr(bias), _bias_code(bias),
+                                                     _DTYPE_CODE[x_dtype], _ptr(xq), c_pad_next, _ptr(sxn), _ptr(ws),
+                                                     _stream(dev)), "conv_requant_next")
     return xq, sxn
 
 

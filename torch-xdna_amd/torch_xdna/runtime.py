@@ -283,7 +283,7 @@ def _gpu_linear(cfg, x2d, qw, bias, dtype):
     dev = kernels.gpu_device(x2d)
     xg = x2d.to(dev)
     wq, sw = qw.gpu(dev)
-    b = None if bias is None else bias.to(dev, torch.float32).contiguous()
+    b = kernels.gpu_bias(bias, dev)
     if kernels.linear_row_ok(xg, qw.Kp):
         y = kernels.linear_row(xg, wq, sw, b, dtype)
         key = ("row", "rowq", _bucket(1, cfg.row_buckets), qw.N, qw.K, str(dtype))
@@ -302,7 +302,7 @@ def _gpu_bf16(cfg, x2d, qw, bias, dtype):
     dev = kernels.gpu_device(x2d)
     xb = kernels.bf16_rows(x2d.to(dev), qw.Kp)
     wb = qw.gpu_bf16(dev)
-    b = None if bias is None else bias.to(dev, torch.float32).contiguous()
+    b = kernels.gpu_bias(bias, dev)
     y = kernels.mm_bf16(xb, wb, b, dtype)
     stats.launches += 1
 
