@@ -286,3 +286,86 @@ def test_precision_bf16(gpu):
     y_cpu = run(net, x, policy="cpu", fallback="eager", precision="bf16")
     assert _stats()["calls"] == {"cpu": 3}
     assert rel_err(y, y_cpu) < 1e-2 and rel_err(y, ref) < 1e-2
+
+
+def _linear_args(gpu, cid, rows=24, k=160, n=72):
+    g = torch.Generator().manual_seed(3)
+    return (torch.randn(rows, k, generator=g).to(gpu), torch.randn(n, k, generator=g).to(gpu) * 0.05,
+            torch.randn(n, generator=g).to(gpu), False, cid)
+
+
+def test_direct_route_modes(gpu):
+    """The ops' direct route for plain GPU calls, and what must not take it: the same values in grad mode, no_grad
+    and inference mode; an output that needs a gradient refuses its backward as before; dispatch modes, fake tensors,
+    make_fx and a profiler see the op; a negated view, vmap and a complex tensor's part give the op's values."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from torch_xdna import Config, ops, runtime
+
+    op = torch.ops.xdna.linear
+    cid = ops.config_id(Config(policy="gpu", verify="off"))
+    x, w, b, t, cid = _linear_args(gpu, cid)
+    want = op(x.cpu(), w.cpu(), b.cpu(), t, ops.config_id(Config(policy="cpu")))
+    y = op(x, w, b, t, cid)
+    assert torch.equal(y.cpu(), want) and not y.requires_grad
+    with torch.no_grad():
+        p = torch.nn.Parameter(w)
+        assert torch.equal(op(x, p, b, t, cid), y)
+    with torch.inference_mode():
+        assert torch.equal(op(x, w, b, t, cid), y)
+    z = op(x, p, b, t, cid)
+    assert z.requires_grad and torch.equal(z, y)
+    with pytest.raises(RuntimeError, match="no autograd formula"):
+        z.sum().backward()
+    z = torch.ops.xdna.linear_cat(x, [w, p], [b, None], cid)
+    assert z.requires_grad and torch.equal(z[:, :72], y)
+
+    seen = []
+
+    class Log(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Log():
+        assert torch.equal(op(x, w, b, t, cid), y)
+    assert any("xdna.linear" in s for s in seen), seen
+    before = runtime.stats.launches
+    with FakeTensorMode() as mode:
+        f = op(mode.from_tensor(x), mode.from_tensor(w), mode.from_tensor(b), t, cid)
+        assert tuple(f.shape) == (24, 72) and f.device.type == "cuda"
+    assert runtime.stats.launches == before, "fake tensors launched kernels"
+    fx = make_fx(lambda a: op(a, w, b, t, cid))(x)
+    assert any("xdna.linear" in str(n.target) for n in fx.graph.nodes)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        op(x, w, b, t, cid)
+    assert any("xdna::linear" in e.key for e in prof.key_averages())
+    neg = torch.conj(torch.complex(torch.zeros_like(x), -x)).imag
+    assert neg.is_neg() and torch.equal(op(neg, w, b, t, cid), y)
+    assert torch.equal(torch.vmap(lambda v: op(v, w, b, t, cid))(torch.stack([x, 2 * x]))[0], y)
+    m = torch.compile(lambda a: torch.relu(op(a, w, b, t, cid)), backend="eager", fullgraph=True)
+    assert torch.equal(m(x), torch.relu(y))
+
+
+def test_direct_route_is_taken(gpu, monkeypatch):
+    """A plain call reaches the op's function without custom_op's wrappers on the stack; one whose input needs a
+    gradient goes through them."""
+    import traceback
+
+    from torch_xdna import Config, ops, runtime
+
+    cid = ops.config_id(Config(policy="gpu", verify="off"))
+    args = _linear_args(gpu, cid)
+    wrapped = []
+    real = runtime.linear
+
+    def spy(*a):
+        wrapped.append(any("_library" in f.filename for f in traceback.extract_stack()))
+        return real(*a)
+
+    monkeypatch.setattr(runtime, "linear", spy)
+    torch.ops.xdna.linear(*args)
+    torch.ops.xdna.linear(args[0].clone().requires_grad_(), *args[1:])
+    assert wrapped == [False, True]

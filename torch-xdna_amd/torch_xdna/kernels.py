@@ -38,6 +38,9 @@ def round_up(x, m):
 # ------------------------------------------------------------------------------ availability
 def available() -> bool:
     """True if xdna ops can run on the GPU in this process (library loads, a GPU is visible)."""
+    ok = _state["ok"]
+    if ok is not None:
+        return ok
     with _lock:
         if _state["ok"] is None:
             try:
@@ -72,6 +75,8 @@ def reset():
 def lib():
     """The loaded library; raises if it is not built or its ABI version differs."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             if not os.path.exists(LIB_PATH):
@@ -153,7 +158,7 @@ def _check(status, what):
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None     # every function's argtypes are declared
 
 
 def gpu_bias(bias, dev):
@@ -163,7 +168,9 @@ def gpu_bias(bias, dev):
         return None
     if bias.dtype not in _DTYPE_CODE:
         return bias.to(dev, torch.float32).contiguous()
-    return bias.to(dev).contiguous()
+    if bias.device != dev:
+        bias = bias.to(dev)
+    return bias if bias.is_contiguous() else bias.contiguous()
 
 
 def _bias_code(bias):
@@ -173,7 +180,7 @@ def _bias_code(bias):
 def _stream(dev):
     """torch's current stream on dev, as the raw HIP stream handle the library launches on."""
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(idx))
+    return torch._C._cuda_getCurrentRawStream(idx)
 
 
 _NOCTX = contextlib.nullcontext()
@@ -183,22 +190,23 @@ def _on(dev):
     """Device context for a launch on dev: none when dev is already the current device (the common
     case, and switching costs microseconds per launch)."""
     idx = dev.index
-    if idx is None or idx == torch.cuda.current_device():
+    if idx is None or idx == torch._C._cuda_getDevice():    # a tensor on dev: CUDA is initialised
         return _NOCTX
     return torch.cuda.device(idx)
 
 
 def _need_gpu(*ts):
     dev = ts[0].device
+    idx = ts[0].get_device()
     for t in ts:
-        if t is not None and (t.device.type != "cuda" or t.device != dev):
+        if t is not None and (not t.is_cuda or t.get_device() != idx):
             raise ValueError(f"xdna launchers take tensors on one GPU, got {t.device} and {dev}")
     return dev
 
 
 def gpu_device(t):
     """The GPU a tensor's GPU route runs on: its own device, or the current GPU for host tensors."""
-    return t.device if t.device.type == "cuda" else torch.device("cuda", torch.cuda.current_device())
+    return t.device if t.is_cuda else torch.device("cuda", torch.cuda.current_device())
 
 
 def num_cus(dev) -> int:
@@ -230,11 +238,26 @@ def direct_ok(N, K) -> bool:
     return K % 9 == 0 and K // 9 in (16, 32, 48, 64) and N % 32 == 0 and N <= 128
 
 
+# What the library plans for a shape, asked once while the tile table stays as it is (at most MAX_PLANS shapes, then
+# forgotten). A device without an index is whichever is current: its plans are asked each time.
+MAX_PLANS = 8192
+_variants = {}
+_plan_epoch = 0
+
+
+def _plans_changed():
+    global _plan_epoch
+    with _lock:
+        _plan_epoch += 1
+        _ws_need.clear()
+        _variants.clear()
+
+
 def tile_set(kind, M, N, K, tile):
     """Make every later launch of exactly (kind, M, N, K) use `tile` (a TILES name; "auto" removes the
     entry). For convs M = n*h*w, N = Co, K = 9*Ci_pad. Results do not depend on the tile."""
     _check(lib().xdna_tile_set(KINDS.get(kind, kind), M, N, K, TILE_ID[tile]), "tile_set")
-    _ws_need.clear()
+    _plans_changed()
 
 
 def tile_get(dev, kind, M, N, K) -> str:
@@ -249,7 +272,7 @@ def tile_get(dev, kind, M, N, K) -> str:
 
 def tile_clear():
     _check(lib().xdna_tile_clear(), "tile_clear")
-    _ws_need.clear()
+    _plans_changed()
 
 
 def tile_plan(dev, kind, M, N, K):
@@ -266,7 +289,23 @@ def gemm_variant(dev, M, N, K, kind=KIND_I8) -> str:
     """The kernels a GEMM of M x N x K runs (the library's plan): the head tile, after a tail split
     "+<tail tile>@<first tail row>", and for an int8 launch that splits K across workgroups "/k<splits>"
     after its tile. One NPU-program key of the reference (runtime.py:207) corresponds to one
-    (variant, N, K) here."""
+    (variant, N, K) here. Kept per shape until the tile table changes."""
+    if dev.index is None:
+        return _gemm_variant(dev, M, N, K, kind)
+    key = (dev.index, M, N, K, kind)
+    name = _variants.get(key)
+    if name is None:
+        if len(_variants) >= MAX_PLANS:
+            _variants.clear()
+        epoch = _plan_epoch
+        name = _gemm_variant(dev, M, N, K, kind)
+        with _lock:
+            if epoch == _plan_epoch:        # else the table changed under it: asked again next time
+                _variants[key] = name
+    return name
+
+
+def _gemm_variant(dev, M, N, K, kind):
     head, m1, tail = tile_plan(dev, kind, M, N, K)
     hk = tk = 1
     if kind == KIND_I8 and K % 16 == 0 and K >= 16:

@@ -12,8 +12,14 @@ calls it as an extern kernel.
 from typing import Optional
 
 import torch
+import torch._dynamo
 
 from . import conv, runtime, stack
+
+try:    # what custom_op registers for autograd (below); without it the ops keep only custom_op's own route
+    from torch._library.autograd import make_autograd_impl as _make_autograd_impl
+except ImportError:
+    _make_autograd_impl = None
 
 _configs = []  # cfg_id -> Config; the op's arguments must be plain values
 
@@ -125,3 +131,46 @@ def qwen3_stack(x: torch.Tensor, mask: torch.Tensor, stack_id: int, cfg_id: int)
 @qwen3_stack.register_fake
 def _(x, mask, stack_id, cfg_id):
     return x.new_empty((x.shape[0], x.shape[1], stack.out_features(stack_id)))
+
+
+# ------------------------------------------------------------------------------ GPU calls that need no autograd
+# custom_op's own route from the dispatcher to the function above passes through its autograd and backend wrappers in
+# Python, 9 us a call, as much as a small op's launches. A call whose tensors are ordinary GPU tensors, none of which
+# needs a gradient, has nothing to do there: the function is called at once. Anything else goes on as before: the
+# test is the dispatcher's own key set of the call, so a dispatch mode (fake tensors, tracing), a negated view, a
+# functional wrapper or any other layer that stands below autograd shows in it.
+_PLAIN = (torch._C.DispatchKeySet(torch._C.DispatchKey.CUDA)
+          | torch._C.DispatchKeySet(torch._C.DispatchKey.AutogradCUDA)).raw_repr()
+
+
+def _needs_grad(args):
+    for a in args:
+        if isinstance(a, torch.Tensor):
+            if a.requires_grad:
+                return True
+        elif isinstance(a, list) and _needs_grad(a):
+            return True
+    return False
+
+
+def _direct(custom, fn):
+    """Registers fn (the op's arguments -> its result) for plain GPU calls of the custom op."""
+    generic = _make_autograd_impl(custom._opoverload, custom)
+
+    def call(keyset, *args):
+        if keyset.raw_repr() != _PLAIN or (torch.is_grad_enabled() and _needs_grad(args)):
+            return generic(keyset, *args)
+        return fn(*args)
+
+    # as custom_op does for its functions: Dynamo never traces into the call
+    _lib.impl(custom._opoverload.name().split("::")[1], torch._dynamo.disable(call), "AutogradCUDA", with_keyset=True)
+
+
+if _make_autograd_impl is not None and hasattr(linear, "_opoverload"):
+    _lib = torch.library.Library("xdna", "FRAGMENT")
+    _direct(linear, lambda x, w, b, transposed, cid: runtime.linear(_configs[cid], x, w, b, transposed))
+    _direct(linear_cat, lambda x, ws, bs, cid: runtime.linear_cat(_configs[cid], x, ws, bs))
+    _direct(conv3x3_fused, lambda x, w, b, relu, cid: conv.conv3x3_fused(_configs[cid], x, w, b, relu))
+    _direct(conv3x3_chain, lambda x, ws, bs, relus, after, pools, cid: conv.conv3x3_chain(
+        _configs[cid], cid, x, list(ws), list(bs), list(relus), list(after), list(pools)))
+    _direct(qwen3_stack, lambda x, mask, sid, cid: stack.run(_configs[cid], sid, x, mask))

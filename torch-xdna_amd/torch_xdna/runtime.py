@@ -167,9 +167,9 @@ class _WeightCache:
         return len(self.entries)
 
     def get(self, ws, transposed):
-        key = (tuple((w.data_ptr(), tuple(w.shape), w._version) for w in ws), transposed)
+        key = (tuple([(w.data_ptr(), w.shape, w._version) for w in ws]), transposed)
         hit = self.entries.get(key)
-        if hit is not None and all(alive() is w for alive, w in zip(hit[0], ws)):
+        if hit is not None and all([alive() is w for alive, w in zip(hit[0], ws)]):
             return hit[1]
         qw = QWeight(ws, transposed)
 
@@ -255,8 +255,12 @@ def _program(cfg, kind, dev, R, qw, dtype=None):
 def _check(cfg, key, got, want, exact=True):
     """Compare one launch with the CPU route unless this program was already verified (Config.verify
     "first"; "always" checks every launch, "off" none): bit for bit, or (exact=False, the bf16 GEMM)
-    to the reference's 5e-2 relative norm with finite values (runtime.py:174-188)."""
-    if cfg.verify == "off" or (cfg.verify == "first" and _verified.get(key)):
+    to the reference's 5e-2 relative norm with finite values (runtime.py:174-188). key() gives the
+    program (worked out only where it is looked at)."""
+    if cfg.verify == "off":
+        return
+    key = key()
+    if cfg.verify == "first" and _verified.get(key):
         return
     want = want()
     got = got.cpu()
@@ -281,18 +285,19 @@ def _gpu_linear(cfg, x2d, qw, bias, dtype):
     """y [R, N] = W8A8(x2d) on the GPU: quantize kernel, then the GEMM with the fused dequantize; a single
     row (decode) whose layout allows it as one launch that quantizes the row itself (xdna_linear_row)."""
     dev = kernels.gpu_device(x2d)
-    xg = x2d.to(dev)
+    xg = x2d if x2d.is_cuda else x2d.to(dev)
     wq, sw = qw.gpu(dev)
     b = kernels.gpu_bias(bias, dev)
-    if kernels.linear_row_ok(xg, qw.Kp):
+    row = x2d.shape[0] == 1 and kernels.linear_row_ok(xg, qw.Kp)
+    if row:
         y = kernels.linear_row(xg, wq, sw, b, dtype)
-        key = ("row", "rowq", _bucket(1, cfg.row_buckets), qw.N, qw.K, str(dtype))
     else:
         xq, sx = kernels.quant_rows(xg, qw.Kp)
         y = kernels.mm_i8_dequant(xq, sx, wq, sw, b, dtype)
-        key = _program(cfg, "dq", dev, x2d.shape[0], qw, dtype)
     stats.launches += 1
-    _check(cfg, key, y, lambda: _cpu_linear(x2d, qw, bias, dtype))
+    _check(cfg, lambda: (("row", "rowq", _bucket(1, cfg.row_buckets), qw.N, qw.K, str(dtype)) if row else
+                         _program(cfg, "dq", dev, x2d.shape[0], qw, dtype)),
+           y, lambda: _cpu_linear(x2d, qw, bias, dtype))
     return y
 
 
@@ -311,7 +316,7 @@ def _gpu_bf16(cfg, x2d, qw, bias, dtype):
         if bias is not None:
             yb += bias.cpu().float()
         return yb.to(dtype)
-    _check(cfg, _program(cfg, "bf16", dev, x2d.shape[0], qw, dtype), y, want, exact=False)
+    _check(cfg, lambda: _program(cfg, "bf16", dev, x2d.shape[0], qw, dtype), y, want, exact=False)
     return y
 
 
@@ -330,7 +335,7 @@ def _gpu_acc(cfg, xq, qw):
     a = kernels.pad_k(xq.to(dev), qw.Kp)
     acc = kernels.mm_i8(a, wq)
     stats.launches += 1
-    _check(cfg, _program(cfg, "i8", dev, xq.shape[0], qw), acc, lambda: _cpu_acc(xq, qw))
+    _check(cfg, lambda: _program(cfg, "i8", dev, xq.shape[0], qw), acc, lambda: _cpu_acc(xq, qw))
     return acc
 
 
@@ -372,13 +377,14 @@ def _choose(cfg, R, qw, on_gpu, gpu_fn, cpu_fn):
     """'gpu' or 'cpu' for a call of R rows; gpu_fn / cpu_fn run it on either (for autotune)."""
     if cfg.policy == "cpu":
         return "cpu"
-    if kernels.available():
+    ok = kernels.available()
+    if ok:
         kernels.use_tuned(cfg.tuned_tilings)
     if on_gpu:
-        _require_lib()
-        if not kernels.available() or _key(cfg, R, qw) in _failed:
+        if not ok:
+            _require_lib()
             return "cpu"
-        return "gpu"
+        return "cpu" if _failed and _key(cfg, R, qw) in _failed else "gpu"
     if R < cfg.min_rows or R * qw.N * qw.K < cfg.min_macs:
         return "cpu"
     if not kernels.available():
@@ -416,10 +422,15 @@ def _float_only(cfg):
 # ------------------------------------------------------------------------------ the ops
 def _linear_impl(cfg, x, qw, bias, w_fp_fn):
     """Shared body of linear / linear_cat (runtime.py:326-355, :402-434)."""
-    shape = x.shape[:-1]
-    x2d = x.reshape(-1, x.shape[-1])
+    x2d = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     R = x2d.shape[0]
-    on_gpu = x.device.type == "cuda"
+    on_gpu = x.is_cuda
+
+    def shaped(y):      # on x's device, in x's shape
+        if y.device != x.device:
+            y = y.to(x.device)
+        return y if x.dim() == 2 else y.reshape(*x.shape[:-1], qw.N)
+
     t0 = time.perf_counter()
     if cfg.precision == "bf16":
         # runtime.py:299-313 / :340-345: the bf16 GEMM on the GPU, the float32 GEMM on the CPU
@@ -436,7 +447,7 @@ def _linear_impl(cfg, x, qw, bias, w_fp_fn):
             if y is None:
                 y = _cpu_bf16(x2d, w_fp_fn(), bias, x.dtype)
         stats.record(device, t0, R * qw.N * qw.K)
-        return y.to(x.device).reshape(*shape, qw.N)
+        return shaped(y)
     with _lock:
         device = _choose(cfg, R, qw, on_gpu, lambda: _gpu_linear(cfg, x2d, qw, bias, x.dtype),
                          lambda: _cpu_linear(x2d, qw, bias, x.dtype))
@@ -454,25 +465,24 @@ def _linear_impl(cfg, x, qw, bias, w_fp_fn):
             else:
                 y = _cpu_linear(x2d, qw, bias, x.dtype)
     stats.record(device, t0, R * qw.N * qw.K)
-    return y.to(x.device).reshape(*shape, qw.N)
+    return shaped(y)
 
 
 def linear(cfg, x, weight, bias, transposed):
     """y = x @ W^T + b (or x @ W when transposed) with W8A8 math on the chosen device."""
     N = weight.shape[1] if transposed else weight.shape[0]
-    if x.numel() == 0 or x.reshape(-1, x.shape[-1]).shape[0] == 0:
+    if x.numel() == 0:
         return x.new_zeros(*x.shape[:-1], N)
-    w_fp = weight.t() if transposed else weight
     if _float_only(cfg):
-        return torch.nn.functional.linear(x, w_fp.to(x.dtype), bias)
+        return torch.nn.functional.linear(x, (weight.t() if transposed else weight).to(x.dtype), bias)
     qw = qweight(weight, transposed)
-    return _linear_impl(cfg, x, qw, bias, lambda: w_fp)
+    return _linear_impl(cfg, x, qw, bias, lambda: weight.t() if transposed else weight)
 
 
 def linear_cat(cfg, x, weights, biases):
     """torch.cat([F.linear(x, w, b) for w, b in zip(weights, biases)], -1) as one W8A8 GEMM."""
     N = sum(w.shape[0] for w in weights)
-    if x.reshape(-1, x.shape[-1]).shape[0] == 0:
+    if x.numel() == 0 and x.reshape(-1, x.shape[-1]).shape[0] == 0:
         return x.new_zeros(*x.shape[:-1], N)
     if any(b is not None for b in biases):
         bias = torch.cat([b if b is not None else w.new_zeros(w.shape[0]) for w, b in zip(weights, biases)])
