@@ -780,6 +780,23 @@ def test_tiles_slices(gpu, tile, tile_table):
                               O.requant(c_oracle.conv3x3_acc(xq.numpy(), wq.numpy()), 9, False)), (n, ci, co, h, w_)
 
 
+@pytest.mark.parametrize("tile", ["auto", "t256x256w8", "t128x128", "t64x64", "t64x64k2", "t32x64k4"])
+@pytest.mark.parametrize("h,w", [(1, 1), (1, 2), (2, 1), (3, 2), (1, 131), (67, 2), (9, 15)])
+def test_conv_taps(gpu, tile, h, w, tile_table):
+    """The taps of a pixel that lie outside its image, for images down to one pixel, one row and one column (every
+    tap but some outside), several to a tile and starting inside one, with channels that are whole slices (one tap
+    per slice) and channels whose slices span taps: exact against the oracle."""
+    from torch_xdna import kernels
+
+    for n, ci, co in [(5, 64, 40), (3, 256, 40), (5, 48, 33), (3, 144, 33)]:
+        kernels.tile_set("conv", n * h * w, co, 9 * ci, tile)
+        xq, wq = _i8((n, ci, h, w), seed=ci + h), _i8((co, ci, 3, 3), seed=co + w)
+        packed = wq.permute(0, 2, 3, 1).reshape(co, 9, ci).contiguous()
+        q = kernels.conv3x3(kernels.nchw_to_nhwc(xq.to(gpu), ci), packed.to(gpu), 9, False)
+        assert np.array_equal(_np(q).transpose(0, 3, 1, 2),
+                              O.requant(c_oracle.conv3x3_acc(xq.numpy(), wq.numpy()), 9, False)), (n, ci, co)
+
+
 @pytest.mark.parametrize("m,n,k", [(16, 8192, 4096), (17, 5120, 1024), (17, 5104, 1024), (33, 2560, 2064), (64, 12900, 512),
                                    (65, 1001, 1552), (257, 1000, 1024), (513, 1024, 1040), (768, 16384, 1024),
                                    (340, 14336, 1024)])
