@@ -780,6 +780,65 @@ def test_tiles_slices(gpu, tile, tile_table):
                               O.requant(c_oracle.conv3x3_acc(xq.numpy(), wq.numpy()), 9, False)), (n, ci, co, h, w_)
 
 
+@pytest.mark.parametrize("tile", ["t256x256w8", "t128x128", "t64x64", "t32x64k4", "t64x32", "small_w4"])
+@pytest.mark.parametrize("ld,off", [(203, 0), (208, 1), (205, 3)])
+def test_unaligned_outputs(gpu, tile, ld, off, tile_table):
+    """GEMM outputs whose rows start at any element (odd row strides, a base off 16 bytes): the same values as into
+    aligned rows (one kernel, so bit for bit), nothing written between the rows."""
+    from torch_xdna import kernels as k
+
+    m, n, kk = 150, 203, 208
+    L, st, p = k.lib(), k._stream(gpu), k._ptr
+    for kind in ("i8", "bf16"):
+        k.tile_set(kind, m, n, kk, tile)
+    a, w = _i8((m, kk), seed=1).to(gpu), _i8((n, kk), seed=2).to(gpu)
+    sx, sw = (torch.rand(m) + 0.5).to(gpu), (torch.rand(n) + 0.5).to(gpu)
+    af, wf = a.to(torch.bfloat16), w.to(torch.bfloat16)
+    b = torch.randn(n).to(gpu)
+
+    def run(dt, code, ld, off, what):
+        buf = torch.full((off + m * ld,), 77, dtype=dt, device=gpu)
+        y = buf[off:]
+        if what == "i32":
+            k._check(L.xdna_gemm_i8_i32(p(a), kk, p(w), kk, p(y), ld, m, n, kk, st), what)
+        elif what == "dq":
+            k._check(L.xdna_gemm_i8_dequant_bias(p(a), kk, p(sx), p(w), kk, p(sw), p(b), k._bias_code(b), p(y), code, ld,
+                                                 m, n, kk, None, 0, st), what)
+        else:
+            k._check(L.xdna_gemm_bf16_bias(p(af), kk, p(wf), kk, p(b), k._bias_code(b), p(y), code, ld, m, n, kk, st), what)
+        assert (buf[:off] == 77).all()
+        rows = y.view(m, ld)
+        assert (rows[:, n:] == 77).all(), what
+        return rows[:, :n]
+
+    for dt, code in list(k._DTYPE_CODE.items()) + [(torch.int32, 0)]:
+        for what in (("i32",) if dt == torch.int32 else ("dq", "bf16")):
+            assert torch.equal(run(dt, code, ld, off, what), run(dt, code, 208, 0, what)), (dt, what)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("n,ci,co,h,w", [(3, 64, 70, 5, 7), (5, 32, 33, 1, 3), (3, 48, 130, 9, 15), (4, 20, 40, 1, 1)])
+@pytest.mark.parametrize("tile", ["auto", "t128x128", "t64x64", "t64x64k2"])
+def test_conv_dequant_odd_images(gpu, tile, dtype, n, ci, co, h, w, tile_table):
+    """Convs with odd pixel and channel counts: int8 rows of any alignment, and the fused dequantize of images whose
+    pixels do not come in aligned fours (pixels of two or more images in one group of four), bit for bit the
+    separate dequantize of the oracle-checked int8 outputs."""
+    from torch_xdna import kernels
+
+    c_pad = -(-ci // 16) * 16
+    kernels.tile_set("conv", n * h * w, co, 9 * c_pad, tile)
+    xq, wq = _i8((n, ci, h, w), seed=ci + h), _i8((co, ci, 3, 3), seed=co + w)
+    packed = torch.zeros(co, 9, c_pad, dtype=torch.int8)
+    packed[:, :, :ci] = wq.permute(0, 2, 3, 1).reshape(co, 9, ci)
+    xn, packed = kernels.nchw_to_nhwc(xq.to(gpu), c_pad), packed.to(gpu)
+    q = kernels.conv3x3(xn, packed, 9, True)
+    assert np.array_equal(_np(q).transpose(0, 3, 1, 2), O.requant(c_oracle.conv3x3_acc(xq.numpy(), wq.numpy()), 9, True))
+    scale, sx, b = (torch.rand(co) + 0.5).to(gpu), (torch.rand(n) + 0.5).to(gpu), torch.randn(co).to(gpu)
+    y = kernels.conv3x3_dequant(xn, packed, 9, True, scale, sx, b, DT[dtype])
+    f = scale.view(1, -1, 1, 1) * sx.view(-1, 1, 1, 1)
+    assert torch.equal(y, (q.permute(0, 3, 1, 2).float() * f + b.view(1, -1, 1, 1)).to(DT[dtype]))
+
+
 @pytest.mark.parametrize("tile", ["auto", "t256x256w8", "t128x128", "t64x64", "t64x64k2", "t32x64k4"])
 @pytest.mark.parametrize("h,w", [(1, 1), (1, 2), (2, 1), (3, 2), (1, 131), (67, 2), (9, 15)])
 def test_conv_taps(gpu, tile, h, w, tile_table):

@@ -69,7 +69,6 @@ struct EpiArgs {
   int shift;            // EPI_REQUANT
   int relu;             // EPI_REQUANT / EPI_CALIB
   int32_t* acc_max;     // EPI_CALIB
-  int vec_ok;           // output 16-byte aligned, row stride a multiple of 8 elements
   int dq_out;           // EPI_REQUANT: 0 writes the integers (NHWC); XDNA_F32 / BF16 / F16 + 1: the
                         // integers dequantized with sw = the conv's weight scales and sx = the per-image
                         // scales (+ bias), written NCHW in that dtype (out, sx not shifted by launch rows)
@@ -165,17 +164,26 @@ struct EpiCols {
   }
 };
 
+// Vectors stored at their elements' alignment (rows of any stride: global stores take them whole). One element at
+// a time where the rows were off 16 bytes: 1999 x 1001 x 1552 int8 to bf16 13.1 us, 11.7 as vectors (1999 x 1000
+// x 1552, aligned, 11.2); bf16 699 x 1001 x 1024 7.6, 7.0; the fused dequantize of 4 x 100 x 75 x 93 -> 200 32.4, 25.4.
+typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2u __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t u32u __attribute__((aligned(2)));
+typedef uint32_t u32x2b __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t u32b __attribute__((aligned(1)));
+
 // One lane's CW outputs: row m, columns n .. n+CW-1 (acc[r] is column n + r). FULL: the caller has
-// established that the whole tile is in bounds and the output rows take CW-wide vector stores, so
-// there are no per-element tests. e.vec_ok: output rows are 16-byte aligned with a row stride that
-// is a multiple of 8 elements (CW-wide stores at column multiples of CW are aligned).
+// established that the whole tile is in bounds, so there are no per-element tests.
 template <int EPI, bool FULL, int CW>
 __device__ __forceinline__ void epilogue_w(const EpiArgs& e, int64_t m, int64_t n, int64_t M, int64_t N,
                                            const int32_t (&acc)[CW], int& calib, const EpiCols<EPI, CW>& cols,
                                            float sxm) {
   static_assert(CW == 4 || CW == 8, "4 or 8 columns per lane");
   if (!FULL && m >= M) return;
-  const bool vec = FULL || (e.vec_ok && n + CW - 1 < N);
+  const bool vec = FULL || n + CW - 1 < N;
   if constexpr (EPI == EPI_CALIB) {
 #pragma unroll
     for (int r = 0; r < CW; ++r)
@@ -185,7 +193,7 @@ __device__ __forceinline__ void epilogue_w(const EpiArgs& e, int64_t m, int64_t 
     if (vec) {
 #pragma unroll
       for (int q = 0; q < CW / 4; ++q)
-        *reinterpret_cast<i32x4*>(c + 4 * q) = i32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+        *reinterpret_cast<i32x4u*>(c + 4 * q) = i32x4u{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
     } else {
 #pragma unroll
       for (int r = 0; r < CW; ++r)
@@ -209,8 +217,8 @@ __device__ __forceinline__ void epilogue_w(const EpiArgs& e, int64_t m, int64_t 
     }
     uint8_t* o = reinterpret_cast<uint8_t*>(e.out) + m * e.ldo + n;
     if (vec) {
-      if constexpr (CW == 8) *reinterpret_cast<uint2*>(o) = make_uint2(packed[0], packed[1]);
-      else *reinterpret_cast<uint32_t*>(o) = packed[0];
+      if constexpr (CW == 8) *reinterpret_cast<u32x2b*>(o) = u32x2b{packed[0], packed[1]};
+      else *reinterpret_cast<u32b*>(o) = packed[0];
     } else {
 #pragma unroll
       for (int r = 0; r < CW; ++r)
@@ -233,12 +241,12 @@ __device__ __forceinline__ void epilogue_w(const EpiArgs& e, int64_t m, int64_t 
     }
     uint16_t* y = reinterpret_cast<uint16_t*>(e.out) + m * e.ldo + n / 2;
     if (vec) {
-      if constexpr (CW == 8) *reinterpret_cast<uint2*>(y) = make_uint2(h[0], h[1]);
-      else *reinterpret_cast<uint32_t*>(y) = h[0];
+      if constexpr (CW == 8) *reinterpret_cast<u32x2u*>(y) = u32x2u{h[0], h[1]};
+      else *reinterpret_cast<u32u*>(y) = h[0];
     } else {
 #pragma unroll
       for (int q = 0; q < CW / 4; ++q)
-        if (n + 4 * q < N) *reinterpret_cast<uint32_t*>(y + 2 * q) = h[q];
+        if (n + 4 * q < N) *reinterpret_cast<u32u*>(y + 2 * q) = h[q];
     }
   } else {
     // EPI_DQ_*: ((float)acc * sx[m]) * sw[n] (+ bias[n]), each step rounded once;
@@ -263,7 +271,7 @@ __device__ __forceinline__ void epilogue_w(const EpiArgs& e, int64_t m, int64_t 
       if (vec) {
 #pragma unroll
         for (int q = 0; q < CW / 4; ++q)
-          *reinterpret_cast<f32x4*>(y + 4 * q) = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+          *reinterpret_cast<f32x4u*>(y + 4 * q) = f32x4u{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
       } else {
 #pragma unroll
         for (int r = 0; r < CW; ++r)
@@ -277,8 +285,8 @@ __device__ __forceinline__ void epilogue_w(const EpiArgs& e, int64_t m, int64_t 
                                                           : f32x2_to_f16x2_bits(v[2 * q], v[2 * q + 1]);
       uint16_t* y = reinterpret_cast<uint16_t*>(e.out) + off;
       if (vec) {
-        if constexpr (CW == 8) *reinterpret_cast<uint4*>(y) = make_uint4(h[0], h[1], h[2], h[3]);
-        else *reinterpret_cast<uint2*>(y) = make_uint2(h[0], h[1]);
+        if constexpr (CW == 8) *reinterpret_cast<u32x4u*>(y) = u32x4u{h[0], h[1], h[2], h[3]};
+        else *reinterpret_cast<u32x2u*>(y) = u32x2u{h[0], h[1]};
       } else {
 #pragma unroll
         for (int r = 0; r < CW; ++r)
@@ -288,7 +296,7 @@ __device__ __forceinline__ void epilogue_w(const EpiArgs& e, int64_t m, int64_t 
   }
 }
 
-// Per element: an image boundary, an unaligned run, the end of the launch's rows.
+// Per element: an image boundary, the end of the launch's rows.
 __device__ __forceinline__ void epilogue_rqdq_each(const EpiArgs& e, int64_t hw, int64_t b, int64_t p, int64_t m,
                                                 int64_t n, int64_t M, int64_t N, const float (&v)[4], float fo, float bo) {
   const int dt = e.dq_out - 1;
@@ -310,7 +318,7 @@ __device__ __forceinline__ void epilogue_rqdq_each(const EpiArgs& e, int64_t hw,
 }
 
 // Where four consecutive output pixels m .. m+3 (launch rows) of the fused dequantize go: image b and pixel p
-// within it, and whether the four lie in one image at an aligned position (then one vector store per channel,
+// within it, and whether the four lie in one image (then one vector store per channel,
 // with the image's scale sx). The same for every channel, so the caller finds it once per four pixels. b_c /
 // sx_c: an image index and its scale the caller loaded ahead (the image of the wave's first pixel), used
 // instead of a load of e.sx[b] when the pixels lie in that image. Rows past M: fast = false, nothing loaded.
@@ -335,7 +343,7 @@ __device__ __forceinline__ RqPix rq_pixel(const EpiArgs& e, const ConvGeom& cg, 
     r.b = gp / hw;
     r.p = gp - r.b * hw;
   }
-  r.fast = m + 3 < M && r.p + 3 < hw && (r.p % 4) == 0 && hw % 4 == 0;
+  r.fast = m + 3 < M && r.p + 3 < hw;
   if (r.fast) r.sx = r.b == b_c ? sx_c : e.sx[r.b];
   return r;
 }
@@ -343,8 +351,8 @@ __device__ __forceinline__ RqPix rq_pixel(const EpiArgs& e, const ConvGeom& cg, 
 // The conv's requantize fused with the op's dequantize: four consecutive output pixels m .. m+3 (launch
 // rows, placed by rq_pixel) of channel n, int32 sums in a[]. Each is requantized as EPI_REQUANT does, then
 // dequantized as the separate dequantize kernel does, y = (float)q * (scale[n] * sx[image]) (+ bias[n]),
-// and stored NCHW in dtype e.dq_out - 1: one 16-byte (float32) or 8-byte store when the four pixels lie in
-// one image at an aligned position, else per element.
+// and stored NCHW in dtype e.dq_out - 1: one 16-byte (float32) or 8-byte store at the elements' alignment when the
+// four pixels lie in one image, else per element.
 __device__ __forceinline__ void epilogue_rqdq(const EpiArgs& e, const ConvGeom& cg, const RqPix& px, int64_t m,
                                               int64_t n, int64_t M, int64_t N, const int32_t (&a)[4], float fo,
                                               float bo) {
@@ -373,11 +381,11 @@ __device__ __forceinline__ void epilogue_rqdq(const EpiArgs& e, const ConvGeom& 
   }
   char* o = reinterpret_cast<char*>(e.out) + ((b * N + n) * hw + p) * (dt == XDNA_F32 ? 4 : 2);
   if (dt == XDNA_F32) {
-    *reinterpret_cast<f32x4*>(o) = f32x4{t[0], t[1], t[2], t[3]};
+    *reinterpret_cast<f32x4u*>(o) = f32x4u{t[0], t[1], t[2], t[3]};
   } else if (dt == XDNA_BF16) {
-    *reinterpret_cast<uint2*>(o) = make_uint2(f32x2_to_bf16x2_bits(t[0], t[1]), f32x2_to_bf16x2_bits(t[2], t[3]));
+    *reinterpret_cast<u32x2u*>(o) = u32x2u{f32x2_to_bf16x2_bits(t[0], t[1]), f32x2_to_bf16x2_bits(t[2], t[3])};
   } else {
-    *reinterpret_cast<uint2*>(o) = make_uint2(f32x2_to_f16x2_bits(t[0], t[1]), f32x2_to_f16x2_bits(t[2], t[3]));
+    *reinterpret_cast<u32x2u*>(o) = u32x2u{f32x2_to_f16x2_bits(t[0], t[1]), f32x2_to_f16x2_bits(t[2], t[3])};
   }
 }
 
@@ -1085,8 +1093,7 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
   for (int jp = 0; jp < FN / CB; ++jp) cols_pre[jp].finish(e);
   int8_t* stg = lds + wave * 32 * PITCH;     // group 0: lds == lds_all
   int calib = 0;
-  // uniform: the whole tile is inside M x N and the output rows take CW-wide vector stores
-  const bool full = m0 + BM <= M && n0 + BN <= N && (EPI == EPI_CALIB || e.vec_ok);
+  const bool full = m0 + BM <= M && n0 + BN <= N;   // uniform: the whole tile is inside M x N
   const int rsub = lane >> 3;            // read-back: row rr * 8 + rsub, columns CW * (lane & 7) ..
   const int cq = lane & 7;
   // the conv's fused dequantize (EPI_REQUANT with e.dq_out, uniform): the staged block (32 pixels x COLS
@@ -2474,7 +2481,6 @@ int xdna_gemm_i8_i32_ws(const int8_t* a, int64_t lda, const int8_t* w, int64_t l
   EpiArgs e{};
   e.out = c;
   e.ldo = ldc;
-  e.vec_ok = (ldc % 8 == 0) && aligned(c, 16);
   e.ws = ws;
   e.ws_bytes = ws ? ws_bytes : 0;
   const int tile = choose_tile(XDNA_KIND_I8, m, n, k, k);
@@ -2504,7 +2510,6 @@ int xdna_gemm_i8_dequant_bias(const int8_t* a, int64_t lda, const float* sx, con
   e.sw = sw;
   e.bias = bias;
   e.bias_dt = bias_dtype;
-  e.vec_ok = (ldy % 8 == 0) && aligned(y, 16);
   e.ws = ws;
   e.ws_bytes = ws ? ws_bytes : 0;
   hipStream_t st = as_stream(stream);
@@ -2572,7 +2577,6 @@ int xdna_gemm_bf16_bias(const void* a, int64_t lda, const void* w, int64_t ldw, 
   e.ldo = ldy;
   e.bias = bias;
   e.bias_dt = bias_dtype;
-  e.vec_ok = (ldy % 8 == 0) && aligned(y, 16);
   // the engine stages bytes: a bf16 row of k values is 2 * k bytes
   const int8_t* ab = static_cast<const int8_t*>(a);
   const int8_t* wb = static_cast<const int8_t*>(w);
@@ -2601,7 +2605,6 @@ int xdna_gemm_bf16_silu(const void* a, int64_t lda, const void* w, int64_t ldw, 
   EpiArgs e{};
   e.out = y;
   e.ldo = ldy;
-  e.vec_ok = (ldy % 4 == 0) && aligned(y, 8);
   const int8_t* ab = static_cast<const int8_t*>(a);
   const int8_t* wb = static_cast<const int8_t*>(w);
   const int tile = choose_tile(XDNA_KIND_BF16, m, n2, k, 2 * k);
@@ -2627,7 +2630,6 @@ int xdna_conv3x3_i8(const int8_t* x, int64_t nb, int64_t h, int64_t w, int64_t c
   e.out = y;
   e.ldo = co;
   e.shift = shift;
-  e.vec_ok = (co % 8 == 0) && aligned(y, 16);
   return launch_conv<EPI_REQUANT>(x, nb, h, w, c_pad, wq, co, e, st);
 }
 
