@@ -217,6 +217,12 @@ int xdna_linear_row(const void* x, int x_dtype, int64_t kx, const int8_t* w, int
 int xdna_gemm_bf16(const void* a, int64_t lda, const void* w, int64_t ldw, const float* bias, void* y, int y_dtype,
                    int64_t ldy, int64_t m, int64_t n, int64_t k, void* stream);
 
+/* y[r, :k] = bf16(x[r, :k]) (round to nearest even), y[r, k:k_pad] = 0: activations of any float dtype,
+ * row stride and element alignment as operand rows of xdna_gemm_bf16 (the .to(torch.bfloat16) of
+ * torch_xdna/runtime.py:212-237 and its zero padding). y: 16-byte aligned, k_pad and ld_y multiples of 8. */
+int xdna_cast_rows_bf16(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t ld_x, void* y, int64_t ld_y,
+                        int64_t k_pad, void* stream);
+
 /* dst[r, :cols] = src[r, :cols], dst[r, cols:cols_pad] = 0 for int8 rows (aligning an int8
  * activation handed to xdna::linear_i8, torch_xdna/ops.py:49-55, to the 16-byte K rule). */
 int xdna_pad_rows_i8(const int8_t* src, int64_t rows, int64_t cols, int64_t ld_src, int8_t* dst,

@@ -92,6 +92,10 @@ def test_argument_validation(lib):
     assert f(None, 1, 16, None, 16, None, None, None, 1, 0, 16, None, None) == 0   # n = 0: nothing to do
     assert lib.xdna_quant_rows(p, 9, 4, 16, 16, p, 16, 16, p, None) == -1
     assert lib.xdna_quant_rows(p, 0, 4, 16, 8, p, 16, 16, p, None) == -1          # ld_x < k
+    assert lib.xdna_cast_rows_bf16(p, 3, 4, 16, 16, p, 16, 16, None) == -1        # x_dtype
+    assert lib.xdna_cast_rows_bf16(p, 0, 4, 16, 16, p, 20, 20, None) == -1        # k_pad % 8
+    assert lib.xdna_cast_rows_bf16(ctypes.c_void_p(18), 0, 4, 16, 16, p, 16, 16, None) == -1   # x off its elements
+    assert lib.xdna_cast_rows_bf16(None, 0, 0, 16, 16, None, 16, 16, None) == 0
     assert lib.xdna_conv3x3_i8(p, 1, 4, 4, 15, p, 8, 3, 0, p, None, None) == -1    # c_pad % 16
     assert lib.xdna_conv3x3_i8(p, 1, 4, 4, 16, p, 8, 0, 0, p, None, None) == -1    # shift 0
     assert "shift" in lib.xdna_last_error().decode()

@@ -120,6 +120,27 @@ def test_conv_quant_ragged(gpu, dtype, n, ch, h, w, c_pad):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("rows,k,off,ld", [(1, 1, 0, 1), (3, 7, 1, 9), (5, 8, 1, 8), (300, 1001, 0, 1001), (64, 1537, 3, 1600),
+                                           (257, 2048, 0, 2048)])
+def test_cast_rows_bf16(gpu, dtype, rows, k, off, ld):
+    """Operand rows of the bf16 GEMM from rows of any dtype, width, stride and alignment: torch's rounding bit for bit
+    (infinities, subnormals and values that round to infinity with it), NaN where it was, zeros past k."""
+    from torch_xdna import kernels
+
+    v = _rand((off + rows * ld,), torch.float32, seed=k)
+    v[: 1 + off] = float("inf")
+    v[-1] = float("nan")
+    if dtype == "f32" and v.numel() > 40:
+        v[20:24] = torch.tensor([3.4e38, 1e-40, -2.0 ** -133, 1.00390625])
+    x = v.to(DT[dtype]).to(gpu)[off:].view(rows, ld)[:, :k]
+    for kp in (-(-k // 8) * 8, -(-k // 8) * 8 + 16):
+        y, want = kernels.bf16_rows(x, kp).cpu(), x.cpu().to(torch.bfloat16)
+        nan = want.isnan()
+        assert torch.equal(y[:, :k].isnan(), nan) and not y[:, k:].any()
+        assert torch.equal(y[:, :k].masked_fill(nan, 0).view(torch.int16), want.masked_fill(nan, 0).view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("k", [1024, 200, 16384, 40000])
 def test_quant_rows_near_half(gpu, dtype, k):
     """Quotients x / s placed within 6e-5 of half-integers, on both sides, exactly on them and at fractions

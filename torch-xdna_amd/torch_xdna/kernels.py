@@ -110,6 +110,7 @@ def _declare(L):
         "xdna_gemm_bf16": ([p, i64, p, i64, p, p, i, i64, i64, i64, i64, p], i),
         "xdna_gemm_bf16_bias": ([p, i64, p, i64, p, i, p, i, i64, i64, i64, i64, p], i),
         "xdna_gemm_bf16_silu": ([p, i64, p, i64, p, i64, i64, i64, i64, p], i),
+        "xdna_cast_rows_bf16": ([p, i, i64, i64, i64, p, i64, i64, p], i),
         "xdna_pad_rows_i8": ([p, i64, i64, i64, p, i64, i64, p], i),
         "xdna_conv_quant_nhwc": ([p, i, i64, i64, i64, i64, p, i64, p, p, p], i),
         "xdna_conv_quant_nhwc_noalloc": ([p, i, i64, i64, i64, i64, p, i64, p, p], i),
@@ -141,7 +142,8 @@ def _declare(L):
 EXPORTS = ("xdna_abi_version", "xdna_last_error", "xdna_device_info", "xdna_quant_rows", "xdna_gemm_i8_i32",
            "xdna_gemm_i8_dequant", "xdna_gemm_ws_bytes", "xdna_gemm_ksplit", "xdna_gemm_i8_i32_ws", "xdna_gemm_i8_dequant_ws",
            "xdna_gemm_i8_dequant_bias", "xdna_linear_row", "xdna_linear_row_bias",
-           "xdna_gemm_bf16", "xdna_gemm_bf16_bias", "xdna_gemm_bf16_silu", "xdna_pad_rows_i8", "xdna_conv_quant_nhwc",
+           "xdna_gemm_bf16", "xdna_gemm_bf16_bias", "xdna_gemm_bf16_silu", "xdna_cast_rows_bf16", "xdna_pad_rows_i8",
+           "xdna_conv_quant_nhwc",
            "xdna_conv_quant_nhwc_noalloc", "xdna_conv_weight_pack",
            "xdna_conv3x3_i8", "xdna_conv_dequant", "xdna_conv3x3_dequant", "xdna_conv3x3_dequant_bias",
            "xdna_conv_requant_next", "xdna_conv_requant_next_bias", "xdna_nchw_to_nhwc_i8",
@@ -510,12 +512,20 @@ def linear_row(x2d, w, sw, bias, out_dtype, sx=None):
 
 def bf16_rows(x2d, k_pad):
     """x2d as bf16 [R, k_pad] rows the bf16 GEMM reads (round to nearest even; zero columns past K,
-    16-byte aligned rows): the tensor itself when it already qualifies, else one copy."""
-    _need_gpu(x2d)
+    16-byte aligned rows): the tensor itself when it already qualifies, else one copy (one launch for rows of
+    contiguous float elements)."""
+    dev = _need_gpu(x2d)
     R, K = x2d.shape
     if (x2d.dtype == torch.bfloat16 and K == k_pad and x2d.stride(1) == 1 and x2d.stride(0) % 8 == 0
             and x2d.data_ptr() % 16 == 0):
         return x2d
+    if x2d.dtype in _DTYPE_CODE and x2d.stride(1) == 1 and x2d.stride(0) >= K > 0 and k_pad % 8 == 0:
+        out = torch.empty((R, k_pad), dtype=torch.bfloat16, device=dev)
+        if R:
+            with _on(dev):
+                _check(lib().xdna_cast_rows_bf16(_ptr(x2d), _DTYPE_CODE[x2d.dtype], R, K, x2d.stride(0), _ptr(out), k_pad,
+                                                 k_pad, _stream(dev)), "cast_rows_bf16")
+        return out
     out = torch.zeros((R, k_pad), dtype=torch.bfloat16, device=x2d.device) if K != k_pad else \
         torch.empty((R, k_pad), dtype=torch.bfloat16, device=x2d.device)
     out[:, :K].copy_(x2d)
