@@ -839,7 +839,7 @@ def test_unaligned_outputs(gpu, tile, ld, off, tile_table):
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("n,ci,co,h,w", [(3, 64, 70, 5, 7), (5, 32, 33, 1, 3), (3, 48, 130, 9, 15), (4, 20, 40, 1, 1)])
-@pytest.mark.parametrize("tile", ["auto", "t128x128", "t64x64", "t64x64k2"])
+@pytest.mark.parametrize("tile", ["auto", "t128x128", "t64x64", "t64x64k2", "t32x32k4", "t32x64k4", "t128x128k2"])
 def test_conv_dequant_odd_images(gpu, tile, dtype, n, ci, co, h, w, tile_table):
     """Convs with odd pixel and channel counts: int8 rows of any alignment, and the fused dequantize of images whose
     pixels do not come in aligned fours (pixels of two or more images in one group of four), bit for bit the
@@ -860,7 +860,29 @@ def test_conv_dequant_odd_images(gpu, tile, dtype, n, ci, co, h, w, tile_table):
     assert torch.equal(y, (q.permute(0, 3, 1, 2).float() * f + b.view(1, -1, 1, 1)).to(DT[dtype]))
 
 
-@pytest.mark.parametrize("tile", ["auto", "t256x256w8", "t128x128", "t64x64", "t64x64k2", "t32x64k4"])
+@pytest.mark.parametrize("n,ci,co,h,w,tile", [(1, 64, 192, 28, 28, "t32x32k4"), (1, 63, 180, 37, 40, "t32x64k4"),
+                                              (8, 96, 96, 30, 30, "t64x64k2"), (1, 48, 192, 28, 28, None),
+                                              (4, 192, 320, 50, 50, "t128x128k2"), (4, 190, 320, 50, 50, "t128x128k2"),
+                                              (4, 176, 320, 50, 50, "t128x128")])
+def test_conv_rule(gpu, n, ci, co, h, w, tile, tile_table):
+    """Convs on both sides of the rule's lines for K groups (the number of tiles against 256 CUs, 576 and 1728 bytes
+    of K), channels whole slices or not: exact against the oracle."""
+    from torch_xdna import kernels
+
+    c_pad = -(-ci // 16) * 16
+    tile_table.tile_clear()
+    if tile is not None:
+        assert kernels.tile_plan(gpu, "conv", n * h * w, co, 9 * c_pad)[0] == tile
+    xq, wq = _i8((n, ci, h, w), seed=ci + h), _i8((co, ci, 3, 3), seed=co + w)
+    packed = torch.zeros(co, 9, c_pad, dtype=torch.int8)
+    packed[:, :, :ci] = wq.permute(0, 2, 3, 1).reshape(co, 9, ci)
+    q = kernels.conv3x3(kernels.nchw_to_nhwc(xq.to(gpu), c_pad), packed.to(gpu), 10, False)
+    assert np.array_equal(_np(q).transpose(0, 3, 1, 2),
+                          O.requant(c_oracle.conv3x3_acc(xq.numpy(), wq.numpy()), 10, False))
+
+
+@pytest.mark.parametrize("tile", ["auto", "t256x256w8", "t128x128", "t64x64", "t64x64k2", "t32x64k4", "t32x32k4",
+                                  "t128x128k2"])
 @pytest.mark.parametrize("h,w", [(1, 1), (1, 2), (2, 1), (3, 2), (1, 131), (67, 2), (9, 15)])
 def test_conv_taps(gpu, tile, h, w, tile_table):
     """The taps of a pixel that lie outside its image, for images down to one pixel, one row and one column (every

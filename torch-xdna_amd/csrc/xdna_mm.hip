@@ -1710,14 +1710,19 @@ int tile_lookup(int kind, int64_t m, int64_t n, int64_t k) {
 //   * GEMMs with few tiles and K of at least 1 KB: the smallest of 32 x 32, 32 x 64 (4 K groups each) and, from 2 KB,
 //     64 x 64 (2 groups) that makes at most one round of workgroups (128 x 1024 x 3072 5.7 against 7.1 us in 32 x 64,
 //     200 x 1001 x 1552 5.4 against 7.8 in 64 x 64 without groups, 512 x 1001 x 1552 7.2 against 8.1);
-//   * convs with few tiles and K of at least 2 KB: 32 x 32 x 4 groups below an eighth of a round of 64 x 64 tiles,
-//     32 x 64 x 4 groups up to half a round, 64 x 64 x 2 groups up to a round;
+//   * convs the same, 64 x 64 too, from K of 576 bytes (64 channels): their slices cost more than a GEMM's, so splitting
+//     them pays earlier (784 pixels x 192 channels 5.4 -> 4.8 us at 64 input channels, 11.9 -> 6.1 at 224; 1480 x 180 x
+//     9 * 112 8.1 -> 5.7; 7200 x 96 x 9 * 200 11.9 -> 9.1, all against 64 x 64 without groups; 64 x 64 with two groups
+//     is even at 64 channels);
 //   * 64 x 64 for N <= 64; for N <= 128 no 256-wide tile (half of it would be idle);
 //   * 256 x 256 with 8 waves (one workgroup per CU) from 1.5 rounds of such tiles, from three quarters of a round for
 //     deep K (>= 4096 bytes), where its lower LDS traffic per MAC outweighs the idle CUs, and, GEMMs, between three
 //     quarters and one round (3000 x 4096 x 1024 21.5 against 23.3 us in 128 x 128); then, GEMMs of K of at least 1 KB,
 //     192 x 256 (699 x 14336 x 4096 50 against 61 us) and the 8-wave 256 x 128 (333 x 14336 x 4096 32 against 36 us,
 //     bf16 1056 x 6144 x 1024 19.1 against 20.1) where they make 0.8 to 1 round;
+//   * convs whose 128 x 128 tiles make three quarters to one round: those with two K groups once there are 27 slices
+//     (6272 x 512 x 4608 30.2 -> 24.5 us, 12544 x 256 x 2304 17.5 -> 16.1, 10000 x 320 x 1728 15.4 -> 15.1; even at 18
+//     slices, 4% slower at 15);
 //   * otherwise, once 128 x 128 tiles fill three quarters of the CUs: 128 x 256 (four waves) for deep K
 //     when there are at least half a round of 256-wide tiles, else 128 x 128;
 //   * 64 x 64 otherwise.
@@ -1730,10 +1735,10 @@ int rule_tile(int64_t M, int64_t N, int64_t kbytes, bool small_ok, bool conv) {
   const int64_t cus = device_cus();
   auto tiles = [&](int64_t bm, int64_t bn) { return cdiv(M, bm) * cdiv(N, bn); };
   const int64_t t64 = tiles(64, 64), t128 = tiles(128, 128), t256 = tiles(256, 256);
-  if (!conv && kbytes >= 1024) {
+  if (kbytes >= (conv ? 576 : 1024)) {
     if (tiles(32, 32) <= cus) return T_32x32K4;
     if (tiles(32, 64) <= cus) return T_32x64K4;
-    if (kbytes >= 2048 && t64 <= cus) return T_64x64K2;
+    if ((conv || kbytes >= 2048) && t64 <= cus) return T_64x64K2;
   }
   if (!conv && M <= 32) return T_32x64;
   // narrow outputs with rows for at least two rounds of 256 x 64 tiles (the VGG-16 224 x 224 convs): a
@@ -1748,12 +1753,8 @@ int rule_tile(int64_t M, int64_t N, int64_t kbytes, bool small_ok, bool conv) {
     if (kbytes >= 1024 && round(tiles(192, 256))) return T_192x256;
     if (kbytes >= 1024 && round(tiles(256, 128))) return T_256x128W8;
   }
+  if (conv && kbytes >= 1728 && 4 * t128 >= 3 * cus && t128 <= cus) return T_128x128K2;
   if (4 * t128 >= 3 * cus) return (N > 128 && deep && 2 * t256 >= cus) ? T_128x256 : T_128x128;
-  if (kbytes >= 2048) {
-    if (8 * t64 < cus) return T_32x32K4;
-    if (2 * t64 <= cus) return T_32x64K4;
-    if (t64 <= cus) return T_64x64K2;
-  }
   return T_64x64;
 }
 
