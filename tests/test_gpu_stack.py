@@ -239,6 +239,42 @@ def test_attention_bf16_forms(gpu, nh, nkv, scale, lens):
             assert rel_err(out[s0:s0 + n, h], p @ v[s0:s0 + n, kv].double()) < 1e-2, (n, h)
 
 
+@pytest.mark.parametrize("n,keys,value,mixed", [
+    (97, (0, 32), "-inf", 0), (200, (32, 64), "-inf", 0), (200, (96, 200), "-inf", 0), (300, (0, 299), "-inf", 0),
+    (33, (0, 33), "-inf", 0),                                   # every key: no weights, NaN
+    (200, (64, 96), "inf", 0), (200, (40, 41), "nan", 0), (130, (0, 128), "-inf", 1),
+    (2048, (0, 64), "-inf", 0), (2049, (64, 2048), "-inf", 0), (2048, (0, 2048), "-inf", 0), (2048, (70, 71), "nan", 0),
+    (2048, (0, 1000), "-inf", 1)])
+def test_attention_infinite_scores(gpu, n, keys, value, mixed):
+    """Scores of -inf (whole key tiles of them, first, last and all of a wave's), +inf and NaN, in both workgroup
+    forms: every row as the float64 softmax has it, weight 0 for -inf, NaN where that is NaN. mixed: the
+    even rows' queries turn the keys' -inf into +inf (NaN rows between finite ones)."""
+    from torch_xdna import kernels
+
+    nh, nkv = 16, 8
+    g = torch.Generator().manual_seed(n + keys[0])
+    q = torch.randn(n, nh, 128, generator=g).to(torch.bfloat16)
+    k = torch.randn(n, nkv, 128, generator=g).to(torch.bfloat16)
+    v = torch.randn(n, nkv, 128, generator=g).to(torch.bfloat16)
+    q[:, :, 0] = 1.0                                            # times -inf: -inf
+    if mixed:
+        q[::2, :, 0] = -1.0
+    k[:, :, 0] = 0.0
+    k[keys[0]:keys[1], :, 0] = float(value)
+    vt = torch.zeros(nkv, 128, -(-n // 32) * 32, dtype=torch.bfloat16)
+    vt[:, :, :n] = v.permute(1, 2, 0)
+    i32 = dict(dtype=torch.int32, device=gpu)
+    out = kernels.attention_bf16(q.to(gpu), k.to(gpu), vt.to(gpu), torch.tensor([0], **i32), torch.tensor([n], **i32),
+                                 torch.tensor([0], **i32), n, 128 ** -0.5).cpu().double()
+    for h in range(nh):
+        p = torch.softmax(q[:, h].double() @ k[:, h // 2].double().t() * 128 ** -0.5, dim=-1)
+        want, got = p @ v[:, h // 2].double(), out[:, h]
+        nan = want.isnan()
+        assert torch.equal(got.isnan(), nan), h
+        if not nan.all():       # the tolerance of test_attention_bf16_forms
+            assert rel_err(got[~nan], want[~nan]) < 1e-2, h
+
+
 def test_silu_mul_and_add(gpu):
     from torch_xdna import kernels
 

@@ -400,7 +400,7 @@ __global__ __launch_bounds__(QW* KW * 64, 2) void attention_kernel(
       for (int db = 0; db < 4; ++db) o[db] *= alpha;
       m = mn;
     }
-    const float mc = m * c;
+    const float mc = m == -INFINITY ? 0.0f : m * c;   // only -inf (or NaN) scores so far: p = 2^-inf = 0, not NaN
     i32x4 pf[2 * NB];
     float ps[2] = {0.0f, 0.0f};
 #pragma unroll
