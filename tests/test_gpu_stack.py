@@ -239,6 +239,35 @@ def test_attention_bf16_forms(gpu, nh, nkv, scale, lens):
             assert rel_err(out[s0:s0 + n, h], p @ v[s0:s0 + n, kv].double()) < 1e-2, (n, h)
 
 
+@pytest.mark.parametrize("n", [1536, 1999])
+def test_attention_bf16_weights(gpu, n):
+    """The 128-row form rounds its weights to bf16 against a maximum that follows every 32 keys: the output is that of the
+    same online softmax in float64, rounded to bf16. What is left is the weights and outputs that float32 puts on the
+    other side of a bf16 rounding boundary, 2^-14 of them for errors of 2^-24 of arguments up to 10 and steps of 2^-9, each
+    2^-8 of itself: some 1e-4 in relative norm (a maximum per 64 keys is 1.1e-3 away)."""
+    from torch_xdna import kernels
+
+    nh, nkv, scale = 16, 8, 128 ** -0.5
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(n, h, 128, generator=g).to(torch.bfloat16) for h in (nh, nkv, nkv))
+    vt = torch.zeros(nkv, 128, -(-n // 32) * 32, dtype=torch.bfloat16)
+    vt[:, :, :n] = v.permute(1, 2, 0)
+    i32 = dict(dtype=torch.int32, device=gpu)
+    out = kernels.attention_bf16(q.to(gpu), k.to(gpu), vt.to(gpu), torch.tensor([0], **i32), torch.tensor([n], **i32),
+                                 torch.tensor([0], **i32), n, scale).cpu().double()
+    for h in (0, 5, 15):
+        s = q[:, h].double() @ k[:, h // 2].double().t() * scale
+        m = torch.full((n, 1), -float("inf"), dtype=torch.float64)
+        l, o = torch.zeros(n, 1, dtype=torch.float64), torch.zeros(n, 128, dtype=torch.float64)
+        for b in range(0, n, 32):
+            mn = torch.maximum(m, s[:, b:b + 32].amax(1, keepdim=True))
+            p = torch.exp(s[:, b:b + 32] - mn)
+            l = l * torch.exp(m - mn) + p.sum(1, keepdim=True)
+            o = o * torch.exp(m - mn) + p.to(torch.bfloat16).double() @ v[b:b + 32, h // 2].double()
+            m = mn
+        assert rel_err(out[:, h], (o / l).to(torch.bfloat16).double()) < 4e-4, h
+
+
 @pytest.mark.parametrize("n,keys,value,mixed", [
     (97, (0, 32), "-inf", 0), (200, (32, 64), "-inf", 0), (200, (96, 200), "-inf", 0), (300, (0, 299), "-inf", 0),
     (33, (0, 33), "-inf", 0),                                   # every key: no weights, NaN

@@ -229,18 +229,20 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const float* __restri
 // 8 u .. 8 u + 7 exactly those of step u, so P goes from one product to the next without leaving its lane.
 // LDS chunks of 16 bytes are XORed with the row so that the 16 lanes of a fragment read's phase cover the banks.
 //
-// Softmax: p = 2^(c (s - m)), c = scale * log2(e) > 0 (a negative scale goes into Q's sign), in float32; O and l
-// are rescaled only in the tiles where some row's running maximum m grows; P is rounded to bf16 for the second
-// product, l sums the unrounded p. (Letting m lag by up to 2^8 skips more of the rescales and runs 4% faster, but
-// the rounding of P then errs by 5% more against 64 bits: not done.)
+// Softmax: p = 2^(c (s - m)), c = scale * log2e > 0 (a negative scale goes into Q's sign), in float32; O and l
+// are rescaled only in the blocks of 32 keys where some row's running maximum m grows; P is rounded to bf16 for the
+// second product, l sums the unrounded p. The maximum follows every 32 keys also where a tile holds 64, and never lags:
+// a key that is the maximum has p = 1, which rounds to itself, so the coarser m follows, the further the result is off
+// (4096 / 1500 / 700 against 64 bits: 2.237e-3, 2.241e-3 with one maximum per 64 keys, which ran 2 to 5% faster;
+// m lagging by up to 2^8: 5% further off and 4% faster; neither is done).
 //
 // What bounds it: per 64 keys and 32 rows a wave issues 32 MFMAs (1024 cycles of its SIMD) and about 400 vector
 // instructions of softmax, so two waves per SIMD (two workgroups per CU, 64 KB of LDS each) fill each other's
 // gaps; with the registers for one wave per SIMD only (no spills either way) the long shapes run 1.5x slower.
-// Measured, 16 q and 8 kv heads: 1 x 4096 queries 189 us (727 TFLOP/s), 4 x 4096 706 us; lengths 4096 / 1500 / 700
-// in one call 206 us against 557 us for one wave per 32 queries of a q head reading its K and V fragments straight
-// from memory, 264 / 222 (the split form) 9.1 against 18.7 us. MFMA issue has priority over the other wave's
-// softmax (s_setprio): 4% on the long shapes.
+// Measured, 16 q and 8 kv heads: 1 x 4096 queries 177 us (777 TFLOP/s), 4 x 4096 679 us; lengths 4096 / 1500 / 700
+// in one call 215 us against 556 us for one wave per 32 queries of a q head reading its K and V fragments straight
+// from memory, 264 / 222 (the split form) 8.7 against 18.7 us. MFMA issue has priority over the other wave's
+// softmax (s_setprio): 2% on the long shapes.
 __device__ __forceinline__ int swap23(int i) { return (i & ~12) | ((i & 4) << 1) | ((i & 8) >> 1); }
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
@@ -361,74 +363,66 @@ __global__ __launch_bounds__(QW* KW * 64, 2) void attention_kernel(
       __builtin_amdgcn_sched_barrier(0);
     }
     if (KW > 1 && kb >= n) continue;       // uniform over the group; the last tile at the earliest
-    f32x16s sc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) sc[b] = f32x16s{};
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-        sc[b] = mfma_bf16(*reinterpret_cast<const i32x4*>(cur + b * 8192 + krd + (((2 * s + half) ^ kx) << 4)), qf[s], sc[b]);
-    if constexpr (ST == 1) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      if (kn < n) load_k(kn, cur);
-    }
-    __builtin_amdgcn_s_setprio(0);
     const bool part = kb + KT > n;         // uniform
-    float mx = -INFINITY;
-    if (part) {
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          if (kb + 32 * b + 16 * (e >> 3) + 8 * half + (e & 7) >= n) sc[b][e] = -INFINITY;
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-      for (int e = 0; e < 16; e += 2)
-        mx = __builtin_elementwise_maximum(mx, __builtin_elementwise_maximum(sc[b][e], sc[b][e + 1]));
-    mx = half_max(mx);
-    const bool grow = mx > m;
-    if (__builtin_amdgcn_ballot_w64(grow)) {
-      const float mn = grow ? mx : m;
-      const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - mn) * c);
-      l *= alpha;
-#pragma unroll
-      for (int db = 0; db < 4; ++db) o[db] *= alpha;
-      m = mn;
-    }
-    const float mc = m == -INFINITY ? 0.0f : m * c;   // only -inf (or NaN) scores so far: p = 2^-inf = 0, not NaN
-    i32x4 pf[2 * NB];
-    float ps[2] = {0.0f, 0.0f};
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      float p[16];
+      f32x16s sc = f32x16s{};
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        sc = mfma_bf16(*reinterpret_cast<const i32x4*>(cur + b * 8192 + krd + (((2 * s + half) ^ kx) << 4)), qf[s], sc);
+      if constexpr (ST == 1) {
+        static_assert(ST == 2 || NB == 1, "a single stage holds one block of keys");
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        if (kn < n) load_k(kn, cur);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      float mx = -INFINITY;
+      if (part) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (kb + 32 * b + 16 * (e >> 3) + 8 * half + (e & 7) >= n) sc[e] = -INFINITY;
+      }
+#pragma unroll
+      for (int e = 0; e < 16; e += 2)
+        mx = __builtin_elementwise_maximum(mx, __builtin_elementwise_maximum(sc[e], sc[e + 1]));
+      mx = half_max(mx);
+      const bool grow = mx > m;
+      if (__builtin_amdgcn_ballot_w64(grow)) {
+        const float mn = grow ? mx : m;
+        const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - mn) * c);
+        l *= alpha;
+#pragma unroll
+        for (int db = 0; db < 4; ++db) o[db] *= alpha;
+        m = mn;
+      }
+      const float mc = m == -INFINITY ? 0.0f : m * c;   // only -inf (or NaN) scores so far: p = 2^-inf = 0, not NaN
+      i32x4 pf[2];
+      float p[16], ps[2] = {0.0f, 0.0f};
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[b][e], c, -mc));
+        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[e], c, -mc));
         if (part && kb + 32 * b + 16 * (e >> 3) + 8 * half + (e & 7) >= n) p[e] = 0.0f;
       }
 #pragma unroll
       for (int e = 0; e < 16; e += 2) {
         ps[0] += p[e];
         ps[1] += p[e + 1];
-        pf[2 * b + (e >> 3)][(e & 7) >> 1] = (int)f32x2_to_bf16x2_bits(p[e], p[e + 1]);
+        pf[e >> 3][(e & 7) >> 1] = (int)f32x2_to_bf16x2_bits(p[e], p[e + 1]);
       }
+      l += ps[0] + ps[1];
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int db = 0; db < 4; ++db) {
+          i32x4 vf = *reinterpret_cast<const i32x4*>(cur + KB + (db * 32 + row) * (2 * KT) + (((4 * b + 2 * u + half) ^ vx) << 4));
+          if (part && kb + 32 * b + 16 * u + 8 * half >= n) vf = i32x4{0, 0, 0, 0};
+          o[db] = mfma_bf16(vf, pf[u], o[db]);
+        }
+      __builtin_amdgcn_s_setprio(0);
     }
-    l += ps[0] + ps[1];
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int u = 0; u < 2 * NB; ++u)
-#pragma unroll
-      for (int db = 0; db < 4; ++db) {
-        i32x4 vf = *reinterpret_cast<const i32x4*>(cur + KB + (db * 32 + row) * (2 * KT) + (((2 * u + half) ^ vx) << 4));
-        if (part && kb + 16 * u + 8 * half >= n) vf = i32x4{0, 0, 0, 0};
-        o[db] = mfma_bf16(vf, pf[u], o[db]);
-      }
-    __builtin_amdgcn_s_setprio(0);
     if constexpr (ST == 1) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
@@ -577,8 +571,11 @@ int xdna_attention_bf16(const void* q, const void* k, const void* vt, int64_t ld
   const uint32_t qsign = scale < 0.0f ? 0x80008000u : 0u;
   // 128 rows per workgroup, sharing each key tile, once such workgroups cover three quarters of the CUs; below that
   // 32 rows with the keys split over four waves, which quarters the chain of tiles a wave walks. Measured, 16 / 8
-  // heads, wide against split: one sequence of 512 20.4 / 10.8 us, 1024 36.6 / 23.5, 1300 (168 wide workgroups)
-  // 47.6 / 44.8, 1500 (192) 53.9 / 53.3, 1800 64.9 / 66.5, 3000 133 / 159; four of 500 (256) 23.4 / 28.2
+  // heads, wide against split: one sequence of 512 20.9 / 10.5 us, 1024 36.7 / 22.3, 1300 (168 wide workgroups)
+  // 46.6 / 42.2, 1500 (192) 52.2 / 46.6, 1800 62.3 / 61.5, 2048 67.9 / 70.1, 3000 124 / 142; several: eight of 190 (192)
+  // 12.0 / 15.7, four of 390 (224) 19.9 / 23.2, four of 500 (256) 22.6 / 26.0. The lengths lie on the GPU, so the
+  // workgroups counted are those of nseq sequences of the longest length: 700 / 20 / 20 / 20 takes the wide
+  // form, 27.6 / 17.5
   const bool wide = 4 * nseq * cdiv(max_len * grp, 128) * nkv >= 3 * (int64_t)device_cus();
   const int64_t qblocks = cdiv(max_len * grp, wide ? 128 : 32);
   XDNA_REQUIRE(qblocks * nkv < (1ll << 31), "sequence too long");
