@@ -239,6 +239,14 @@ def test_attention_bf16_forms(gpu, nh, nkv, scale, lens):
             assert rel_err(out[s0:s0 + n, h], p @ v[s0:s0 + n, kv].double()) < 1e-2, (n, h)
 
 
+@pytest.mark.parametrize("nh,nkv,lens", [(16, 8, [1]), (16, 8, [32, 5, 31]), (6, 1, [17, 32]), (16, 8, [20] * 40), (16, 8, [33]),
+                                         (16, 8, [64, 1, 32, 63]), (3, 3, [50] * 9), (6, 1, [64, 33]), (16, 8, [65, 20])])
+def test_attention_short_sequences(gpu, nh, nkv, lens):
+    """The forms of one wave (a longest sequence of up to 32 tokens), two (64) and four per row block, at their
+    edges: as test_attention_bf16_forms."""
+    test_attention_bf16_forms(gpu, nh, nkv, 128 ** -0.5, lens)
+
+
 @pytest.mark.parametrize("n", [1536, 1999])
 def test_attention_bf16_weights(gpu, n):
     """The 128-row form rounds its weights to bf16 against a maximum that follows every 32 keys: the output is that of the

@@ -576,7 +576,10 @@ int xdna_attention_bf16(const void* q, const void* k, const void* vt, int64_t ld
   // 12.0 / 15.7, four of 390 (224) 19.9 / 23.2, four of 500 (256) 22.6 / 26.0. The lengths lie on the GPU, so the
   // workgroups counted are those of nseq sequences of the longest length: 700 / 20 / 20 / 20 takes the wide
   // form, 27.6 / 17.5
-  const bool wide = 4 * nseq * cdiv(max_len * grp, 128) * nkv >= 3 * (int64_t)device_cus();
+  // A wave per 32 keys at the most: sequences of up to 64 take two waves, of up to 32 one, which needs no combination
+  // at the end (and no wide form: 64 sequences of 20 6.8 / 7.5 us). One wave / two / four: 20 tokens 4.2 / 4.9 / 5.6 us,
+  // 64 tokens 5.2 / 5.0 / 5.7, sixteen of 50 6.8 / 6.6 / 7.9, 97 tokens 7.5 / 6.2 / 5.9
+  const bool wide = max_len > 32 && 4 * nseq * cdiv(max_len * grp, 128) * nkv >= 3 * (int64_t)device_cus();
   const int64_t qblocks = cdiv(max_len * grp, wide ? 128 : 32);
   XDNA_REQUIRE(qblocks * nkv < (1ll << 31), "sequence too long");
   const int64_t step = ((1ll << 31) - 1) / (qblocks * nkv);   // sequences per launch
@@ -585,12 +588,14 @@ int xdna_attention_bf16(const void* q, const void* k, const void* vt, int64_t ld
     const uint16_t *qp = static_cast<const uint16_t*>(q), *kp = static_cast<const uint16_t*>(k),
                    *vp = static_cast<const uint16_t*>(vt);
     uint16_t* op = static_cast<uint16_t*>(out);
-    if (wide)
-      attention_kernel<4, 1, 64, 2><<<g, 256, 0, as_stream(stream)>>>(qp, kp, vp, ld_vt, seq_start + s0, seq_len + s0,
-                                                                       seq_vt + s0, (int)qblocks, nh, nkv, c, qsign, op);
-    else
-      attention_kernel<1, 4, 32, 1><<<g, 256, 0, as_stream(stream)>>>(qp, kp, vp, ld_vt, seq_start + s0, seq_len + s0,
-                                                                       seq_vt + s0, (int)qblocks, nh, nkv, c, qsign, op);
+#define XDNA_ATT(QW_, KW_, KT_, ST_)                                                                              \
+  attention_kernel<QW_, KW_, KT_, ST_><<<g, QW_ * KW_ * 64, 0, as_stream(stream)>>>(                              \
+      qp, kp, vp, ld_vt, seq_start + s0, seq_len + s0, seq_vt + s0, (int)qblocks, nh, nkv, c, qsign, op)
+    if (wide) XDNA_ATT(4, 1, 64, 2);
+    else if (max_len <= 32) XDNA_ATT(1, 1, 32, 1);
+    else if (max_len <= 64) XDNA_ATT(1, 2, 32, 1);
+    else XDNA_ATT(1, 4, 32, 1);
+#undef XDNA_ATT
   }
   return launch_status("attention_bf16");
 }
