@@ -312,6 +312,40 @@ def test_attention_infinite_scores(gpu, n, keys, value, mixed):
             assert rel_err(got[~nan], want[~nan]) < 1e-2, h
 
 
+def test_more_workgroups_than_a_launch(gpu):
+    """Calls whose workgroups are more than one launch takes (2^24 of 256 threads): 2^21 + 3 short sequences of 8 kv
+    heads, and 2^24 + 40 tokens of one head; what the last launch does is that of a call of its own."""
+    from torch_xdna import kernels
+
+    g = torch.Generator().manual_seed(2)
+    rand = lambda *s: torch.randn(*s, generator=g)
+    i32 = dict(dtype=torch.int32, device=gpu)
+    q, k = (rand(40, 8, 128).to(torch.bfloat16).to(gpu) for _ in range(2))
+    vt = rand(8, 128, 64).to(torch.bfloat16).to(gpu)
+    nseq = 2 ** 21 + 3
+    start, length = torch.zeros(nseq, **i32), torch.ones(nseq, **i32)
+    start[-2:], length[-2:] = torch.tensor([1, 3], **i32), torch.tensor([2, 37], **i32)
+    col = torch.zeros(nseq, **i32)
+    col[-1] = 8
+    out = kernels.attention_bf16(q, k, vt, start, length, col, 40, 128 ** -0.5)
+    want = kernels.attention_bf16(q, k, vt, start[-3:].contiguous(), length[-3:].contiguous(), col[-3:].contiguous(), 40,
+                                  128 ** -0.5)
+    assert rel_err(out.double().cpu(), want.double().cpu()) < 1e-2     # the two forms: as test_attention_bf16_forms
+
+    T = 2 ** 24 + 40
+    qkv = torch.zeros(T, 3 * 128, device=gpu)
+    qkv[-64:] = rand(64, 3 * 128).to(gpu)
+    w, freq = (1 + 0.1 * rand(128)).to(gpu), (1.0 / (1e6 ** (torch.arange(0, 128, 2) / 128))).to(gpu)
+    pos, col = torch.zeros(T, **i32), torch.zeros(T, **i32)
+    pos[-64:], col[-64:] = torch.arange(64, **i32), torch.arange(64, **i32)
+    qkv[:-64, 256:] = qkv[-64, 256:]                                   # all other tokens' V go to column 0 too
+    vt = torch.zeros(1, 128, 64, dtype=torch.bfloat16, device=gpu)
+    got = kernels.qk_norm_rope(qkv, 1, 1, w, w, freq, pos, col, 1e-6, vt)
+    vt2 = torch.zeros_like(vt)
+    want = kernels.qk_norm_rope(qkv[-64:], 1, 1, w, w, freq, pos[-64:], col[-64:], 1e-6, vt2)
+    assert torch.equal(got[0][-64:], want[0]) and torch.equal(got[1][-64:], want[1]) and torch.equal(vt, vt2)
+
+
 def test_silu_mul_and_add(gpu):
     from torch_xdna import kernels
 

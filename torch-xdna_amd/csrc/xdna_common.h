@@ -24,6 +24,8 @@ void set_error(const std::string& msg);
 
 // Status of the launches just made on this thread (hipGetLastError), as an ABI status.
 int launch_status(const char* where);
+// Threads of a launch along x that HIP takes (blocks times threads per block, a 32-bit count).
+constexpr int64_t MAX_LAUNCH_THREADS = (1ll << 32) - 1;
 // Compute units of the current device (cached per device).
 int device_cus();
 

@@ -541,20 +541,24 @@ int xdna_qk_norm_rope(const float* qkv, int64_t T, int nh, int nkv, const void* 
   XDNA_REQUIRE(T >= 0 && nh >= 1 && nkv >= 1 && nh % nkv == 0, "bad head counts");
   if (T == 0) return XDNA_OK;
   XDNA_REQUIRE(qkv && q_w && k_w && inv_freq && pos && vt_col && q && k && vt && ld_vt >= 1, "bad arguments");
-  const int64_t vblocks = cdiv(T, V_TOK) * nkv;
-  XDNA_REQUIRE(vblocks + T < (1ll << 31), "too many tokens");
+  // tokens of a launch: a workgroup each and nkv per V_TOK of them
+  const int64_t most = MAX_LAUNCH_THREADS / 256 / (V_TOK + nkv) * V_TOK;
+  XDNA_REQUIRE(most > 0, "too many kv heads");
   hipStream_t st = as_stream(stream);
-  dim3 g((unsigned)(vblocks + T));
-  uint16_t *qb = static_cast<uint16_t*>(q), *kb = static_cast<uint16_t*>(k), *vb = static_cast<uint16_t*>(vt);
-  if (w_dtype == XDNA_F32)
-    qk_norm_rope_kernel<XDNA_F32><<<g, 256, 0, st>>>(qkv, T, nh, nkv, q_w, k_w, inv_freq, pos, vt_col, eps, qb, kb, vb, ld_vt,
-                                                       vblocks);
-  else if (w_dtype == XDNA_BF16)
-    qk_norm_rope_kernel<XDNA_BF16><<<g, 256, 0, st>>>(qkv, T, nh, nkv, q_w, k_w, inv_freq, pos, vt_col, eps, qb, kb, vb, ld_vt,
-                                                       vblocks);
-  else
-    qk_norm_rope_kernel<XDNA_F16><<<g, 256, 0, st>>>(qkv, T, nh, nkv, q_w, k_w, inv_freq, pos, vt_col, eps, qb, kb, vb, ld_vt,
-                                                       vblocks);
+  for (int64_t t0 = 0; t0 < T; t0 += most) {
+    const int64_t n = std::min(most, T - t0), vblocks = cdiv(n, V_TOK) * nkv;
+    const dim3 g((unsigned)(vblocks + n));
+    const float* x = qkv + t0 * (nh + 2 * (int64_t)nkv) * 128;
+    uint16_t *qb = static_cast<uint16_t*>(q) + t0 * nh * 128, *kb = static_cast<uint16_t*>(k) + t0 * nkv * 128,
+             *vb = static_cast<uint16_t*>(vt);
+#define XDNA_QKR(DT)                                                                                              \
+  qk_norm_rope_kernel<DT><<<g, 256, 0, st>>>(x, n, nh, nkv, q_w, k_w, inv_freq, pos + t0, vt_col + t0, eps, qb, kb, vb, \
+                                             ld_vt, vblocks)
+    if (w_dtype == XDNA_F32) XDNA_QKR(XDNA_F32);
+    else if (w_dtype == XDNA_BF16) XDNA_QKR(XDNA_BF16);
+    else XDNA_QKR(XDNA_F16);
+#undef XDNA_QKR
+  }
   return launch_status("qk_norm_rope");
 }
 
@@ -581,8 +585,9 @@ int xdna_attention_bf16(const void* q, const void* k, const void* vt, int64_t ld
   // 64 tokens 5.2 / 5.0 / 5.7, sixteen of 50 6.8 / 6.6 / 7.9, 97 tokens 7.5 / 6.2 / 5.9
   const bool wide = max_len > 32 && 4 * nseq * cdiv(max_len * grp, 128) * nkv >= 3 * (int64_t)device_cus();
   const int64_t qblocks = cdiv(max_len * grp, wide ? 128 : 32);
-  XDNA_REQUIRE(qblocks * nkv < (1ll << 31), "sequence too long");
-  const int64_t step = ((1ll << 31) - 1) / (qblocks * nkv);   // sequences per launch
+  const int64_t threads = wide || max_len > 64 ? 256 : max_len > 32 ? 128 : 64;
+  const int64_t step = MAX_LAUNCH_THREADS / threads / (qblocks * nkv);   // sequences per launch
+  XDNA_REQUIRE(step > 0, "sequence too long");
   for (int64_t s0 = 0; s0 < nseq; s0 += step) {
     const dim3 g((unsigned)(std::min(step, nseq - s0) * qblocks * nkv));
     const uint16_t *qp = static_cast<const uint16_t*>(q), *kp = static_cast<const uint16_t*>(k),
