@@ -369,3 +369,40 @@ def test_direct_route_is_taken(gpu, monkeypatch):
     torch.ops.xdna.linear(*args)
     torch.ops.xdna.linear(args[0].clone().requires_grad_(), *args[1:])
     assert wrapped == [False, True]
+
+
+def test_direct_route_registered_kernels(gpu):
+    """A kernel that a program registers for an op on GPUs is what plain calls reach: through register_kernel, switched
+    off and on with set_kernel_enabled, and through torch.library's impl for the CUDA and the AutogradCUDA key."""
+    from torch_xdna import ops
+
+    @torch.library.custom_op("xdna_test::twice", mutates_args=())
+    def twice(x: torch.Tensor) -> torch.Tensor:
+        return x * 2
+
+    @torch.library.custom_op("xdna_test::thrice", mutates_args=())
+    def thrice(x: torch.Tensor) -> torch.Tensor:
+        return x * 3
+
+    lib = torch.library.Library("xdna_test", "FRAGMENT")
+    direct = []
+    for op, f in ((twice, 2), (thrice, 3)):
+        ops._direct(op, lambda x, f=f: (direct.append(f), x * f)[1], lib)
+    x = torch.randn(8, device=gpu)
+    with torch.no_grad():
+        assert torch.equal(twice(x), x * 2) and torch.equal(thrice(x), x * 3) and direct == [2, 3]
+        for key in ("CUDA", "AutogradCUDA"):
+            with torch.library._scoped_library("xdna_test", "IMPL") as mine:
+                mine.impl("thrice", lambda x: x * 5, key)
+                assert torch.equal(thrice(x), x * 5), key
+            assert torch.equal(thrice(x), x * 3), key
+        assert direct == [2, 3, 3, 3]
+        thrice.register_kernel(None)(lambda x: x * 11)
+        assert torch.equal(thrice(x), x * 11)
+        twice.register_kernel("cuda")(lambda x: x * 7)
+        assert torch.equal(twice(x), x * 7)
+        with twice.set_kernel_enabled("cuda", False):
+            assert torch.equal(twice(x), x * 2)
+        assert torch.equal(twice(x), x * 7) and direct == [2, 3, 3, 3]
+    for name in ("linear", "linear_cat", "conv3x3_fused", "conv3x3_chain", "qwen3_stack"):
+        assert f"xdna/{name}/CUDA" not in torch.library._impls and f"xdna/{name}/Autograd" in torch.library._impls

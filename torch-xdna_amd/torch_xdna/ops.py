@@ -16,7 +16,7 @@ import torch._dynamo
 
 from . import conv, runtime, stack
 
-try:    # what custom_op registers for autograd (below); without it the ops keep only custom_op's own route
+try:    # what custom_op registers for autograd (below)
     from torch._library.autograd import make_autograd_impl as _make_autograd_impl
 except ImportError:
     _make_autograd_impl = None
@@ -138,7 +138,10 @@ def _(x, mask, stack_id, cfg_id):
 # Python, 9 us a call, as much as a small op's launches. A call whose tensors are ordinary GPU tensors, none of which
 # needs a gradient, has nothing to do there: the function is called at once. Anything else goes on as before: the
 # test is the dispatcher's own key set of the call, so a dispatch mode (fake tensors, tracing), a negated view, a
-# functional wrapper or any other layer that stands below autograd shows in it.
+# functional wrapper or any other layer that stands below autograd shows in it, and so does
+# inference mode, which has no autograd keys at all. A kernel that a program has registered for the op on GPUs
+# (register_kernel, or torch.library's impl for the CUDA key) is what its calls reach, by the
+# generic route, which also knows whether it is switched off (set_kernel_enabled).
 _PLAIN = (torch._C.DispatchKeySet(torch._C.DispatchKey.CUDA)
           | torch._C.DispatchKeySet(torch._C.DispatchKey.AutogradCUDA)).raw_repr()
 
@@ -153,24 +156,31 @@ def _needs_grad(args):
     return False
 
 
-def _direct(custom, fn):
-    """Registers fn (the op's arguments -> its result) for plain GPU calls of the custom op."""
+def _direct(custom, fn, lib):
+    """Registers fn (the op's arguments -> its result) in lib for plain GPU calls of the custom op."""
+    op = custom._opoverload.name().replace("::", "/")
+    registered = getattr(torch.library, "_impls", ())      # "namespace/op/key" of every kernel registered from Python
+    if _make_autograd_impl is None or not hasattr(custom, "_backend_fns") or f"{op}/Autograd" not in registered:
+        return                                              # another torch: the ops keep only custom_op's own route
     generic = _make_autograd_impl(custom._opoverload, custom)
+    default, on_gpu = custom._backend_fns.get(None), f"{op}/CUDA"
 
     def call(keyset, *args):
-        if keyset.raw_repr() != _PLAIN or (torch.is_grad_enabled() and _needs_grad(args)):
+        if (keyset.raw_repr() != _PLAIN or on_gpu in torch.library._impls or custom._backend_fns.get(None) is not default
+                or (torch.is_grad_enabled() and _needs_grad(args))):
             return generic(keyset, *args)
         return fn(*args)
 
     # as custom_op does for its functions: Dynamo never traces into the call
-    _lib.impl(custom._opoverload.name().split("::")[1], torch._dynamo.disable(call), "AutogradCUDA", with_keyset=True)
+    lib.impl(op.split("/")[1], torch._dynamo.disable(call), "AutogradCUDA", with_keyset=True)
+    torch.library._impls.discard(f"{op}/AutogradCUDA")      # the key stays free for a registration of the program's own
 
 
-if _make_autograd_impl is not None and hasattr(linear, "_opoverload"):
+if hasattr(linear, "_opoverload"):
     _lib = torch.library.Library("xdna", "FRAGMENT")
-    _direct(linear, lambda x, w, b, transposed, cid: runtime.linear(_configs[cid], x, w, b, transposed))
-    _direct(linear_cat, lambda x, ws, bs, cid: runtime.linear_cat(_configs[cid], x, ws, bs))
-    _direct(conv3x3_fused, lambda x, w, b, relu, cid: conv.conv3x3_fused(_configs[cid], x, w, b, relu))
+    _direct(linear, lambda x, w, b, transposed, cid: runtime.linear(_configs[cid], x, w, b, transposed), _lib)
+    _direct(linear_cat, lambda x, ws, bs, cid: runtime.linear_cat(_configs[cid], x, ws, bs), _lib)
+    _direct(conv3x3_fused, lambda x, w, b, relu, cid: conv.conv3x3_fused(_configs[cid], x, w, b, relu), _lib)
     _direct(conv3x3_chain, lambda x, ws, bs, relus, after, pools, cid: conv.conv3x3_chain(
-        _configs[cid], cid, x, list(ws), list(bs), list(relus), list(after), list(pools)))
-    _direct(qwen3_stack, lambda x, mask, sid, cid: stack.run(_configs[cid], sid, x, mask))
+        _configs[cid], cid, x, list(ws), list(bs), list(relus), list(after), list(pools)), _lib)
+    _direct(qwen3_stack, lambda x, mask, sid, cid: stack.run(_configs[cid], sid, x, mask), _lib)
