@@ -953,6 +953,26 @@ def test_bias_dtypes(gpu, dtype, tile_table):
             assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), (n, ci, co, pool)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_conv_dequant_bias_dtypes(gpu, dtype):
+    """The separate dequantize takes the biases that the fused conv takes: 16-bit ones as their float32 copies, equal to
+    the conv with its dequantize; a float64 one is refused by both."""
+    from torch_xdna import kernels as k
+
+    x, wt = _conv_case(2, 20, 48, 5, 7, seed=3)
+    xq, sx = k.conv_quant(x.to(gpu), 32)
+    wq, sw = k.conv_weight_pack(wt.to(gpu), 32)
+    b = _rand((48,), DT[dtype], seed=4).to(gpu)
+    q = k.conv3x3(xq, wq, 9, False)
+    y = k.conv_dequant(q, False, sw, sx, b, DT[dtype])
+    assert torch.equal(y, k.conv_dequant(q, False, sw, sx, b.float(), DT[dtype]))
+    assert torch.equal(y, k.conv3x3_dequant(xq, wq, 9, False, sw, sx, b, DT[dtype]))
+    for call in (lambda: k.conv_dequant(q, False, sw, sx, b.double(), DT[dtype]),
+                 lambda: k.conv3x3_dequant(xq, wq, 9, False, sw, sx, b.double(), DT[dtype])):
+        with pytest.raises(TypeError, match="biases"):
+            call()
+
+
 def _ksplit(cus, bm, bn, kg, tiles, k):
     """Workgroups per tile along K that the library gives a launch: 1 above 64 x 64 or when the tiles fill
     more than half of the CUs, else up to CUs / tiles, at most 16, with at least 16 slices of 64 per K

@@ -176,7 +176,11 @@ def gpu_bias(bias, dev):
 
 
 def _bias_code(bias):
-    return F32 if bias is None else _DTYPE_CODE[bias.dtype]
+    if bias is None:
+        return F32
+    if bias.dtype not in _DTYPE_CODE:
+        raise TypeError(f"xdna launchers take float32/bfloat16/float16 biases, got {bias.dtype}")
+    return _DTYPE_CODE[bias.dtype]
 
 
 def _stream(dev):
@@ -638,6 +642,9 @@ def conv3x3_calibrate(xq, wq, relu):
 def conv_dequant(q, relu, scale, sx, bias, out_dtype):
     """NHWC q [N, H, W, Co] -> NCHW y = q * (scale[co] * sx[n]) (+ bias[co]) as out_dtype."""
     dev = _need_gpu(q, scale, sx, bias)
+    if bias is not None and bias.dtype != torch.float32:
+        _bias_code(bias)            # a dtype the other biased launchers take; this entry point's bias is float32
+        bias = bias.float()
     n, h, w, co = q.shape
     y = torch.empty((n, co, h, w), dtype=out_dtype, device=dev)
     if n:
