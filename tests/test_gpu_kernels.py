@@ -1052,6 +1052,34 @@ def test_gemm_ksplit(gpu, tile, tile_table):
         assert int(buf[:65536].view(torch.int32).abs().sum()) == 0, "arrival counters not back to zero"
 
 
+@pytest.mark.parametrize("tile", sorted(KSPLIT_TILES))
+@pytest.mark.parametrize("k", [10256, 14352, 4096, 3088])
+def test_gemm_ksplit_parts(gpu, tile, k, tile_table):
+    """Every part of a K split has slices to sum, also where the tile's slices are 128 bytes long and do not go evenly
+    into the parts: the partial sums that the workgroups leave in the workspace are those of K ranges that
+    follow each other, none empty, and add up to the product."""
+    from torch_xdna import kernels
+
+    bm, bn, kg = KSPLIT_TILES[tile]
+    m, n = bm, bn                                                  # one tile
+    ks = _ksplit(kernels.num_cus(gpu), bm, bn, kg, 1, k)
+    kernels.tile_set("i8", m, n, k, tile)
+    a, w = _i8((m, k), seed=k).to(gpu), _i8((n, k), seed=k + 1).to(gpu)
+    need = kernels.lib().xdna_gemm_ws_bytes(m, n, k)
+    ws = torch.zeros(need, dtype=torch.uint8, device=gpu)
+    c = torch.empty(m, n, dtype=torch.int32, device=gpu)
+    p = kernels._ptr
+    kernels._check(kernels.lib().xdna_gemm_i8_i32_ws(p(a), k, p(w), k, p(c), n, m, n, k, p(ws), need,
+                                                     kernels._stream(gpu)), "gemm")
+    assert torch.equal(c, (a.double() @ w.double().t()).to(torch.int32))
+    if ks == 1:
+        return
+    waves = {"t64x32": 2, "t64x64": 4, "t64x64k2": 4, "t64x64k4": 4, "t32x64": 2, "t32x64k4": 2}.get(tile, 1)
+    part = ws[65536:65536 + m * n * 4 * ks].view(torch.int32).view(waves, ks, -1)
+    assert torch.equal(part.sum(1).flatten().sort().values, c.flatten().sort().values)
+    assert bool((part != 0).any(-1).all()), "a part without slices"
+
+
 @pytest.mark.parametrize("tile", ["t256x256w8", "t128x256w8"])
 def test_conv_halo(gpu, tile, tile_table):
     """The conv from a haloed input tile (the 8-wave 256 x 256 and 128 x 256 tiles when a tile is whole image

@@ -714,9 +714,10 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
   int64_t kbase = 0, nk = nk_all;
   if constexpr (CAN_SPLIT) {
     if (e.ksplit > 1) {
-      const int64_t per = (nk_all + e.ksplit - 1) / e.ksplit;
-      kbase = (int64_t)blockIdx.y * per;
-      nk = max<int64_t>(0, min(nk_all, kbase + per) - kbase);
+      // dealt out evenly: at least one each, whatever the slices' length (32-bit: K < 2^31, at most 16 splits)
+      const uint32_t n = (uint32_t)nk_all, ks = (uint32_t)e.ksplit;
+      kbase = blockIdx.y * n / ks;
+      nk = (blockIdx.y + 1) * n / ks - kbase;
     }
   }
   // CONVM 1: a group's slices are issued in order, KG slices apart, so the tap and channel offset of
@@ -1805,7 +1806,7 @@ int ksplit_for(const TileCfg& t, int64_t tiles, int64_t K) {
   const int64_t ks = std::min<int64_t>({cus / tiles, nk / (16 * t.kg), 16});
   if (ks < 2) return 1;
   const int64_t per = (nk + ks - 1) / ks;
-  return (int)((nk + per - 1) / per);     // no split without slices
+  return (int)((nk + per - 1) / per);     // as few as keep the longest at `per` (the kernel leaves none without slices)
 }
 
 int64_t split_ws_bytes(const TileCfg& t, int64_t tiles, int ks) {
