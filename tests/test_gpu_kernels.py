@@ -899,13 +899,26 @@ def test_conv_taps(gpu, tile, h, w, tile_table):
                               O.requant(c_oracle.conv3x3_acc(xq.numpy(), wq.numpy()), 9, False)), (n, ci, co)
 
 
-@pytest.mark.parametrize("m,n,k", [(16, 8192, 4096), (17, 5120, 1024), (17, 5104, 1024), (33, 2560, 2064), (64, 12900, 512),
-                                   (65, 1001, 1552), (257, 1000, 1024), (513, 1024, 1040), (768, 16384, 1024),
-                                   (340, 14336, 1024)])
-def test_rule_tiles(gpu, m, n, k, tile_table):
+@pytest.mark.parametrize("m,n,k,i8,bf16", [
+    (16, 8192, 4096, "t32x32k4", None), (17, 5120, 1024, "t32x32k4", None), (17, 5104, 1024, "small_w2", None),
+    (33, 2560, 2064, "t32x32k4", None), (64, 12900, 512, "t64x64", None), (65, 1001, 1552, "t32x32k4", None),
+    (257, 1000, 1024, "t32x64k4", None), (513, 1024, 1040, "t64x64", None), (768, 16384, 1024, "t256x256w8", None),
+    (340, 14336, 1024, "t256x128w8", None),
+    # up to 64 rows: bytes of weight, workgroups (whole 128-byte lines or not), the int8 GEMM's K split, up to 16 rows
+    (64, 1376, 3840, "t32x32k4", None), (64, 1376, 3712, "small_w2", None), (64, 1344, 5120, "small_w2", None),
+    (24, 2048, 2688, "t32x32k4", None), (24, 1984, 2688, "small_w2", None), (24, 4096, 3088, "t32x32k4", None),
+    (24, 4064, 3088, "small_w2", None),
+    (17, 640, 11264, "t32x32k4", "small_w4"), (17, 480, 11264, "small_w4", None), (16, 4096, 8192, "t32x32k4", None),
+    (16, 4064, 8320, "t32x32k4", "small_w4"), (13, 8384, 5968, "small_w2", None), (16, 12300, 2736, "t32x64k4", None)])
+def test_rule_tiles(gpu, m, n, k, i8, bf16, tile_table):
     """Shapes on both sides of the tile rule's lines (small-M kernel or engine, K groups, one round of the large
-    tiles), as the rule plans them: int32 sums exact and, for bf16 operands of the same bytes, within 1e-5
+    tiles), as the rule plans them on 256 CUs (bf16 as int8 of the same bytes but where named): int32 sums exact and, for
+    bf16 operands of the same bytes, within 1e-5
     of the float64 product's norm (float32 sums: about 2^-24 times the square root of K roundings)."""
+    tile_table.tile_clear()
+    if tile_table.num_cus(gpu) == 256:
+        assert tile_table.tile_plan(gpu, "i8", m, n, k)[0] == i8
+        assert tile_table.tile_plan(gpu, "bf16", m, n, k // 2)[0] == (bf16 or i8)
     a, w = _i8((m, k), seed=m + k), _i8((n, k), seed=n + k)
     want = torch._int_mm(torch.cat([a, a.new_zeros(max(0, 17 - m), k)]), w.t().contiguous())[:m]
     assert torch.equal(tile_table.mm_i8(a.to(gpu), w.to(gpu)).cpu(), want)

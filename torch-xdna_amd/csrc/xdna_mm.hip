@@ -1701,13 +1701,35 @@ int tile_lookup(int kind, int64_t m, int64_t n, int64_t k) {
   return it == g_tiles.end() ? T_AUTO : it->second;
 }
 
+int ksplit_for(const TileCfg& t, int64_t tiles, int64_t K);
+
+// 2 to 64 rows: whether the engine's tiles beat the small-M kernel, which reads the weight again for every 16 rows.
+// They do from 5 MB of weight on (32 MB up to 16 rows, whose weight the small-M kernel reads once) where they
+// also make workgroups enough: 32 x 32 tiles times the int8 GEMM's K split, a quarter of the CUs for up to 32 rows of whole
+// 128-byte lines, a third above (half as many where K is split: the small-M kernel's loads of long whole-line rows are
+// slow), and half for rows off whole lines, whose slices begin inside a line, and up to 16 rows (there 32 x 64 tiles of
+// such rows need three quarters). Measured over 384 drawn sizes, none of which the engine runs slower by this line; small-M
+// kernel / tile, by bytes: 64 x 1024 x 3072 5.0 / 5.7 us, 40 x 14336 x 4096 42 / 16.5, 16 x 4096 x 4096 6.1 / 6.3,
+// 16 x 14336 x 4096 18 / 14.7; by workgroups, whole lines: 17 x 1984 x 1920 bf16 (62) 6.4 / 7.2, 17 x 2240 x 4992 (70) 9.8 /
+// 8.6, 47 x 1344 x 2304 bf16 (84) 7.0 / 7.7, 48 x 1472 x 3008 bf16 (92) 1.39 times as fast, 17 x 832 x 10752 in two splits
+// (52) 12.0 / 9.9; others: 33 x 1280 x 8092 (80) 8.3 / 11.0, 17 x 2688 x 7152 (84) 9.7 / 12.1, 20 x 3776 x 3008 (118) 6.8 /
+// 7.2, 32 x 4320 x 2784 (135) 8.8 / 8.1, 64 x 1736 x 11216 (220) 21.2 / 13.5; up to 16 rows: 16 x 3456 x 6464 bf16 (108)
+// 15.1 / 17.0, 13 x 3648 x 13342 bf16 (114) 25.3 / 32.0, 12 x 5952 x 7104 bf16 (186) 26.3 / 19.6,
+// 16 x 9996 x 2392 bf16 (157 of 32 x 64) 15.2 / 16.3, 12 x 14208 x 4288 (222 of 32 x 64) 16.5 / 14.6.
+bool engine_rows64(int64_t M, int64_t N, int64_t kbytes, int kind) {
+  if (N * kbytes < (M <= 16 ? int64_t(32) << 20 : int64_t(5) << 20)) return false;
+  const int64_t cus = device_cus(), t32 = cdiv(M, 32) * cdiv(N, 32);
+  const int64_t ks = kind == XDNA_KIND_I8 ? ksplit_for(tile_cfg(T_32x32K4), t32, kbytes) : 1;
+  const bool lines = kbytes % 128 == 0;
+  if (M <= 16 && !lines && t32 > cus) return 4 * cdiv(N, 64) >= 3 * cus;
+  if (M <= 16 || !lines) return 2 * t32 * ks >= cus;
+  return t32 * ks * (ks > 1 ? 2 : 1) * (M <= 32 ? 4 : 3) >= cus;
+}
+
 // The built-in rule, from back-to-back timed sweeps of every tile shape (rotating weights; kbytes: K in bytes):
 //   * M == 1: the one-row kernel, 4 waves (one output column each) per workgroup;
 //   * 2 <= M <= 8 with K of at least 2 KB: the few-row kernel, 8 output columns per workgroup;
-//   * M <= 64 with a weight small enough that reading it again for every 16 rows stays cheap (5 MB, or 32 MB up to 16
-//     rows): the small-M kernel, 2 waves per workgroup, 4 once K exceeds 8 KB. Either side of the line, int8, small-M
-//     kernel / tile: 64 x 1024 x 3072 5.0 / 5.7 us, bf16 40 x 1024 x 2048 5.6 / 5.9, 20 x 12900 x 512 6.2 / 4.7, bf16
-//     40 x 4096 x 1024 7.5 / 4.8, 40 x 14336 x 4096 42 / 16.5, 16 x 4096 x 4096 6.1 / 6.3, 16 x 14336 x 4096 18 / 14.7;
+//   * M <= 64 unless the engine is faster (engine_rows64): the small-M kernel, 2 waves per workgroup, 4 once K exceeds 8 KB;
 //   * GEMMs with few tiles and K of at least 1 KB: the smallest of 32 x 32, 32 x 64 (4 K groups each) and, from 2 KB,
 //     64 x 64 (2 groups) that makes at most one round of workgroups (128 x 1024 x 3072 5.7 against 7.1 us in 32 x 64,
 //     200 x 1001 x 1552 5.4 against 7.8 in 64 x 64 without groups, 512 x 1001 x 1552 7.2 against 8.1);
@@ -1728,11 +1750,11 @@ int tile_lookup(int kind, int64_t m, int64_t n, int64_t k) {
 //     when there are at least half a round of 256-wide tiles, else 128 x 128;
 //   * 64 x 64 otherwise.
 // A shape the tuned table lists uses the table's tile instead.
-int rule_tile(int64_t M, int64_t N, int64_t kbytes, bool small_ok, bool conv) {
+int rule_tile(int64_t M, int64_t N, int64_t kbytes, bool small_ok, int kind) {
+  const bool conv = kind == XDNA_KIND_CONV;
   if (small_ok && M == 1) return T_GEMV4;
   if (small_ok && M <= 8 && kbytes >= 2048) return T_SEG4R2;
-  if (small_ok && M <= 64 && N * kbytes < (M <= 16 ? int64_t(32) << 20 : int64_t(5) << 20))
-    return (kbytes + 63) / 64 > 128 ? T_SMALL4 : T_SMALL2;
+  if (small_ok && M <= 64 && !engine_rows64(M, N, kbytes, kind)) return (kbytes + 63) / 64 > 128 ? T_SMALL4 : T_SMALL2;
   const int64_t cus = device_cus();
   auto tiles = [&](int64_t bm, int64_t bn) { return cdiv(M, bm) * cdiv(N, bn); };
   const int64_t t64 = tiles(64, 64), t128 = tiles(128, 128), t256 = tiles(256, 256);
@@ -1765,7 +1787,7 @@ int choose_tile(int kind, int64_t m, int64_t n, int64_t k, int64_t kbytes) {
   if (t == T_DIRECT && !(kind == XDNA_KIND_CONV && direct_ok(n, k))) t = T_AUTO;   // not a shape it takes
   if (t != T_AUTO) return t;
   if (kind == XDNA_KIND_CONV && direct_ok(n, k)) return T_DIRECT;
-  return rule_tile(m, n, kbytes, kind != XDNA_KIND_CONV, kind == XDNA_KIND_CONV);
+  return rule_tile(m, n, kbytes, kind != XDNA_KIND_CONV, kind);
 }
 
 // Buffer resources address at most 2 GB; larger operands are processed in row chunks.
@@ -1958,7 +1980,7 @@ TilePlan plan_tiles(int kind, int64_t M, int64_t N, int64_t kbytes, int64_t ktab
   int tail = tile_lookup(kind, M - m1, N, ktab);
   if (is_small(tail) || is_gemv(tail) || is_seg4(tail) || tail == T_DIRECT) tail = T_AUTO;
   if (tail == T_AUTO)
-    tail = (tile == T_256x256W8 || tile == T_256x256PP) ? T_128x256W8 : rule_tile(M - m1, N, kbytes, false, kind == XDNA_KIND_CONV);
+    tail = (tile == T_256x256W8 || tile == T_256x256PP) ? T_128x256W8 : rule_tile(M - m1, N, kbytes, false, kind);
   // only when the leftover rows fit one round of the tail's tiles (8192 x 3072 in 256 x 256 tiles leaves
   // 2816 rows, 264 tiles of 128 x 256: measured slower split than not)
   const TileCfg tt = tile_cfg(tail);
@@ -2010,11 +2032,12 @@ int launch_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, int6
                 const EpiArgs& e, int tile, hipStream_t st) {
   // the one-row kernel takes one row; the small-M kernel addresses the whole activation with one buffer
   // resource, 16 rows per grid row
-  if (is_gemv(tile) && M != 1) tile = rule_tile(M, N, K, M > 1, false);
-  if (is_seg4(tile) && M > 16) tile = rule_tile(M, N, K, true, false);
+  constexpr int kind = epi_bf(EPI) ? XDNA_KIND_BF16 : XDNA_KIND_I8;
+  if (is_gemv(tile) && M != 1) tile = rule_tile(M, N, K, M > 1, kind);
+  if (is_seg4(tile) && M > 16) tile = rule_tile(M, N, K, true, kind);
   // the one-row and few-row kernels write one column per lane: the fused SiLU needs a column's partner
   if (EPI == EPI_BF_SILU && (is_gemv(tile) || is_seg4(tile))) tile = T_SMALL2;
-  if (is_small(tile) && (M * lda > MAX_BUF || (M + 15) / 16 >= 65536)) tile = rule_tile(M, N, K, false, false);
+  if (is_small(tile) && (M * lda > MAX_BUF || (M + 15) / 16 >= 65536)) tile = rule_tile(M, N, K, false, kind);
   if constexpr (EPI != EPI_BF_SILU) {
   if (is_seg4(tile)) {
     // four rows per segment group; the workgroup's 4 waves split K into multiples of 256 bytes
@@ -2450,7 +2473,7 @@ int launch_conv(const int8_t* x, int64_t nb, int64_t h, int64_t w, int64_t c_pad
         continue;
       }
     }
-    const int etile = tile == T_DIRECT ? rule_tile(nb * h * w, co, K, false, true) : tile;
+    const int etile = tile == T_DIRECT ? rule_tile(nb * h * w, co, K, false, XDNA_KIND_CONV) : tile;
     // the haloed input tile where the tile allows it; the running tap counters of CONVM 1 step by KG
     // slices of 64 channels
     const int mode = conv_mode(etile, h, w, c_pad);
@@ -2699,9 +2722,9 @@ int xdna_tile_plan(int kind, int64_t m, int64_t n, int64_t k, int* head, int64_t
   // the launchers' own substitutions: the one-row and few-row kernels take only their row counts, and
   // the small-M kernel addresses the whole activation with one buffer resource
   if (kind != XDNA_KIND_CONV) {
-    if (is_gemv(t) && m != 1) t = rule_tile(m, n, kbytes, m > 1, false);
-    if (is_seg4(t) && m > 16) t = rule_tile(m, n, kbytes, true, false);
-    if (is_small(t) && (m * kbytes > MAX_BUF || (m + 15) / 16 >= 65536)) t = rule_tile(m, n, kbytes, false, false);
+    if (is_gemv(t) && m != 1) t = rule_tile(m, n, kbytes, m > 1, kind);
+    if (is_seg4(t) && m > 16) t = rule_tile(m, n, kbytes, true, kind);
+    if (is_small(t) && (m * kbytes > MAX_BUF || (m + 15) / 16 >= 65536)) t = rule_tile(m, n, kbytes, false, kind);
   }
   // GEMM operands above one buffer resource run in row chunks (with dense rows, lda = k): the plan of
   // the first chunk
