@@ -899,6 +899,25 @@ def test_conv_taps(gpu, tile, h, w, tile_table):
                               O.requant(c_oracle.conv3x3_acc(xq.numpy(), wq.numpy()), 9, False)), (n, ci, co)
 
 
+@pytest.mark.parametrize("tile", ["auto", "t128x128", "t64x64", "t64x64k2", "t32x32k4"])
+def test_conv_taps_16_channels(gpu, tile, tile_table):
+    """Inputs of 16 channels, a chunk per tap, in the engine (rows of 9 chunks: the last slice partial), with the
+    dequantize too, for images down to one pixel: exact against the oracle."""
+    from torch_xdna import kernels
+
+    for n, ci, co, h, w in [(1, 3, 33, 1, 1), (3, 16, 40, 5, 7), (2, 3, 168, 16, 66)]:
+        kernels.tile_set("conv", n * h * w, co, 144, tile)
+        xq, wq = _i8((n, ci, h, w), seed=ci + h), _i8((co, ci, 3, 3), seed=co + w)
+        packed = torch.zeros(co, 9, 16, dtype=torch.int8)
+        packed[:, :, :ci] = wq.permute(0, 2, 3, 1).reshape(co, 9, ci)
+        xn, packed = kernels.nchw_to_nhwc(xq.to(gpu), 16), packed.to(gpu)
+        q = kernels.conv3x3(xn, packed, 7, True)
+        assert np.array_equal(_np(q).transpose(0, 3, 1, 2), O.requant(c_oracle.conv3x3_acc(xq.numpy(), wq.numpy()), 7, True))
+        one = torch.ones(max(n, co), device=gpu)
+        y = kernels.conv3x3_dequant(xn, packed, 7, True, one[:co], one[:n], None, torch.float32)
+        assert torch.equal(y, q.permute(0, 3, 1, 2).float()), (n, ci, co)
+
+
 @pytest.mark.parametrize("m,n,k,i8,bf16", [
     (16, 8192, 4096, "t32x32k4", None), (17, 5120, 1024, "t32x32k4", None), (17, 5104, 1024, "small_w2", None),
     (33, 2560, 2064, "t32x32k4", None), (64, 12900, 512, "t64x64", None), (65, 1001, 1552, "t32x32k4", None),

@@ -85,6 +85,8 @@ struct EpiArgs {
 struct ConvGeom {
   int64_t h, w, c_pad;  // NHWC input geometry
   int64_t m0;           // pixel (within the launch's images) of the launch's row 0
+  uint32_t tap_inv;     // 2^31 / (c_pad / 16), rounded up: the loader of any c_pad finds a chunk's tap with it
+  uint32_t in_bytes;    // the launch's whole images: where the input's buffer resource ends
 };
 
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
@@ -601,9 +603,9 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
     cols_pre[jp] = EpiCols<EPI, CW>(e, n0 + wn * TN + jp * 32 * CB + (lane & 7) * CW, N);
 
   // conv: the launch's rows lie in whole images that start at a; a 3 x 3 window reads past the launch's
-  // first and last rows within those images
-  const int64_t conv_px = CONV ? (cg.m0 + M + cg.h * cg.w - 1) / (cg.h * cg.w) * (cg.h * cg.w) : 0;
-  const __amdgpu_buffer_rsrc_t ra_rsrc = make_rsrc(a, (uint32_t)(CONV ? (conv_px * cg.c_pad) : (M * lda)));
+  // first and last rows within those images (their bytes from the host: rounding the rows up to images here was a
+  // 64-bit division in every workgroup, 0.3 us of a small conv)
+  const __amdgpu_buffer_rsrc_t ra_rsrc = make_rsrc(a, CONV ? cg.in_bytes : (uint32_t)(M * lda));
   const __amdgpu_buffer_rsrc_t rw_rsrc = make_rsrc(w, (uint32_t)(N * ldw));
 
   // This lane's rows: DMA instruction j of this wave covers tile rows r0 = (wave * I + j) * RPI .. + RPI,
@@ -730,11 +732,8 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
   }
   (void)dtap;
   (void)dc0;
-  // CONVM 2: 16-byte chunks per tap and their reciprocal (0: divide)
-  const uint32_t c2_cp = CONVM == 2 ? (uint32_t)(cg.c_pad >> 4) : 1u;
-  const uint32_t c2_inv = CONVM == 2 && c2_cp > 1 && c2_cp < 16384 ? 0xffffffffu / c2_cp + 1u : 0u;
+  const uint32_t c2_cp = CONVM == 2 ? (uint32_t)(cg.c_pad >> 4) : 1u;   // 16-byte chunks per tap
   (void)c2_cp;
-  (void)c2_inv;
   const uint32_t c_rowx = CONV ? (uint32_t)((int)cg.w - 3) * (uint32_t)cg.c_pad : 0u;
   (void)c_rowx;
   auto dma_slice = [&](int64_t kt, int8_t* stage) {
@@ -758,10 +757,13 @@ __global__ __launch_bounds__(WM * WN * KG * 64) void mm_tile_kernel(const int8_t
     } else if constexpr (CONVM == 2) {
       // a lane's chunk is the same K chunk kc in all its rows (f(row) repeats every 16 rows)
       static_assert(BK == 64, "one K chunk per lane");
-      // tap = chunk / (c_pad / 16) as a product with the rounded-up reciprocal (exact below 9 taps for c_pad under
-      // 2^18: the error, chunk * cp16 / 2^32 at most, stays below 1 / cp16); wider inputs divide
+      // tap = chunk / cp16 (cp16 = c_pad / 16): the product with the reciprocal is too large by less than 2 chunk / 2^32
+      // (below 1: chunk < 2^27), so its whole part by at most one. No branch and no division: either
+      // would cut the slice's instructions in two and wait between them (2 x 3 x 16 x 264 -> 168 with both 10.1 us,
+      // 8.9 this way)
       const uint32_t kc = ((uint32_t)k0 >> 4) + (uint32_t)ca[0];
-      const uint32_t tap = c2_inv ? __umulhi(kc, c2_inv) : kc / c2_cp;
+      uint32_t tap = __umulhi(kc << 1, cg.tap_inv);
+      tap -= tap * c2_cp > kc ? 1u : 0u;
       const uint32_t bit = live && kc < (uint32_t)(K >> 4) ? 1u << tap : 0u;
       const uint32_t delta = (kc << 4) + (tap >= 3 ? c_rowx : 0u) + (tap >= 6 ? c_rowx : 0u);
 #pragma unroll
@@ -2453,9 +2455,10 @@ int launch_conv(const int8_t* x, int64_t nb, int64_t h, int64_t w, int64_t c_pad
   }
   const int64_t K = 9 * c_pad;
   const int tile = choose_tile(XDNA_KIND_CONV, nb * h * w, co, K, K);
-  ConvGeom cg{h, w, c_pad};
+  ConvGeom cg{h, w, c_pad, 0, (uint32_t)(((int64_t(1) << 31) + c_pad / 16 - 1) / (c_pad / 16)), 0};
   for (int64_t b0 = 0; b0 < nb; b0 += imgs) {
     const int64_t bc = std::min(imgs, nb - b0);
+    cg.in_bytes = (uint32_t)(bc * per_img);
     EpiArgs eb = e;
     if (e.dq_out) eb.px0 = e.px0 + b0 * h * w;   // NCHW output: addressed by global pixel, not by row
     else eb = shift_epi(e, 1, b0 * h * w, 0);
