@@ -120,6 +120,25 @@ def test_conv_quant_ragged(gpu, dtype, n, ch, h, w, c_pad):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("rows,k,ld,k_pad", [(2049, 7, 7, 16), (2050, 15, 15, 32), (2049, 16, 17, 16), (2049, 17, 17, 32),
+                                             (262, 501, 501, 512), (256, 511, 513, 512), (257, 511, 513, 528),
+                                             (300, 513, 513, 544), (5, 513, 513, 528), (2048, 63, 63, 64)])
+def test_quant_rows_ragged_lines(gpu, dtype, rows, k, ld, k_pad):
+    """Both sides of the line between an element per lane and 16-element groups (rows, elements of a row and in all), rows
+    below one group among them: as test_quant_rows_ragged."""
+    test_quant_rows_ragged(gpu, dtype, rows, k, ld, k_pad)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("n,ch,h,w,c_pad", [(520, 50, 1, 3, 64), (520, 60, 1, 5, 64), (4, 130, 105, 107, 144),
+                                            (2, 4, 9, 11, 16), (2, 5, 9, 11, 16), (3, 67, 13, 17, 80)])
+def test_conv_quant_ragged_lines(gpu, dtype, n, ch, h, w, c_pad):
+    """Images off 16 bytes with four pixels per lane (also where an image has fewer) and one, with a wave's channels
+    up to four, more and none: as test_conv_quant_ragged."""
+    test_conv_quant_ragged(gpu, dtype, n, ch, h, w, c_pad)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("rows,k,off,ld", [(1, 1, 0, 1), (3, 7, 1, 9), (5, 8, 1, 8), (300, 1001, 0, 1001), (64, 1537, 3, 1600),
                                            (257, 2048, 0, 2048)])
 def test_cast_rows_bf16(gpu, dtype, rows, k, off, ld):

@@ -360,6 +360,7 @@ __global__ __launch_bounds__(256) void quant_rows_stream_kernel(const void* __re
 typedef uint32_t u32x4_e4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x4_e2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x2_e2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t u32x4_e1 __attribute__((ext_vector_type(4), aligned(1)));
 template <int DT>
 __device__ __forceinline__ uint4 load_u4_any(const void* p) {
   if constexpr (DT == XDNA_F32) {
@@ -386,9 +387,10 @@ __device__ __forceinline__ uint4 load_u4_first(const void* p, int n) {
 
 // Rows of any length and stride (their starts aligned to the element only), kept in registers like those of the
 // kernels above: TPR threads per row (a wave, four rows per block, or the block), thread t owning groups t, t + TPR,
-// ... of 16 elements, read with unaligned 16-byte loads and written as one 16-byte store; the row's last group is
-// read element by element, its padding bytes cleared. Needs 16-byte aligned output rows with room for whole groups.
-// float32 1999 x 1537: 5.7 us, 8.8 us one element per lane with the row read twice.
+// ... of 16 elements, read with unaligned 16-byte loads and written as one 16-byte store. The row's last group is the
+// 16 elements that end it, some of them a second time, at any byte of the output row (the same bytes twice); rows below 16
+// elements are read one by one. Bytes past the row are cleared. Needs 16-byte aligned output rows with room for whole
+// groups. float32 1999 x 1537: 5.7 us, 8.8 us one element per lane with the row read twice; bf16 16 x 701 2.7, one element per lane 2.9.
 template <int DT, int TPR, int G>
 __global__ __launch_bounds__(256) void quant_rows_ragged_kernel(const void* __restrict__ x, int64_t rows, int64_t k,
                                                                 int64_t ld_x, int8_t* __restrict__ q, int64_t ld_q,
@@ -403,19 +405,16 @@ __global__ __launch_bounds__(256) void quant_rows_ragged_kernel(const void* __re
   if (TPR == 64 && row >= rows) return;    // wave-uniform, and a wave's row meets no barrier
   const char* xr = reinterpret_cast<const char*>(x) + row * ld_x * ESZ;
   const int ki = (int)k;                   // at most 16 TPR G (checked by the launcher)
+  const bool shorter = ki < 16;            // uniform
+  auto start = [&](int j) { return min((t + j * TPR) * 16, max(0, ki - 16)); };
   V v[G][LPG];
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
-    const int e0 = (t + j * TPR) * 16;
-    if (e0 + 16 <= ki) {
+  for (int j = 0; j < G; ++j)
 #pragma unroll
-      for (int l = 0; l < LPG; ++l) v[j][l].raw = load_u4_any<DT>(xr + (e0 + l * VEC) * ESZ);
-    } else {
-#pragma unroll
-      for (int l = 0; l < LPG; ++l)
-        v[j][l].raw = load_u4_first<DT>(xr + (int64_t)min(e0 + l * VEC, ki) * ESZ, ki - (e0 + l * VEC));
+    for (int l = 0; l < LPG; ++l) {
+      if (shorter) v[j][l].raw = load_u4_first<DT>(xr + min(l * VEC, ki) * ESZ, ki - l * VEC);
+      else v[j][l].raw = load_u4_any<DT>(xr + (start(j) + l * VEC) * ESZ);
     }
-  }
   AbsMaxBits<DT> am;
 #pragma unroll
   for (int j = 0; j < G; ++j)
@@ -428,20 +427,24 @@ __global__ __launch_bounds__(256) void quant_rows_ragged_kernel(const void* __re
   int8_t* qr = q + row * ld_q;
 #pragma unroll
   for (int j = 0; j < G; ++j) {
-    const int e0 = (t + j * TPR) * 16;
-    if (e0 < ki) {
+    if ((t + j * TPR) * 16 < ki) {
       float f[16];
 #pragma unroll
       for (int l = 0; l < LPG; ++l)
 #pragma unroll
         for (int e = 0; e < VEC; ++e) f[l * VEC + e] = v[j][l].get(e);
-      uint32_t w[4], keep[4];
+      uint32_t w[4];
       quant_pack<16>(f, sc, rc, w);
-      valid_masks(min(16, ki - e0), keep);
-      *reinterpret_cast<uint4*>(qr + e0) = make_uint4(w[0] & keep[0], w[1] & keep[1], w[2] & keep[2], w[3] & keep[3]);
+      if (shorter) {
+        uint32_t keep[4];
+        valid_masks(ki, keep);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] &= keep[i];
+      }
+      *reinterpret_cast<u32x4_e1*>(qr + start(j)) = u32x4_e1{w[0], w[1], w[2], w[3]};
     }
   }
-  for (int64_t c = (int64_t)cdiv(k, 16) * 16 + t; c < k_pad; c += TPR) qr[c] = 0;
+  for (int64_t c = (int64_t)max(ki, 16) + t; c < k_pad; c += TPR) qr[c] = 0;
 }
 
 // Scalar path for any k / stride / alignment: one block per row, the row read twice.
@@ -484,7 +487,10 @@ int launch_quant_rows(const void* x, int64_t rows, int64_t k, int64_t ld_x, int8
   const bool vec_ok = (k % VEC == 0) && (ld_x % VEC == 0) && aligned(x, 16) && aligned(q, 16) && (ld_q % 16 == 0);
   // rows without whole 16-element groups or 16-byte starts, into output rows with room for whole groups
   const int64_t rg = cdiv(k, 16);
-  if (!vec_ok && aligned(q, 16) && ld_q % 16 == 0 && k_pad >= rg * 16 && rg <= 256 * (DT == XDNA_F32 ? 4 : 8)) {
+  // (short rows, few of them, stay with an element per lane: 100 x 97 2.3 us, 3.1 in groups of 16, which keep a lane
+  // in eight busy; 400 x 333 2.8 either way, 2000 x 161 float32 3.3 / 3.0, 8192 x 15 5.8 / 4.9)
+  const bool little = k <= 512 && rows <= 2048 && rows * k <= (1 << 17);
+  if (!vec_ok && !little && aligned(q, 16) && ld_q % 16 == 0 && k_pad >= rg * 16 && rg <= 256 * (DT == XDNA_F32 ? 4 : 8)) {
 #define XDNA_QG(TPR_, G_) \
   quant_rows_ragged_kernel<DT, TPR_, G_><<<dim3((unsigned)cdiv(rows, 256 / TPR_)), 256, 0, st>>>(x, rows, k, ld_x, q, ld_q, k_pad, s)
     if (rg <= 64) XDNA_QG(64, 1);
@@ -788,12 +794,13 @@ __global__ __launch_bounds__(256) void conv_quant_nhwc_narrow_kernel(const void*
   }
 }
 
-// The same for images of any size and alignment: a block covers 64 channels x 64 P pixels, wave w pixels 16 P w ..,
-// lane l channels 16 (l / 16) .. of P pixels (4, or 1 where that leaves blocks for less than a round), read as one
-// load at the elements' alignment; a lane past the channel's last whole P takes the P that end it (some pixels twice:
-// the same bytes). Tile rows of 80 bytes: the 16 pixels x 4 chunks of a write fall evenly on the banks. With the
-// image max: 4 x 100 x 75 x 93 bf16 10.4 us (28.6 us one pixel per lane and quotient), 3 x 256 x 37 x 37 float32
-// 7.5 (11.5), 2 x 40 x 31 x 33 bf16 8.5 (8.1).
+// The same for images of any size and alignment: a block covers 64 channels x 64 P pixels. P = 4: wave w pixels 64 w ..,
+// lane l channels 16 (l / 16) .. of four pixels, read as one load at the elements' alignment; a lane past the channel's
+// last whole four takes the four that end it (some pixels twice: the same bytes). P = 1, where four leave blocks for less
+// than a round: wave w channels 16 w .., a pixel per lane (as for P = 4, each load would touch four channels: 2 x 16 x 477
+// x 17 bf16 8.5 us, 7.5 this way). Tile rows of 80 bytes: the 16 pixels x 4 chunks of a write fall evenly on the banks.
+// With the image max: 4 x 100 x 75 x 93 bf16 10.4 us (28.6 us one pixel per lane and quotient), 3 x 256 x 37 x 37
+// float32 6.9 (11.5), 2 x 40 x 31 x 33 bf16 7.6 (8.0).
 template <int DT, int P>
 __global__ __launch_bounds__(256) void conv_quant_nhwc_any_kernel(const void* __restrict__ x, int64_t ch, int64_t hw,
                                                                   const float* __restrict__ parts, int nparts,
@@ -806,18 +813,22 @@ __global__ __launch_bounds__(256) void conv_quant_nhwc_any_kernel(const void* __
   __shared__ float red[4];
   const int64_t b = blockIdx.z;
   const int64_t p0 = (int64_t)blockIdx.x * (64 * P), c0 = (int64_t)blockIdx.y * 64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t cl = c0 + 16 * (lane >> 4);                // the lane's first channel
-  const int64_t pe = max<int64_t>(0, min<int64_t>(p0 + 16 * P * wave + P * (lane & 15), hw - P));   // and pixel
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = P == 1 ? wave : lane >> 4;               // the lane's 16 channels of the 64
+  const int64_t cl = c0 + 16 * grp;                        // the first
+  const int64_t pe = max<int64_t>(0, min<int64_t>(p0 + (P == 1 ? lane : 16 * P * wave + P * (lane & 15)), hw - P));   // pixel
   const char* xb = reinterpret_cast<const char*>(x) + (b * ch * hw + pe) * ESZ;
-  const int nl = (int)min<int64_t>(16, ch - c0);           // uniform: below 16 only where the block has no more channels
+  // uniform: below 16 only where the block (P == 1: the wave) has no more channels
+  const int nl = (int)min<int64_t>(16, ch - (P == 1 ? cl : c0));
   Vec16<DT> v[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     v[i].raw = make_uint4(0, 0, 0, 0);
     if (i < nl) {
       const char* px = xb + min(cl + i, ch - 1) * hw * ESZ;   // channels past ch: cleared below
-      if (P == 1 || hw < P) v[i].raw = load_u4_first<DT>(px, (int)min<int64_t>(P, hw));
+      if constexpr (P == 1) {
+        v[i].raw.x = DT == XDNA_F32 ? *reinterpret_cast<const uint32_t*>(px) : (uint32_t)*reinterpret_cast<const uint16_t*>(px);
+      } else if (hw < P) v[i].raw = load_u4_first<DT>(px, (int)hw);
       else if constexpr (DT == XDNA_F32) v[i].raw = load_u4_any<DT>(px);
       else {
         const u32x2_e2 h = *reinterpret_cast<const u32x2_e2*>(px);
@@ -836,10 +847,17 @@ __global__ __launch_bounds__(256) void conv_quant_nhwc_any_kernel(const void* __
     float f[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) f[i] = v[i].get(j);
-    uint32_t w[4];
-    quant_pack<16>(f, sc, rc, w);
+    uint32_t w[4] = {0, 0, 0, 0};
+    if (P == 1 && nl <= 4) {               // images of few channels: the others stay 0
+      const float f4[4] = {f[0], f[1], f[2], f[3]};
+      uint32_t w4[1];
+      quant_pack<4>(f4, sc, rc, w4);
+      w[0] = w4[0];
+    } else {
+      quant_pack<16>(f, sc, rc, w);
+    }
     if (row0 + j >= 0)
-      *reinterpret_cast<uint4*>(&tile[(row0 + j) * PITCH + 16 * (lane >> 4)]) =
+      *reinterpret_cast<uint4*>(&tile[(row0 + j) * PITCH + 16 * grp]) =
           make_uint4(w[0] & keep[0], w[1] & keep[1], w[2] & keep[2], w[3] & keep[3]);
   }
   __syncthreads();
@@ -1516,7 +1534,11 @@ int xdna_conv_quant_nhwc(const void* x, int x_dtype, int64_t nb, int64_t ch, int
   const dim3 gn((unsigned)cdiv(hw, 256 * (16 / esz)), (unsigned)nb, 1);
   const dim3 ga((unsigned)cdiv(hw, 256), (unsigned)cdiv(c_pad, 64), (unsigned)nb);
   const dim3 g1p((unsigned)cdiv(hw, 64), (unsigned)cdiv(c_pad, 64), (unsigned)nb);
-  const bool four = 2 * cdiv(hw, 256) * cdiv(c_pad, 64) * nb >= device_cus();
+  // four pixels a lane once their blocks make half a round (bf16), a round (float32) or two (float16, whose conversions
+  // cost more in fewer lanes); four against one: 121 x 121 x 64 (58 blocks) bf16 8.6 / 8.0 us, 4 x 256 x 37 x 50 (128) 9.0 /
+  // 11.1, float32 8.95 / 7.6, 8 x 512 x 29 x 29 (256) 9.6 / 9.95, float16 13.7 / 12.7, 8 x 256 x 57 x 57 (416) 15.05 / 14.9
+  const int64_t blocks4 = cdiv(hw, 256) * cdiv(c_pad, 64) * nb;
+  const bool four = blocks4 * (x_dtype == XDNA_BF16 ? 4 : x_dtype == XDNA_F32 ? 2 : 1) >= 2 * (int64_t)device_cus();
 #define XDNA_CQ(DT)                                                                                        \
   if (nt) image_absmax_kernel<DT, true><<<g1, 1024, 0, st>>>(x, per, amax_ws);                              \
   else image_absmax_kernel<DT, false><<<g1, 1024, 0, st>>>(x, per, amax_ws);                                \
