@@ -941,7 +941,7 @@ def test_conv_taps_16_channels(gpu, tile, tile_table):
     (16, 8192, 4096, "t32x32k4", None), (17, 5120, 1024, "t32x32k4", None), (17, 5104, 1024, "small_w2", None),
     (33, 2560, 2064, "t32x32k4", None), (64, 12900, 512, "t64x64", None), (65, 1001, 1552, "t32x32k4", None),
     (257, 1000, 1024, "t32x64k4", None), (513, 1024, 1040, "t64x64", None), (768, 16384, 1024, "t256x256w8", None),
-    (340, 14336, 1024, "t256x128w8", None),
+    (340, 14336, 1024, "t256x128w8", None), (213, 656, 12944, "t32x64k4", "t32x32k4"), (213, 656, 12160, "t32x32k4", None),
     # up to 64 rows: bytes of weight, workgroups (whole 128-byte lines or not), the int8 GEMM's K split, up to 16 rows
     (64, 1376, 3840, "t32x32k4", None), (64, 1376, 3712, "small_w2", None), (64, 1344, 5120, "small_w2", None),
     (24, 2048, 2688, "t32x32k4", None), (24, 1984, 2688, "small_w2", None), (24, 4096, 3088, "t32x32k4", None),

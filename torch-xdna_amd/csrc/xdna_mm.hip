@@ -431,14 +431,14 @@ __device__ __forceinline__ void tile_coords(uint32_t pid, uint32_t tiles_m, uint
   tn = rdiv;
 }
 
-// LDS rows are 64 bytes (one 64-deep K slice of a tile row); the 16-byte chunk c (0..3) of row r sits
+// An LDS row is one K slice of a tile row, BK = 64 or 128 bytes. BK = 64: the 16-byte chunk c (0..3) of row r sits
 // at chunk c ^ f(r) with f(r) = (r >> 2) & 3. A fragment read touches 32 consecutive rows at logical
 // chunks 2 ks and 2 ks + 1 (lanes 0-31 and 32-63). Under this f every 16 consecutive lanes cover the 16
 // bank groups of a 256-byte line and lanes l, l + 32 never share a 16-byte group within a 4-row block;
 // measured on gfx950 (rocprofv3 SQ_LDS_IDX_ACTIVE / SQ_INSTS_LDS) at 4.0 cycles per ds_read_b128,
 // the conflict-free minimum. f depends only on r & 15, so fragments 32 rows apart differ by a
 // constant offset.
-// BK = 128: rows of 128 bytes, chunk c (0..7) at c ^ ((r >> 1) & 7): again 16 consecutive rows at one chunk cover the
+// BK = 128: chunk c (0..7) at c ^ ((r >> 1) & 7): again 16 consecutive rows at one chunk cover the
 // 16 groups of a 256-byte line, and f depends only on r & 15.
 template <int BK = 64>
 __device__ __forceinline__ int swz_f(int row) {
@@ -1734,7 +1734,9 @@ bool engine_rows64(int64_t M, int64_t N, int64_t kbytes, int kind) {
 //   * M <= 64 unless the engine is faster (engine_rows64): the small-M kernel, 2 waves per workgroup, 4 once K exceeds 8 KB;
 //   * GEMMs with few tiles and K of at least 1 KB: the smallest of 32 x 32, 32 x 64 (4 K groups each) and, from 2 KB,
 //     64 x 64 (2 groups) that makes at most one round of workgroups (128 x 1024 x 3072 5.7 against 7.1 us in 32 x 64,
-//     200 x 1001 x 1552 5.4 against 7.8 in 64 x 64 without groups, 512 x 1001 x 1552 7.2 against 8.1);
+//     200 x 1001 x 1552 5.4 against 7.8 in 64 x 64 without groups, 512 x 1001 x 1552 7.2 against 8.1); int8 in 32 x 64
+//     where those split K three ways and 32 x 32 not at all (213 x 656 x 12944 15.7 against 18.7 us, 196 x 604 x 14000 14.8
+//     against 16.3; two ways are not enough: 235 x 557 x 9504 14.3 against 12.6);
 //   * convs the same, 64 x 64 too, from K of 576 bytes (64 channels): their slices cost more than a GEMM's, so splitting
 //     them pays earlier (784 pixels x 192 channels 5.4 -> 4.8 us at 64 input channels, 11.9 -> 6.1 at 224; 1480 x 180 x
 //     9 * 112 8.1 -> 5.7; 7200 x 96 x 9 * 200 11.9 -> 9.1, all against 64 x 64 without groups; 64 x 64 with two groups
@@ -1761,7 +1763,11 @@ int rule_tile(int64_t M, int64_t N, int64_t kbytes, bool small_ok, int kind) {
   auto tiles = [&](int64_t bm, int64_t bn) { return cdiv(M, bm) * cdiv(N, bn); };
   const int64_t t64 = tiles(64, 64), t128 = tiles(128, 128), t256 = tiles(256, 256);
   if (kbytes >= (conv ? 576 : 1024)) {
-    if (tiles(32, 32) <= cus) return T_32x32K4;
+    if (tiles(32, 32) <= cus) {
+      const bool split3 = kind == XDNA_KIND_I8 && 2 * tiles(32, 32) > cus &&
+                          ksplit_for(tile_cfg(T_32x64K4), tiles(32, 64), kbytes) > 2;
+      return split3 ? T_32x64K4 : T_32x32K4;
+    }
     if (tiles(32, 64) <= cus) return T_32x64K4;
     if ((conv || kbytes >= 2048) && t64 <= cus) return T_64x64K2;
   }
