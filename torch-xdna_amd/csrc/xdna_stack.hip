@@ -141,7 +141,7 @@ int launch_rmsnorm(float* x, const float* a, int64_t rows, int64_t d, const void
 
 // ------------------------------------------------------------------------------ q / k norm + RoPE
 // Two kinds of workgroups. The first V_TOK-token blocks per kv head copy V transposed: 32 tokens x 128 dims come in
-// as float4 rows, turn in LDS and leave with 32 tokens side by side in a store instruction (any vt_col; consecutive
+// as float2 rows, turn in LDS and leave with 32 tokens side by side in a store instruction (any vt_col; consecutive
 // columns make whole 64-byte runs. One dim per lane at one token's column scattered every store over 64 lines).
 // The others take one token each: the rotation of its 64 angles once, in LDS, then half a wave per q or k head, lane
 // i of it holding dims 2 i, 2 i + 1 and 64 + those, which RoPE rotates into each other (rotate_half), so only the
