@@ -390,7 +390,9 @@ __device__ __forceinline__ uint4 load_u4_first(const void* p, int n) {
 // ... of 16 elements, read with unaligned 16-byte loads and written as one 16-byte store. The row's last group is the
 // 16 elements that end it, some of them a second time, at any byte of the output row (the same bytes twice); rows below 16
 // elements are read one by one. Bytes past the row are cleared. Needs 16-byte aligned output rows with room for whole
-// groups. float32 1999 x 1537: 5.7 us, 8.8 us one element per lane with the row read twice; bf16 16 x 701 2.7, one element per lane 2.9.
+// groups. One element per lane with the row read twice / this: float32 1999 x 1537 8.8 / 5.6 us, bf16 8192 x 4095 68 / 20.3,
+// float32 3281 x 13683 110 / 38.4; bf16 16 x 701 2.9 / 2.7. Lanes past the row load nothing (reading its last group again there cost
+// 3281 x 13683 8 us).
 template <int DT, int TPR, int G>
 __global__ __launch_bounds__(256) void quant_rows_ragged_kernel(const void* __restrict__ x, int64_t rows, int64_t k,
                                                                 int64_t ld_x, int8_t* __restrict__ q, int64_t ld_q,
@@ -411,10 +413,18 @@ __global__ __launch_bounds__(256) void quant_rows_ragged_kernel(const void* __re
 #pragma unroll
   for (int j = 0; j < G; ++j)
 #pragma unroll
-    for (int l = 0; l < LPG; ++l) {
-      if (shorter) v[j][l].raw = load_u4_first<DT>(xr + min(l * VEC, ki) * ESZ, ki - l * VEC);
-      else v[j][l].raw = load_u4_any<DT>(xr + (start(j) + l * VEC) * ESZ);
-    }
+    for (int l = 0; l < LPG; ++l) v[j][l].raw = make_uint4(0, 0, 0, 0);
+  if (shorter) {
+#pragma unroll
+    for (int l = 0; l < LPG; ++l) v[0][l].raw = load_u4_first<DT>(xr + min(l * VEC, ki) * ESZ, t == 0 ? ki - l * VEC : 0);
+  } else {
+#pragma unroll
+    for (int j = 0; j < G; ++j)
+      if ((t + j * TPR) * 16 < ki) {
+#pragma unroll
+        for (int l = 0; l < LPG; ++l) v[j][l].raw = load_u4_any<DT>(xr + (start(j) + l * VEC) * ESZ);
+      }
+  }
   AbsMaxBits<DT> am;
 #pragma unroll
   for (int j = 0; j < G; ++j)
