@@ -947,7 +947,10 @@ def test_conv_taps_16_channels(gpu, tile, tile_table):
     (24, 2048, 2688, "t32x32k4", None), (24, 1984, 2688, "small_w2", None), (24, 4096, 3088, "t32x32k4", None),
     (24, 4064, 3088, "small_w2", None),
     (17, 640, 11264, "t32x32k4", "small_w4"), (17, 480, 11264, "small_w4", None), (16, 4096, 8192, "t32x32k4", None),
-    (16, 4064, 8320, "t32x32k4", "small_w4"), (13, 8384, 5968, "small_w2", None), (16, 12300, 2736, "t32x64k4", None)])
+    (16, 4064, 8320, "t32x32k4", "small_w4"), (13, 8384, 5968, "small_w2", None), (16, 12300, 2736, "t32x64k4", None),
+    (24, 3296, 5136, "t32x32k4", None), (24, 3264, 5136, "small_w2", None), (24, 3296, 5104, "small_w2", None),
+    (13, 8384, 6160, "t32x64k4", None), (20, 7168, 832, "small_w2", None), (20, 8256, 832, "small_w2", None),
+    (20, 12288, 832, "t32x64", None), (20, 8192, 896, "t32x64", None)])
 def test_rule_tiles(gpu, m, n, k, i8, bf16, tile_table):
     """Shapes on both sides of the tile rule's lines (small-M kernel or engine, K groups, one round of the large
     tiles), as the rule plans them on 256 CUs (bf16 as int8 of the same bytes but where named): int32 sums exact and, for

@@ -1707,24 +1707,27 @@ int ksplit_for(const TileCfg& t, int64_t tiles, int64_t K);
 
 // 2 to 64 rows: whether the engine's tiles beat the small-M kernel, which reads the weight again for every 16 rows.
 // They do from 5 MB of weight on (32 MB up to 16 rows, whose weight the small-M kernel reads once) where they
-// also make workgroups enough: 32 x 32 tiles times the int8 GEMM's K split, a quarter of the CUs for up to 32 rows of whole
+// also make workgroups enough: 32 x 32 tiles (32 x 64 below 1 KB of K) times the int8 GEMM's K split, a quarter of the CUs for up to 32 rows of whole
 // 128-byte lines, a third above (half as many where K is split: the small-M kernel's loads of long whole-line rows are
-// slow), and half for rows off whole lines, whose slices begin inside a line, and up to 16 rows (there 32 x 64 tiles of
-// such rows need three quarters). Measured over 384 drawn sizes, none of which the engine runs slower by this line; small-M
+// slow), and half for rows off whole lines, whose slices begin inside a line (two fifths from 5 KB of K on), and up to 16 rows (32 x 64 tiles of
+// such rows need three quarters: below 1 KB of K, and up to 16 rows below 6 KB). Measured over 384 drawn sizes, none of which the engine runs slower by this line; small-M
 // kernel / tile, by bytes: 64 x 1024 x 3072 5.0 / 5.7 us, 40 x 14336 x 4096 42 / 16.5, 16 x 4096 x 4096 6.1 / 6.3,
 // 16 x 14336 x 4096 18 / 14.7; by workgroups, whole lines: 17 x 1984 x 1920 bf16 (62) 6.4 / 7.2, 17 x 2240 x 4992 (70) 9.8 /
 // 8.6, 47 x 1344 x 2304 bf16 (84) 7.0 / 7.7, 48 x 1472 x 3008 bf16 (92) 1.39 times as fast, 17 x 832 x 10752 in two splits
 // (52) 12.0 / 9.9; others: 33 x 1280 x 8092 (80) 8.3 / 11.0, 17 x 2688 x 7152 (84) 9.7 / 12.1, 20 x 3776 x 3008 (118) 6.8 /
-// 7.2, 32 x 4320 x 2784 (135) 8.8 / 8.1, 64 x 1736 x 11216 (220) 21.2 / 13.5; up to 16 rows: 16 x 3456 x 6464 bf16 (108)
+// 7.2, 23 x 3584 x 5786 bf16 (112) 18.9 / 17.7, 53 x 1664 x 10852 bf16 with SiLU (104) 33.5 / 29.6, 32 x 4320 x 2784 (135) 8.8 / 8.1, 64 x 1736 x 11216 (220) 21.2 / 13.5; up to 16 rows: 16 x 3456 x 6464 bf16 (108)
 // 15.1 / 17.0, 13 x 3648 x 13342 bf16 (114) 25.3 / 32.0, 12 x 5952 x 7104 bf16 (186) 26.3 / 19.6,
-// 16 x 9996 x 2392 bf16 (157 of 32 x 64) 15.2 / 16.3, 12 x 14208 x 4288 (222 of 32 x 64) 16.5 / 14.6.
+// 16 x 9996 x 2392 bf16 (157 of 32 x 64) 15.2 / 16.3, 12 x 14208 x 4288 (222 of 32 x 64) 16.5 / 14.6, 14 x 9728 x 7486 (152)
+// 21.1 / 20.1, 12 x 9472 x 13505 bf16 (148) 73.9 / 68.8; below 1 KB of K 20 x 7168 x 832 (112 of 32 x 64) 4.4 / 5.4, 26 x 9728 x 465 bf16 (152) 5.5 / 6.2,
+// 17 x 13120 x 256 bf16 (205) 5.9 / 4.2.
 bool engine_rows64(int64_t M, int64_t N, int64_t kbytes, int kind) {
   if (N * kbytes < (M <= 16 ? int64_t(32) << 20 : int64_t(5) << 20)) return false;
-  const int64_t cus = device_cus(), t32 = cdiv(M, 32) * cdiv(N, 32);
+  const int64_t cus = device_cus(), t32 = cdiv(M, 32) * cdiv(N, kbytes >= 1024 ? 32 : 64);
   const int64_t ks = kind == XDNA_KIND_I8 ? ksplit_for(tile_cfg(T_32x32K4), t32, kbytes) : 1;
   const bool lines = kbytes % 128 == 0;
-  if (M <= 16 && !lines && t32 > cus) return 4 * cdiv(N, 64) >= 3 * cus;
-  if (M <= 16 || !lines) return 2 * t32 * ks >= cus;
+  if (M <= 16 && !lines && t32 > cus && kbytes < 6144) return 4 * cdiv(N, 64) >= 3 * cus;
+  if (!lines && kbytes < 1024) return 4 * t32 >= 3 * cus;
+  if (M <= 16 || !lines) return 2 * t32 * ks >= cus || (M > 16 && kbytes >= 5120 && 5 * t32 >= 2 * cus);
   return t32 * ks * (ks > 1 ? 2 : 1) * (M <= 32 ? 4 : 3) >= cus;
 }
 

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const float* __restri
 // are rescaled only in the blocks of 32 keys where some row's running maximum m grows; P is rounded to bf16 for the
 // second product, l sums the unrounded p. The maximum follows every 32 keys also where a tile holds 64, and never lags:
 // a key that is the maximum has p = 1, which rounds to itself, so the coarser m follows, the further the result is off
-// (4096 / 1500 / 700 against 64 bits: 2.237e-3, 2.241e-3 with one maximum per 64 keys, which ran 2 to 5% faster;
+// (4096 / 1500 / 700 against 64 bits: 2.237e-3, 2.241e-3 with one maximum per 64 keys, which ran 2 to 10% faster;
 // m lagging by up to 2^8: 5% further off and 4% faster; neither is done).
 //
 // What bounds it: per 64 keys and 32 rows a wave issues 32 MFMAs (1024 cycles of its SIMD) and about 400 vector
